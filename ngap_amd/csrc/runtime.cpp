@@ -65,10 +65,15 @@ int RunCtx::init() {
   HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   HIP_TRY(hipEventCreate(&ev0));
   HIP_TRY(hipEventCreate(&ev1));
-  HIP_TRY(counters.reserve(kCounterBytes));
+  static_assert(kCounterBytes % 8 == 0, "report slots follow the counters");
+  HIP_TRY(counters.reserve(kCounterBytes + kSmallReports * 8));
   // the reset kernel clears the counters a run uses; the rest stays zero
-  HIP_TRY(hipMemset(counters.p, 0, counters.n));
-  HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&host_cnt), kCounterBytes, hipHostMallocDefault));
+  HIP_TRY(hipMemset(counters.p, 0, kCounterBytes));
+  report_slots = counters.as<uint64_t>() + kCounterBytes / 8;
+  HIP_TRY(hipMemset(report_slots, 0xFF, kSmallReports * 8));  // every slot empty
+  HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&host_cnt),
+                        kCounterBytes + (kSmallReports + 1) * 8, hipHostMallocDefault));
+  host_reports = reinterpret_cast<uint64_t *>(host_cnt) + kCounterBytes / 8;
   return NGAP_OK;
 }
 
@@ -194,6 +199,7 @@ void attach_ctx(KParams &P, RunCtx &ctx) {
   P.overflow_count = reinterpret_cast<uint32_t *>(counters + 3);
   P.reports = ctx.reports.as<uint64_t>();
   P.report_cap = ctx.report_cap;
+  ctx.sorted = false;  // the launch that follows overwrites the last run's reports
 }
 
 // Kernel kind an engine run of o launches: 0 k_batched (traces), 1
@@ -458,6 +464,33 @@ int sorted_reports(RunCtx &ctx, std::vector<uint64_t> &v) {
 }
 
 namespace {
+
+// ngap_get_reports: sorts the last run's reports, once per run, on the device;
+// on the host (the result goes back to ctx.reports) where no memory is left
+// for the device's work area.
+int sort_reports(const ngap_engine *eng, RunCtx &ctx) {
+  if (ctx.sorted) return NGAP_OK;
+  const uint64_t n = ctx.last_count;
+  ctx.unique_reports = 0;
+  ctx.sorted_on_host = false;
+  if (n) {
+    uint32_t bits = 0;
+    while (bits < 32 && ((eng->chunk_len * eng->num_seg - 1) >> bits)) bits++;
+    const hipError_t e = sort_reports_device(ctx, n, bits);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      std::vector<uint64_t> v;
+      if (const int rc = sorted_reports(ctx, v)) return rc;
+      for (uint64_t &k : v) k = (k << 32) | (k >> 32);
+      HIP_TRY(hipMemcpy(ctx.reports.p, v.data(), v.size() * 8, hipMemcpyHostToDevice));
+      ctx.unique_reports = v.size();
+    } else {
+      HIP_TRY(e);
+    }
+  }
+  ctx.sorted = true;
+  return NGAP_OK;
+}
 
 // Static schedule (no host work items): a group whose roots are rare under the
 // input's byte histogram takes whole chunks per work item; others take
@@ -1147,14 +1180,13 @@ int ngap_get_reports(ngap_engine *eng, uint64_t *out, uint64_t cap, uint64_t *n_
     if (ctx.last_count > ctx.report_cap)
       return ngap_fail(NGAP_ERR_OVERFLOW, "reports exceeded the capacity of the last run");
     HIP_TRY(hipSetDevice(eng->device));
-    std::vector<uint64_t> v;
-    int rc = sorted_reports(ctx, v);
-    if (rc) return rc;
-    *n_out = v.size();
-    if (out) {
-      uint64_t n = std::min<uint64_t>(cap, v.size());
-      for (uint64_t i = 0; i < n; i++) out[i] = (v[i] << 32) | (v[i] >> 32);
-    }
+    if (const int rc = sort_reports(eng, ctx)) return rc;
+    *n_out = ctx.unique_reports;
+    const uint64_t n = out ? std::min<uint64_t>(cap, ctx.unique_reports) : 0;
+    if (n && ctx.sorted_on_host)
+      std::copy(ctx.host_reports + 1, ctx.host_reports + 1 + n, out);
+    else if (n)
+      HIP_TRY(hipMemcpy(out, ctx.reports.p, n * 8, hipMemcpyDeviceToHost));
     return NGAP_OK;
   });
 }

@@ -94,6 +94,7 @@ struct InputStage {
 };
 
 // One stream with its own per-run buffers and captured graph.
+constexpr uint32_t kSmallReports = 16384;  // sorted by rank, above by radix (reports.hip)
 struct RunCtx {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -107,6 +108,14 @@ struct RunCtx {
   uint32_t root_boost = 1;      // doubles (up to 64x) after a root area overflowed,
   uint64_t root_gen = 0;        // for this engine generation (groups and input)
   uint64_t report_cap = 0, last_count = 0;
+  // the last run's reports once ngap_get_reports sorted them (until the next
+  // launch): unique_reports of them, encoded, in host_reports[1..] (pinned) or
+  // in `reports`
+  bool sorted = false, sorted_on_host = false;
+  uint64_t unique_reports = 0;
+  uint64_t *host_reports = nullptr;  // kSmallReports + 1 words behind host_cnt
+  uint64_t *report_slots = nullptr;  // the rank sort's, behind the counters; ~0 = empty
+  DevBuf sort_area;                  // the radix sort's
   bool last_report_off = false, have_run = false;
   bool tasks_resident = false;  // `tasks` holds last_tasks
   bool last_traces = false;     // the last run recorded items per work item
@@ -135,6 +144,12 @@ struct Mapping {
 
 bool map_algorithm(int algorithm, int depth_req, int loaded_depth, Mapping &m, std::string &err);
 uint32_t lds_bytes(uint32_t ring = kRing);
+
+// Sorts ctx's last n reports (offsets below 2^offset_bits) on the device and
+// encodes them (reports.hip): into ctx.host_reports[1..] up to kSmallReports,
+// else in place in ctx.reports.  Sets ctx.unique_reports and
+// ctx.sorted_on_host.
+hipError_t sort_reports_device(RunCtx &ctx, uint64_t n, uint32_t offset_bits);
 
 // Kernel launchers (kernels.hip).  launch_reset clears the run's counters
 // and n per-work-item flags (and root counts, when given); launch_roots runs
