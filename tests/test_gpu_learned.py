@@ -5,7 +5,7 @@ import pytest
 
 import oracle
 from oracle import mlp_ref
-from ngap_amd import learned, synth
+from ngap_amd import NgapError, learned, synth
 from ngap_amd.mlp import MLP
 
 pytestmark = pytest.mark.gpu
@@ -109,4 +109,73 @@ def test_learned_schedule_end_to_end(engine):
                     fallback=True)
     assert np.array_equal(engine.reports(), want)
     assert st["num_tasks"] == len(ctasks)
+    m.close()
+
+
+@pytest.mark.parametrize("n", [15, 16, 31, 32, 33, 512, 16384 + 1, 40000])
+def test_gradient_tiles_match_oracle(n):
+    """Sizes around a tile (32 samples), and several tiles per workgroup."""
+    rng = np.random.default_rng(n)
+    m = MLP(0, seed=4)
+    p = m.params.astype(np.float64)
+    x = rng.normal(size=(n, 264)).astype(np.float32)
+    t = rng.normal(size=n).astype(np.float32)
+    say("mlp tiles", n)
+    y_ref, _ = mlp_ref.forward(p, x.astype(np.float64))
+    assert np.allclose(m.predict(x), y_ref, rtol=1e-4, atol=1e-4)
+    g, loss = m.gradient(x, t)
+    g_ref, loss_ref = mlp_ref.gradient(p, x.astype(np.float64), t.astype(np.float64))
+    assert np.isclose(loss, loss_ref, rtol=1e-4)
+    assert np.max(np.abs(g - g_ref)) <= 1e-4 * np.abs(g_ref).max() + 1e-6
+    m.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 49153, 100000])
+def test_pairs_rounds_match_dense(mlp, n):
+    """Pairs around a wave's round (16) and a full grid of rounds (49,152)."""
+    rng = np.random.default_rng(n)
+    hist = rng.random((33, 256)).astype(np.float32) / 128
+    stats = rng.random((17, 8)).astype(np.float32)
+    pairs = np.stack([rng.integers(0, 17, n), rng.integers(0, 33, n)], 1)
+    say("mlp pairs", n)
+    y = mlp.predict_pairs(hist, stats, pairs)
+    assert np.array_equal(y, mlp.predict(learned.features(hist, stats, pairs)))
+    for bad in ((17, 0), (0, 33)):
+        wrong = pairs.copy()
+        wrong[n // 2] = bad
+        with pytest.raises(NgapError, match="pair out of range"):
+            mlp.predict_pairs(hist, stats, wrong)
+
+
+def test_training_steps_match_oracle():
+    """Mini-batches with a remainder, shuffled rows, Adam: parameters after
+    two epochs against the same steps in float64."""
+    rng = np.random.default_rng(6)
+    n, batch = 1000, 300
+    x = rng.random((n, 264)).astype(np.float32)
+    t = x[:, 0].astype(np.float32)
+    m = MLP(0, seed=8)
+    p = m.params.astype(np.float64)
+    say("mlp training steps")
+    loss = m.train(x, t, epochs=2, batch=batch, lr=1e-3, seed=11)
+    z, idx, step = 11, list(range(n)), 0
+    mom, var = np.zeros_like(p), np.zeros_like(p)
+    for _ in range(2):
+        for i in range(n - 1, 0, -1):
+            z = (z * 6364136223846793005 + 1442695040888963407) & (2**64 - 1)
+            j = (z >> 33) % (i + 1)
+            idx[i], idx[j] = idx[j], idx[i]
+        total = 0.0
+        for a in range(0, n, batch):
+            rows = idx[a:a + batch]
+            g, l = mlp_ref.gradient(p, x[rows].astype(np.float64), t[rows].astype(np.float64))
+            total += l * len(rows)
+            step += 1
+            mom = 0.9 * mom + 0.1 * g
+            var = 0.999 * var + 0.001 * g * g
+            p = p - 1e-3 * (mom / (1 - 0.9**step)) / (np.sqrt(var / (1 - 0.999**step)) + 1e-8)
+    # eight steps of at most 1e-3 per parameter, each to FP32 accuracy but for
+    # parameters whose gradient is itself rounding noise
+    assert np.linalg.norm(m.params - p) <= 1e-5 * np.linalg.norm(p)
+    assert np.isclose(loss, total / n, rtol=1e-4)
     m.close()
