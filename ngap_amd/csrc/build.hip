@@ -33,7 +33,6 @@
 
 #include <algorithm>
 #include <cstring>
-#include <thread>
 
 #include "runtime.h"
 
@@ -481,6 +480,7 @@ __global__ void k_x3_flags(const uint32_t *xmask1, const uint32_t *x2rep, uint32
 struct Prim {
   hipStream_t s;
   DevBuf tmp;
+  Prim(hipStream_t stream, Slab &slab) : s(stream), tmp(slab) {}
   hipError_t sort(const uint64_t *in, uint64_t *out, uint64_t n, int bits) {
     if (n == 0) return hipSuccess;
     size_t bytes = 0;
@@ -489,33 +489,16 @@ struct Prim {
     if ((e = tmp.reserve(bytes)) != hipSuccess) return e;
     return rocprim::radix_sort_keys(tmp.p, bytes, in, out, n, 0, bits, s);
   }
-  // out[i] = in[0] + ... + in[i-1], n + 1 entries (out[n] = total)
+  // out[i] = in[0] + ... + in[i-1], n + 1 entries (out[n] = total; in[n] is
+  // read, whatever it holds)
   template <class In, class Out>
   hipError_t exscan(const In *in, Out *out, uint64_t n) {
     size_t bytes = 0;
     hipError_t e =
-        rocprim::exclusive_scan(nullptr, bytes, in, out, Out(0), n, rocprim::plus<Out>(), s);
+        rocprim::exclusive_scan(nullptr, bytes, in, out, Out(0), n + 1, rocprim::plus<Out>(), s);
     if (e != hipSuccess) return e;
     if ((e = tmp.reserve(bytes)) != hipSuccess) return e;
-    if (n && (e = rocprim::exclusive_scan(tmp.p, bytes, in, out, Out(0), n,
-                                          rocprim::plus<Out>(), s)) != hipSuccess)
-      return e;
-    return total(in, out, n);
-  }
-  // out[n] = out[n-1] + in[n-1]
-  template <class In, class Out>
-  hipError_t total(const In *in, Out *out, uint64_t n) {
-    if (n == 0) return hipMemsetAsync(out, 0, sizeof(Out), s);
-    Out a = 0;
-    In b = 0;
-    hipError_t e = hipMemcpyAsync(&a, out + n - 1, sizeof(Out), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&b, in + n - 1, sizeof(In), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return e;
-    a += (Out)b;
-    e = hipMemcpyAsync(out + n, &a, sizeof(Out), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    return e;
+    return rocprim::exclusive_scan(tmp.p, bytes, in, out, Out(0), n + 1, rocprim::plus<Out>(), s);
   }
   template <class In, class Out>
   hipError_t inscan(const In *in, Out *out, uint64_t n) {
@@ -611,43 +594,59 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
   }
   const uint64_t N = sb[G], E = eb[G], A = ab[G], Q = qb[G];
   img.total_states = N;
-  // upload: one pinned staging buffer, copied in by host threads
+  // upload, through the engine's pinned blocks: host threads gather one block
+  // from the groups' arrays while the other's copy runs.  (A pinned buffer of
+  // the whole size, filled, copied and freed per load, took 8 ms for 76 MB.)
   const uint64_t o_row = 0, o_col = o_row + (N + G) * 4, o_sets = o_col + E * 4,
                  o_attr = o_sets + N * 32, o_aas = o_attr + ((N + 3) & ~3ull),
                  o_sod = o_aas + A * 4, o_end = o_sod + Q * 4;
-  DevBuf d_in;
+  Slab &slab = eng->build_slab;
+  slab.expect(4 * o_end + ((depth >= 3 ? 160ull : 8ull) << 20));
+  DevBuf d_in(slab);
   HIP_TRY(d_in.reserve(o_end + 16));
   {
-    uint8_t *pin = nullptr;
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&pin), o_end + 16, hipHostMallocDefault));
-    std::vector<std::thread> pool;
-    const unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    for (unsigned t = 0; t < nt; t++)
-      pool.emplace_back([&, t] {
-        for (int32_t g = (int32_t)t; g < G; g += (int32_t)nt) {
-          const HostGroup &h = hg[g];
-          const int n = h.num_states;
-          if (n > 0) {
-            memcpy(pin + o_row + ((uint64_t)sb[g] + g) * 4, h.row, (size_t)(n + 1) * 4);
-            memcpy(pin + o_sets + (uint64_t)sb[g] * 32, h.sets, (size_t)n * 32);
-            memcpy(pin + o_attr + sb[g], h.attrs, (size_t)n);
-          } else {
-            const int32_t zero = 0;
-            memcpy(pin + o_row + ((uint64_t)sb[g] + g) * 4, &zero, 4);
-          }
-          if (eb[g + 1] > eb[g])
-            memcpy(pin + o_col + eb[g] * 4, h.col, (size_t)(eb[g + 1] - eb[g]) * 4);
-          if (ab[g + 1] > ab[g])
-            memcpy(pin + o_aas + ab[g] * 4, h.aas, (size_t)(ab[g + 1] - ab[g]) * 4);
-          if (qb[g + 1] > qb[g])
-            memcpy(pin + o_sod + qb[g] * 4, h.sod, (size_t)(qb[g + 1] - qb[g]) * 4);
+    struct Part {
+      uint64_t at;
+      const void *src;
+      uint64_t n;
+    };
+    std::vector<Part> parts;  // ascending; only the attributes' padding is in none
+    parts.reserve((size_t)G * 6);
+    const auto add = [&](uint64_t at, const void *src, uint64_t n) {
+      if (n) parts.push_back(Part{at, src, n});
+    };
+    static const int32_t kZero = 0;
+    for (int32_t g = 0; g < G; g++) {
+      const uint64_t at = o_row + ((uint64_t)sb[g] + g) * 4;
+      if (hg[g].num_states > 0) add(at, hg[g].row, ((uint64_t)hg[g].num_states + 1) * 4);
+      else add(at, &kZero, 4);
+    }
+    for (int32_t g = 0; g < G; g++) add(o_col + eb[g] * 4, hg[g].col, (eb[g + 1] - eb[g]) * 4);
+    for (int32_t g = 0; g < G; g++)
+      add(o_sets + (uint64_t)sb[g] * 32, hg[g].sets, (uint64_t)(sb[g + 1] - sb[g]) * 32);
+    for (int32_t g = 0; g < G; g++) add(o_attr + sb[g], hg[g].attrs, sb[g + 1] - sb[g]);
+    for (int32_t g = 0; g < G; g++) add(o_aas + ab[g] * 4, hg[g].aas, (ab[g + 1] - ab[g]) * 4);
+    for (int32_t g = 0; g < G; g++) add(o_sod + qb[g] * 4, hg[g].sod, (qb[g + 1] - qb[g]) * 4);
+    InputStage &stg = eng->stage;
+    HIP_TRY(stg.init());
+    for (uint64_t off = 0, k = 0; off < o_end; off += InputStage::kBlock, k++) {
+      const size_t len = (size_t)std::min<uint64_t>(InputStage::kBlock, o_end - off);
+      uint8_t *st = stg.buf[k & 1];
+      if (k >= 2) HIP_TRY(hipEventSynchronize(stg.done[k & 1]));  // its last copy is done
+      stg.pool->run_parts(len, [&](size_t, size_t a, size_t b) {
+        const uint64_t from = off + a, to = off + b;
+        auto x = std::upper_bound(parts.begin(), parts.end(), from,
+                                  [](uint64_t v, const Part &q) { return v < q.at; });
+        if (x != parts.begin()) --x;
+        for (; x != parts.end() && x->at < to; ++x) {
+          const uint64_t lo = std::max(from, x->at), hi = std::min(to, x->at + x->n);
+          if (lo < hi)
+            memcpy(st + (lo - off), static_cast<const uint8_t *>(x->src) + (lo - x->at), hi - lo);
         }
       });
-    for (auto &t : pool) t.join();
-    hipError_t e = hipMemcpyAsync(d_in.p, pin, o_end, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipHostFree(pin);
-    HIP_TRY(e);
+      HIP_TRY(hipMemcpyAsync(d_in.as<uint8_t>() + off, st, len, hipMemcpyHostToDevice, s));
+      HIP_TRY(hipEventRecord(stg.done[k & 1], s));
+    }
   }
   uint8_t *in = d_in.as<uint8_t>();
   const int32_t *row_l = reinterpret_cast<const int32_t *>(in + o_row);
@@ -657,12 +656,20 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
   const int32_t *aas_l = reinterpret_cast<const int32_t *>(in + o_aas);
   const int32_t *sod_l = reinterpret_cast<const int32_t *>(in + o_sod);
 
-  Prim prim{s, {}};
-  DevBuf d_sb, d_eb, d_ab, d_qb, d_sgrp, d_grow, d_isaas, d_err, d_cnt8;
-  HIP_TRY(d_sb.upload(sb));
-  HIP_TRY(d_eb.upload(eb));
-  HIP_TRY(d_ab.upload(ab));
-  HIP_TRY(d_qb.upload(qb));
+  // (on stream s like everything here: the slab's memory may still be in use there)
+  const auto upload = [s](DevBuf &d, const auto &v) {
+    hipError_t e = d.reserve(v.size() * sizeof(v[0]));
+    if (e == hipSuccess && !v.empty())
+      e = hipMemcpyAsync(d.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s);
+    return e;
+  };
+  Prim prim(s, slab);
+  DevBuf d_sb(slab), d_eb(slab), d_ab(slab), d_qb(slab), d_sgrp(slab), d_grow(slab),
+      d_isaas(slab), d_err(slab), d_cnt8(slab);
+  HIP_TRY(upload(d_sb, sb));
+  HIP_TRY(upload(d_eb, eb));
+  HIP_TRY(upload(d_ab, ab));
+  HIP_TRY(upload(d_qb, qb));
   HIP_TRY(d_sgrp.reserve(N * 2 + 2));
   HIP_TRY(d_grow.reserve(N * 8 + 8));
   HIP_TRY(d_isaas.reserve(N + 1));
@@ -685,7 +692,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     if (e0) return NGAP_ERR_INVALID;
   }
   // distinct successors
-  DevBuf d_ekeys, d_esorted, d_dkeys, d_nsucc, d_indeg, d_soff;
+  DevBuf d_ekeys(slab), d_esorted(slab), d_dkeys(slab), d_nsucc(slab), d_indeg(slab), d_soff(slab);
   HIP_TRY(d_ekeys.reserve(E * 8 + 8));
   HIP_TRY(d_esorted.reserve(E * 8 + 8));
   hipLaunchKernelGGL(k_edge_keys, dim3(grid_for(N)), dim3(kThreads), 0, s, d_grow.as<uint64_t>(),
@@ -714,7 +721,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
   HIP_TRY(d_soff.reserve((N + 1) * 8));
   HIP_TRY(prim.exscan(d_nsucc.as<uint32_t>(), d_soff.as<uint64_t>(), N));
   // tags, tests, records
-  DevBuf d_tag, d_test, d_ext, d_extscan, d_recbase;
+  DevBuf d_tag(slab), d_test(slab), d_ext(slab), d_extscan(slab), d_recbase(slab);
   HIP_TRY(d_tag.reserve(N * 4 + 4));
   HIP_TRY(d_test.reserve(N * 4 + 4));
   HIP_TRY(d_ext.reserve(N * 4 + 4));
@@ -775,11 +782,13 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     m.num_states = (uint32_t)hg[g].num_states;
     m.num_aas = (uint32_t)std::max(0, hg[g].num_aas);
   }
-  HIP_TRY(eng->d_meta.upload(img.meta));
+  HIP_TRY(upload(eng->d_meta, img.meta));
   sz.meta = (uint64_t)G * sizeof(GroupMeta);
 
   // memo level 1
-  DevBuf d_cnt, d_off, d_keys, d_sorted, d_ent[kMaxMemoDepth];
+  static_assert(kMaxMemoDepth == 3, "one buffer a level");
+  DevBuf d_cnt(slab), d_off(slab), d_keys(slab), d_sorted(slab);
+  DevBuf d_ent[kMaxMemoDepth] = {DevBuf(slab), DevBuf(slab), DevBuf(slab)};
   uint64_t nent[kMaxMemoDepth] = {0, 0, 0};
   HIP_TRY(d_cnt.reserve(A * 4 + 4));
   HIP_TRY(d_off.reserve((A + 1) * 8));
@@ -799,8 +808,8 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
   HIP_TRY(prim.unique(d_sorted.as<uint64_t>(), d_ent[0].as<uint64_t>(), T, &nent[0], d_cnt8));
   {
     const uint64_t K1 = (uint64_t)G * 256;
-    DevBuf d_c1, d_r1;
-    HIP_TRY(d_c1.reserve(K1 * 4));
+    DevBuf d_c1(slab), d_r1(slab);
+    HIP_TRY(d_c1.reserve(K1 * 4 + 4));
     HIP_TRY(d_r1.reserve(K1 * 4));
     HIP_TRY(hipMemsetAsync(d_c1.p, 0, K1 * 4, s));
     HIP_TRY(hipMemsetAsync(d_r1.p, 0, K1 * 4, s));
@@ -820,8 +829,8 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     hipLaunchKernelGGL(k_mask1, dim3(grid_for(K1)), dim3(kThreads), 0, s, d_c1.as<uint32_t>(),
                        d_r1.as<uint32_t>(), (uint32_t)G, eng->d_mask1.as<uint32_t>());
     // cross-group byte index
-    DevBuf d_xc;
-    HIP_TRY(d_xc.reserve(256 * 4));
+    DevBuf d_xc(slab);
+    HIP_TRY(d_xc.reserve(257 * 4));
     HIP_TRY(eng->d_xr1.reserve(257 * 4));
     HIP_TRY(eng->d_xmask1.reserve(8 * 4));
     HIP_TRY(hipMemsetAsync(eng->d_xmask1.p, 0, 32, s));
@@ -847,7 +856,8 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(hipStreamSynchronize(s));
   }
   // levels 2 and 3
-  DevBuf d_lgrp[kMaxMemoDepth], d_lgram[kMaxMemoDepth];
+  DevBuf d_lgrp[kMaxMemoDepth] = {DevBuf(slab), DevBuf(slab), DevBuf(slab)};
+  DevBuf d_lgram[kMaxMemoDepth] = {DevBuf(slab), DevBuf(slab), DevBuf(slab)};
   uint64_t nlists[kMaxMemoDepth] = {(uint64_t)G * 256, 0, 0};
   for (int d = 2; d <= depth; d++) {
     const uint64_t n = nent[d - 2];
@@ -876,7 +886,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     }
     const uint64_t *ent = d_ent[d - 1].as<uint64_t>();
     // lists: runs of equal (group, d-gram)
-    DevBuf d_flag, d_runscan;
+    DevBuf d_flag(slab), d_runscan(slab);
     HIP_TRY(d_flag.reserve(m * 4 + 4));
     HIP_TRY(d_runscan.reserve(m * 4 + 4));
     hipLaunchKernelGGL(k_run_starts, dim3(grid_for(m)), dim3(kThreads), 0, s, ent, m,
@@ -899,7 +909,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(hipGetLastError());
     // rank table
     const uint64_t pairs = d == 2 ? (uint64_t)G * 2048 : nlists[1] * 8;
-    DevBuf d_words, d_pc, d_ranks;
+    DevBuf d_words(slab), d_pc(slab), d_ranks(slab);
     HIP_TRY(d_words.reserve(pairs * 4 + 4));
     HIP_TRY(d_pc.reserve(pairs * 4 + 4));
     HIP_TRY(d_ranks.reserve((pairs + 1) * 4));
@@ -932,7 +942,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
   d_sorted.release();
   if (depth >= 2) {
     const uint64_t L2 = nlists[1];
-    DevBuf d_k, d_o, d_c;
+    DevBuf d_k(slab), d_o(slab), d_c(slab);
     HIP_TRY(d_k.reserve(L2 * 8 + 8));
     HIP_TRY(d_o.reserve(L2 * 8 + 8));
     HIP_TRY(d_c.reserve(65537 * 4));
@@ -959,7 +969,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     hipLaunchKernelGGL(k_x2rep, dim3(grid_for(L2)), dim3(kThreads), 0, s,
                        d_lgram[1].as<uint32_t>(), eng->d_nrep[1].as<uint32_t>(), L2,
                        eng->d_x2rep.as<uint32_t>());
-    DevBuf d_k, d_o, d_start, d_contrib, d_xpos, d_big;
+    DevBuf d_k(slab), d_o(slab), d_start(slab), d_contrib(slab), d_xpos(slab), d_big(slab);
     HIP_TRY(d_k.reserve(L3 * 8 + 8));
     HIP_TRY(d_o.reserve(L3 * 8 + 8));
     HIP_TRY(d_start.reserve(L3 * 4 + 4));

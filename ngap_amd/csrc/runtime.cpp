@@ -39,17 +39,83 @@ hipError_t DevBuf::reserve(size_t bytes) {
   if (bytes <= n && p) return hipSuccess;
   release();
   size_t want = bytes ? bytes : 8;
-  hipError_t e = hipMalloc(&p, want);
+  hipError_t e = slab ? slab->take(want, &p) : hipMalloc(&p, want);
   if (e == hipSuccess) n = want;
   else p = nullptr;
   return e;
 }
 
 void DevBuf::release() {
-  if (p && owned) (void)hipFree(p);
+  if (p && owned) {
+    if (slab) slab->give(p);
+    else (void)hipFree(p);
+  }
   p = nullptr;
   n = 0;
   owned = true;
+}
+
+hipError_t Slab::take(size_t bytes, void **p) {
+  constexpr size_t kAlign = 256, kFirst = 4u << 20;
+  const size_t want = (bytes + kAlign - 1) / kAlign * kAlign;
+  *p = nullptr;
+  auto best = free_.end();
+  for (auto f = free_.begin(); f != free_.end(); ++f)
+    if (f->n >= want && (best == free_.end() || f->n < best->n)) best = f;
+  if (best == free_.end()) {
+    // the chunks double what there is; where that much is not free, what is asked for
+    char *c = nullptr;
+    size_t n = std::max(want, total_ ? total_ : std::max(expected_, kFirst));
+    hipError_t e = hipMalloc(reinterpret_cast<void **>(&c), n);
+    if (e != hipSuccess && n > want) {
+      (void)hipGetLastError();
+      n = want;
+      e = hipMalloc(reinterpret_cast<void **>(&c), n);
+    }
+    if (e != hipSuccess) return e;
+    total_ += n;
+    chunks_.push_back(c);
+    best = free_.insert(free_.end(), Piece{chunks_.size() - 1, 0, n});
+  }
+  const Piece got{best->chunk, best->at, want};
+  best->at += want;
+  best->n -= want;
+  if (best->n == 0) free_.erase(best);
+  *p = chunks_[got.chunk] + got.at;
+  used_.emplace_back(*p, got);
+  return hipSuccess;
+}
+
+void Slab::give(void *p) {
+  for (size_t i = 0; i < used_.size(); i++) {
+    if (used_[i].first != p) continue;
+    const Piece x = used_[i].second;
+    used_[i] = used_.back();
+    used_.pop_back();
+    auto f = free_.begin();
+    while (f != free_.end() && (f->chunk < x.chunk || (f->chunk == x.chunk && f->at < x.at))) ++f;
+    f = free_.insert(f, x);
+    const auto joins = [](const Piece &a, const Piece &b) {
+      return a.chunk == b.chunk && a.at + a.n == b.at;
+    };
+    if (f + 1 != free_.end() && joins(*f, *(f + 1))) {
+      f->n += (f + 1)->n;
+      free_.erase(f + 1);
+    }
+    if (f != free_.begin() && joins(*(f - 1), *f)) {
+      (f - 1)->n += f->n;
+      free_.erase(f);
+    }
+    return;
+  }
+}
+
+void Slab::clear() {
+  for (char *c : chunks_) (void)hipFree(c);
+  chunks_.clear();
+  free_.clear();
+  used_.clear();
+  expected_ = total_ = 0;
 }
 
 RunCtx::~RunCtx() {
@@ -738,15 +804,9 @@ namespace {
 // the arrays (a very large image), they stay where they are.
 int pack_image(ngap_engine *eng) {
   using ngapamd::DevBuf;
-  DevBuf *arr[] = {&eng->d_succ4,  &eng->d_cls,     &eng->d_xs3,     &eng->d_xp3,
-                   &eng->d_list[0], &eng->d_list[1], &eng->d_list[2], &eng->d_sel[0],
-                   &eng->d_sel[1], &eng->d_sel[2],  &eng->d_beg[0],  &eng->d_beg[1],
-                   &eng->d_beg[2], &eng->d_nrep[0], &eng->d_nrep[1], &eng->d_nrep[2],
-                   &eng->d_xr1,    &eng->d_xe1,     &eng->d_xmask1,  &eng->d_xr2,
-                   &eng->d_xe2,    &eng->d_xsod,    &eng->d_x2rep,   &eng->d_meta,
-                   &eng->d_sod,    &eng->d_mask1};
+  const auto arr = eng->image_arrays();
   constexpr size_t kBig = 2u << 20, kSmall = 256;
-  constexpr int kN = sizeof(arr) / sizeof(arr[0]);
+  constexpr int kN = (int)std::tuple_size<decltype(eng->image_arrays())>::value;
   size_t off[kN], total = 0;
   for (int pass = 0; pass < 2; pass++)
     for (int i = 0; i < kN; i++) {
@@ -756,13 +816,16 @@ int pack_image(ngap_engine *eng) {
       off[i] = total;
       total += arr[i]->n;
     }
-  DevBuf arena;
   if (total == 0) return NGAP_OK;
-  if (arena.reserve(total) != hipSuccess) {
-    (void)hipGetLastError();
-    return NGAP_OK;
+  // an arena of the last load that fits, and is no more than twice as large, stays
+  if (eng->d_arena.n < total || eng->d_arena.n / 2 > total) {
+    eng->d_arena.release();
+    if (eng->d_arena.reserve(total) != hipSuccess) {
+      (void)hipGetLastError();
+      return NGAP_OK;
+    }
   }
-  char *base = arena.as<char>();
+  char *base = eng->d_arena.as<char>();
   for (int i = 0; i < kN; i++)
     if (arr[i]->p)
       HIP_TRY(hipMemcpyAsync(base + off[i], arr[i]->p, arr[i]->n, hipMemcpyDeviceToDevice,
@@ -776,8 +839,7 @@ int pack_image(ngap_engine *eng) {
     arr[i]->n = n;
     arr[i]->owned = false;
   }
-  std::swap(eng->d_arena.p, arena.p);  // the previous arena is freed on return
-  std::swap(eng->d_arena.n, arena.n);
+  eng->build_slab.clear();
   return NGAP_OK;
 }
 
@@ -809,10 +871,19 @@ int ngap_load_groups_ex(ngap_engine *eng, const ngap_group_desc *groups, int32_t
     eng->ctx.have_run = false;
     eng->ctx.drop_graph();
     const int depth = max_depth < 1 ? 1 : max_depth;
+    for (DevBuf *d : eng->image_arrays()) {
+      d->release();
+      d->slab = build == NGAP_BUILD_DEVICE ? &eng->build_slab : nullptr;
+    }
+    eng->build_slab.clear();  // (holds what a failed load, or one without an arena, left)
     if (build == NGAP_BUILD_DEVICE) {
       const int rc = build_image_device(eng, hg.data(), num_groups, depth, eng->ctx.stream,
                                         eng->img, eng->img_sizes, err);
-      if (rc) return err.empty() ? rc : ngap_fail(rc, err);
+      if (rc) {
+        for (DevBuf *d : eng->image_arrays()) d->release();
+        eng->build_slab.clear();
+        return err.empty() ? rc : ngap_fail(rc, err);
+      }
     } else {
       if (!build_image(hg.data(), num_groups, depth, eng->img, err))
         return ngap_fail(NGAP_ERR_INVALID, err);

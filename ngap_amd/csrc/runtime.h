@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include <memory>
@@ -31,11 +33,41 @@ namespace ngapamd {
 constexpr uint32_t kRing = 256, kRbuf = 128, kDc = 256;
 constexpr uint32_t kMinRing = 64, kMaxRing = 2048;  // batched ring_capacity range
 
+// Device memory for one load: the builder's temporaries and the arrays it
+// builds come out of a few large chunks, by best fit, and go back to them.  What
+// is given back is handed out again without waiting, so all of it is used on one
+// stream.  (A load made 65 hipMalloc and 65 hipFree calls, 8.5 of its 20 ms at
+// 128 automata of up to 50,000 states: each free waits for the device and unmaps.
+// With a few chunks, and the uploads through the pinned blocks, it takes 5.5 ms.)
+class Slab {
+ public:
+  Slab() = default;
+  Slab(const Slab &) = delete;
+  Slab &operator=(const Slab &) = delete;
+  ~Slab() { clear(); }
+  // the size of the first chunk, where the caller can tell what it will need
+  void expect(size_t bytes) { expected_ = bytes; }
+  hipError_t take(size_t bytes, void **p);
+  void give(void *p);
+  void clear();  // frees the chunks; nothing taken may be used any more
+
+ private:
+  struct Piece {
+    size_t chunk, at, n;
+  };
+  std::vector<char *> chunks_;
+  std::vector<Piece> free_;  // ascending (chunk, at), neighbours joined
+  std::vector<std::pair<void *, Piece>> used_;
+  size_t expected_ = 0, total_ = 0;
+};
+
 struct DevBuf {
   void *p = nullptr;
   size_t n = 0;
   bool owned = true;  // false: a view into another buffer (the image arena)
+  Slab *slab = nullptr;  // where its memory comes from (null: hipMalloc)
   DevBuf() = default;
+  explicit DevBuf(Slab &from) : slab(&from) {}
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
   ~DevBuf() { release(); }
@@ -52,8 +84,9 @@ struct DevBuf {
   T *as() const { return reinterpret_cast<T *>(p); }
 };
 
-// Pinned staging of ngap_set_input: two blocks, so that host threads fill one
-// while the other's copy to the device runs.
+// Pinned staging of ngap_set_input and of the groups' arrays at a load: two
+// blocks, so that host threads fill one while the other's copy to the device
+// runs.
 struct InputStage {
   static constexpr size_t kBlock = 8u << 20;
   uint8_t *buf[2] = {nullptr, nullptr};
@@ -173,14 +206,21 @@ struct ngap_engine {
   int batched_per_cu[12 * ngapamd::kBatchedKinds] = {0};
   ngapamd::Image img;
   bool loaded = false;
+  ngapamd::Slab build_slab;  // the device builder's memory while a load runs
   ngapamd::DevBuf d_meta, d_succ4, d_cls, d_sod, d_mask1;
   ngapamd::DevBuf d_beg[ngapamd::kMaxMemoDepth], d_nrep[ngapamd::kMaxMemoDepth],
       d_list[ngapamd::kMaxMemoDepth], d_sel[ngapamd::kMaxMemoDepth];
   ngapamd::DevBuf d_xr1, d_xe1, d_xmask1, d_xr2, d_xe2, d_xsod, d_xs3, d_xp3, d_x2rep;
+  std::array<ngapamd::DevBuf *, 26> image_arrays() {
+    return {&d_succ4, &d_cls, &d_xs3, &d_xp3, &d_list[0], &d_list[1], &d_list[2], &d_sel[0],
+            &d_sel[1], &d_sel[2], &d_beg[0], &d_beg[1], &d_beg[2], &d_nrep[0], &d_nrep[1],
+            &d_nrep[2], &d_xr1, &d_xe1, &d_xmask1, &d_xr2, &d_xe2, &d_xsod, &d_x2rep, &d_meta,
+            &d_sod, &d_mask1};
+  }
   // one allocation holding every image array above (they are views into it)
   ngapamd::DevBuf d_arena;
   ngapamd::DevBuf d_input;
-  ngapamd::InputStage stage;    // pinned staging of ngap_set_input
+  ngapamd::InputStage stage;    // pinned staging of ngap_set_input and of loads
   uint64_t chunk_len = 0;
   uint32_t num_seg = 0;
   bool have_input = false;

@@ -126,3 +126,21 @@ def test_device_build_rejects_malformed_groups(engine):
             msgs.append(str(ei.value))
         assert msgs[0] == msgs[1], msgs
     engine.load_groups([good], 3)  # the engine stays usable
+
+
+@pytest.mark.parametrize("sizes", [[90000] * 8, [40], [300000, 20, 260000]])
+def test_loads_after_each_other(engine, sizes):
+    # uploads of one pinned block and of several, a group's arrays across the
+    # blocks' borders, an arena that stays and one that is replaced
+    rng = np.random.default_rng(len(sizes))
+    groups = [synth.regex_group(rng, s) for s in sizes]
+    for depth in (2, 1):
+        compare_builds(engine, groups, depth, f"loads {sizes}")
+        compare_builds(engine, groups[-1:], depth, "its last group")
+    with pytest.raises(NgapError):  # and after a load that failed half way
+        bad = groups[0]
+        col = bad.col.copy()
+        col[-1] = bad.num_states
+        engine.load_groups([Group(bad.row, col, bad.sets, bad.attrs, bad.aas, bad.sod)], 2,
+                           build="device")
+    compare_builds(engine, groups, 3, f"loads {sizes}")
