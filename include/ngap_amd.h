@@ -186,8 +186,8 @@ typedef struct {
 int ngap_image_info(ngap_engine *eng, ngap_image_summary *info);
 
 /* Copies the device image array `name` (meta, succ4, cls, sod, beg1-3,
- * nrep1-3, list1-3, sel2, sel3, mask1, xr1, xe1, xmask1, xr2, xe2, xsod, xs3,
- * xp3, x2rep; layout in ngap_amd/csrc/layout.h) into out (at most cap bytes);
+ * nrep1-3, list1-3, filt1-3, sel2, sel3, mask1, xr1, xe1, xmask1, xr2, xe2,
+ * xsod, xs3, xp3, xf3, xb3, x2rep; layout in ngap_amd/csrc/layout.h) into out (at most cap bytes);
  * *n_bytes gets its size (out may be NULL to query it). */
 int ngap_image_array(ngap_engine *eng, const char *name, void *out, uint64_t cap,
                      uint64_t *n_bytes);

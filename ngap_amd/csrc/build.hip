@@ -162,6 +162,22 @@ __global__ void k_tags(const uint32_t *sb, const uint16_t *sgrp, const uint8_t *
   }
 }
 
+// Next-byte filters of the states (layout.h): their successors' classes.
+__global__ void k_filters(const uint32_t *sb, const uint16_t *sgrp, const uint64_t *succ_off,
+                          const uint64_t *dkeys, const uint32_t *cls, uint64_t N,
+                          uint32_t *nfilt) {
+  GRID_LOOP(s, N) {
+    const uint64_t base = sb[sgrp[s]];
+    uint32_t f = 0;
+    for (uint64_t q = succ_off[s]; q < succ_off[s + 1]; q++) {
+      const uint64_t u = base + (dkeys[q] & kKeyStateMask);
+#pragma unroll
+      for (int w = 0; w < 8; w++) f |= cls[u * 8 + w];
+    }
+    nfilt[s] = filter_of(f);
+  }
+}
+
 // Group record bases: group g's records start at sb[g] + (continuation
 // records of the groups before it).
 __global__ void k_rec_base(const uint32_t *sb, const uint64_t *ext_scan, uint32_t G,
@@ -296,12 +312,15 @@ __global__ void k_run_starts(const uint64_t *ent, uint64_t n, uint32_t *flag) {
 // Lists of a level from its sorted entries: list[j] = tagged state, list
 // starts (beg), reporting entries (nrep), group and d-gram of each list.
 __global__ void k_lists(const uint64_t *ent, uint64_t n, const uint32_t *run_scan,
-                        const uint32_t *sb, const int32_t *tag, int32_t *list, uint32_t *beg,
-                        uint32_t *nrep, uint32_t *lgrp, uint32_t *lgram, uint64_t nlists) {
+                        const uint32_t *sb, const int32_t *tag, const uint32_t *nfilt,
+                        int32_t *list, uint32_t *filt, uint32_t *beg, uint32_t *nrep,
+                        uint32_t *lgrp, uint32_t *lgram, uint64_t nlists) {
   GRID_LOOP(j, n) {
     const uint64_t e = ent[j];
     const uint32_t g = (uint32_t)(e >> kKeyGroupShift);
-    list[j] = tag[sb[g] + (e & kKeyStateMask)];
+    const uint64_t s = sb[g] + (e & kKeyStateMask);
+    list[j] = tag[s];
+    filt[j] = nfilt[s];
     const uint32_t li = run_scan[j];  // inclusive scan of the start flags, minus 1 below
     const bool start = j == 0 || (e >> kKeyGramShift) != (ent[j - 1] >> kKeyGramShift);
     if (start) {
@@ -326,10 +345,12 @@ __global__ void k_l1_counts(const uint64_t *ent, uint64_t n, uint32_t *cnt, uint
 }
 
 __global__ void k_l1_list(const uint64_t *ent, uint64_t n, const uint32_t *sb, const int32_t *tag,
-                          int32_t *list) {
+                          const uint32_t *nfilt, int32_t *list, uint32_t *filt) {
   GRID_LOOP(j, n) {
     const uint64_t e = ent[j];
-    list[j] = tag[sb[(uint32_t)(e >> kKeyGroupShift)] + (e & kKeyStateMask)];
+    const uint64_t s = sb[(uint32_t)(e >> kKeyGroupShift)] + (e & kKeyStateMask);
+    list[j] = tag[s];
+    filt[j] = nfilt[s];
   }
 }
 
@@ -414,9 +435,12 @@ __global__ void k_xe2(const uint64_t *sorted, uint64_t nlists, const uint32_t *b
 }
 
 __global__ void k_x2rep(const uint32_t *lgram, const uint32_t *nrep, uint64_t nlists,
-                        uint32_t *x2rep) {
+                        uint32_t *x2rep, uint32_t *any) {
   GRID_LOOP(li, nlists)
-    if (nrep[li]) atomicOr(&x2rep[lgram[li] >> 5], 1u << (lgram[li] & 31));
+    if (nrep[li]) {
+      atomicOr(&x2rep[lgram[li] >> 5], 1u << (lgram[li] & 31));
+      *any = 1u;
+    }
 }
 
 // x3: lists sorted by (3-gram, list index).  Run starts of equal 3-grams and
@@ -436,23 +460,26 @@ __global__ void k_x3_runs(const uint64_t *sorted, uint64_t n, const uint32_t *be
 }
 
 __global__ void k_x3_fill(const uint64_t *sorted, uint64_t n, const uint32_t *beg,
-                          const int32_t *list3, const uint32_t *lgrp, const uint64_t *xpos,
-                          uint32_t *xs3, uint32_t *xp3, uint32_t *err_big) {
+                          const int32_t *list3, const uint32_t *filt3, const uint32_t *lgrp,
+                          const uint64_t *xpos, uint32_t *xs3, uint32_t *xp3, uint32_t *xf3,
+                          uint32_t *xb3, uint32_t *err_big) {
   GRID_LOOP(j, n) {
     const uint32_t k = (uint32_t)(sorted[j] >> 32);
     const uint32_t li = (uint32_t)sorted[j];
     const bool first = j == 0 || (uint32_t)(sorted[j - 1] >> 32) != k;
     const bool last = j + 1 == n || (uint32_t)(sorted[j + 1] >> 32) != k;
     const uint32_t b0 = beg[li], len = beg[li + 1] - b0;
+    if (first) atomicOr(&xb3[k >> 5], 1u << (k & 31));
     if (first && last && len == 1) {
-      xs3[2 * (uint64_t)k] = (uint32_t)list3[b0];
-      xs3[2 * (uint64_t)k + 1] = kSlotInline | lgrp[li];
+      xs3[2 * (uint64_t)k] = (uint32_t)list3[b0] | slot_filter_low(filt3[b0]);
+      xs3[2 * (uint64_t)k + 1] = kSlotInline | lgrp[li] | slot_filter_high(filt3[b0]);
       continue;
     }
     const uint64_t p = xpos[j];
     for (uint32_t e = 0; e < len; e++) {
       xp3[2 * (p + e)] = (uint32_t)list3[b0 + e];
       xp3[2 * (p + e) + 1] = lgrp[li];
+      xf3[p + e] = filt3[b0 + e];
     }
     if (first) {
       // the run's pairs: from this list's first to the run end's last
@@ -732,6 +759,11 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
                      d_indeg.as<uint32_t>(), N, d_tag.as<int32_t>(), d_test.as<uint32_t>(),
                      d_ext.as<uint32_t>());
   HIP_TRY(prim.exscan(d_ext.as<uint32_t>(), d_extscan.as<uint64_t>(), N));
+  DevBuf d_nfilt(slab);
+  HIP_TRY(d_nfilt.reserve(N * 4 + 4));
+  hipLaunchKernelGGL(k_filters, dim3(grid_for(N)), dim3(kThreads), 0, s, d_sb.as<uint32_t>(),
+                     d_sgrp.as<uint16_t>(), d_soff.as<uint64_t>(), d_dkeys.as<uint64_t>(), sets,
+                     N, d_nfilt.as<uint32_t>());
   hipLaunchKernelGGL(k_rec_base, dim3(grid_for(G + 1)), dim3(kThreads), 0, s,
                      d_sb.as<uint32_t>(), d_extscan.as<uint64_t>(), (uint32_t)G,
                      d_recbase.as<uint64_t>());
@@ -821,9 +853,11 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(eng->d_nrep[0].reserve(K1 * 4));
     HIP_TRY(hipMemcpyAsync(eng->d_nrep[0].p, d_r1.p, K1 * 4, hipMemcpyDeviceToDevice, s));
     HIP_TRY(eng->d_list[0].reserve(nent[0] * 4 + 4));
+    HIP_TRY(eng->d_filt[0].reserve(nent[0] * 4 + 4));
     hipLaunchKernelGGL(k_l1_list, dim3(grid_for(nent[0])), dim3(kThreads), 0, s,
                        d_ent[0].as<uint64_t>(), nent[0], d_sb.as<uint32_t>(),
-                       d_tag.as<int32_t>(), eng->d_list[0].as<int32_t>());
+                       d_tag.as<int32_t>(), d_nfilt.as<uint32_t>(),
+                       eng->d_list[0].as<int32_t>(), eng->d_filt[0].as<uint32_t>());
     HIP_TRY(eng->d_mask1.reserve((uint64_t)G * 64));
     HIP_TRY(hipMemsetAsync(eng->d_mask1.p, 0, (uint64_t)G * 64, s));
     hipLaunchKernelGGL(k_mask1, dim3(grid_for(K1)), dim3(kThreads), 0, s, d_c1.as<uint32_t>(),
@@ -838,6 +872,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
                        nullptr, d_xc.as<uint32_t>(), nullptr, eng->d_xmask1.as<uint32_t>());
     HIP_TRY(prim.exscan(d_xc.as<uint32_t>(), eng->d_xr1.as<uint32_t>(), 256));
     const uint32_t nx1 = read1(s, eng->d_xr1.as<uint32_t>() + 256);
+    img.short_reports = nx1 != 0;
     HIP_TRY(eng->d_xe1.reserve((uint64_t)nx1 * 4 + 4));
     hipLaunchKernelGGL(k_x1, dim3(1), dim3(256), 0, s, d_r1.as<uint32_t>(), (uint32_t)G,
                        eng->d_xr1.as<uint32_t>(), nullptr, eng->d_xe1.as<uint32_t>(), nullptr);
@@ -845,6 +880,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     sz.beg[0] = (K1 + 1) * 4;
     sz.nrep[0] = K1 * 4;
     sz.list[0] = nent[0] * 4;
+    sz.filt[0] = nent[0] * 4;
     sz.sel[0] = 0;
     sz.mask1 = (uint64_t)G * 64;
     sz.xr1 = 257 * 4;
@@ -895,6 +931,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     const uint64_t L = m ? read1(s, d_runscan.as<uint32_t>() + m - 1) : 0;
     nlists[d - 1] = L;
     HIP_TRY(eng->d_list[d - 1].reserve(m * 4 + 4));
+    HIP_TRY(eng->d_filt[d - 1].reserve(m * 4 + 4));
     HIP_TRY(eng->d_beg[d - 1].reserve((L + 1) * 4));
     HIP_TRY(eng->d_nrep[d - 1].reserve(L * 4 + 4));
     HIP_TRY(d_lgrp[d - 1].reserve(L * 4 + 4));
@@ -903,7 +940,8 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(hipMemsetAsync(eng->d_beg[d - 1].p, 0, 4, s));
     hipLaunchKernelGGL(k_lists, dim3(grid_for(m)), dim3(kThreads), 0, s, ent, m,
                        d_runscan.as<uint32_t>(), d_sb.as<uint32_t>(), d_tag.as<int32_t>(),
-                       eng->d_list[d - 1].as<int32_t>(), eng->d_beg[d - 1].as<uint32_t>(),
+                       d_nfilt.as<uint32_t>(), eng->d_list[d - 1].as<int32_t>(),
+                       eng->d_filt[d - 1].as<uint32_t>(), eng->d_beg[d - 1].as<uint32_t>(),
                        eng->d_nrep[d - 1].as<uint32_t>(), d_lgrp[d - 1].as<uint32_t>(),
                        d_lgram[d - 1].as<uint32_t>(), L);
     HIP_TRY(hipGetLastError());
@@ -928,6 +966,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     sz.beg[d - 1] = (L + 1) * 4;
     sz.nrep[d - 1] = L * 4;
     sz.list[d - 1] = m * 4;
+    sz.filt[d - 1] = m * 4;
     sz.sel[d - 1] = pairs * 8;
   }
   // levels above the depth: one list offset (0), as the host image has
@@ -966,17 +1005,18 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     const uint64_t L2 = nlists[1], L3 = nlists[2];
     HIP_TRY(eng->d_x2rep.reserve(2048 * 4));
     HIP_TRY(hipMemsetAsync(eng->d_x2rep.p, 0, 2048 * 4, s));
+    // d_big: a 3-gram has too many states; some depth-2 list reports
+    DevBuf d_k(slab), d_o(slab), d_start(slab), d_contrib(slab), d_xpos(slab), d_big(slab);
+    HIP_TRY(d_big.reserve(8));
+    HIP_TRY(hipMemsetAsync(d_big.p, 0, 8, s));
     hipLaunchKernelGGL(k_x2rep, dim3(grid_for(L2)), dim3(kThreads), 0, s,
                        d_lgram[1].as<uint32_t>(), eng->d_nrep[1].as<uint32_t>(), L2,
-                       eng->d_x2rep.as<uint32_t>());
-    DevBuf d_k(slab), d_o(slab), d_start(slab), d_contrib(slab), d_xpos(slab), d_big(slab);
+                       eng->d_x2rep.as<uint32_t>(), d_big.as<uint32_t>() + 1);
     HIP_TRY(d_k.reserve(L3 * 8 + 8));
     HIP_TRY(d_o.reserve(L3 * 8 + 8));
     HIP_TRY(d_start.reserve(L3 * 4 + 4));
     HIP_TRY(d_contrib.reserve(L3 * 8 + 8));
     HIP_TRY(d_xpos.reserve((L3 + 1) * 8));
-    HIP_TRY(d_big.reserve(4));
-    HIP_TRY(hipMemsetAsync(d_big.p, 0, 4, s));
     hipLaunchKernelGGL(k_sort_keys_of_lists, dim3(grid_for(L3)), dim3(kThreads), 0, s,
                        d_lgram[2].as<uint32_t>(), L3, d_k.as<uint64_t>());
     HIP_TRY(prim.sort(d_k.as<uint64_t>(), d_o.as<uint64_t>(), L3, 56));
@@ -992,22 +1032,30 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(eng->d_xs3.reserve((2ull << 24) * 4));
     HIP_TRY(hipMemsetAsync(eng->d_xs3.p, 0, (2ull << 24) * 4, s));
     HIP_TRY(eng->d_xp3.reserve(P3 * 8 + 8));
+    HIP_TRY(eng->d_xf3.reserve(P3 * 4 + 4));
+    HIP_TRY(eng->d_xb3.reserve((1ull << 19) * 4));
+    HIP_TRY(hipMemsetAsync(eng->d_xb3.p, 0, (1ull << 19) * 4, s));
     hipLaunchKernelGGL(k_x3_fill, dim3(grid_for(L3)), dim3(kThreads), 0, s, d_o.as<uint64_t>(),
                        L3, eng->d_beg[2].as<uint32_t>(), eng->d_list[2].as<int32_t>(),
-                       d_lgrp[2].as<uint32_t>(), d_xpos.as<uint64_t>(),
-                       eng->d_xs3.as<uint32_t>(), eng->d_xp3.as<uint32_t>(),
-                       d_big.as<uint32_t>());
+                       eng->d_filt[2].as<uint32_t>(), d_lgrp[2].as<uint32_t>(),
+                       d_xpos.as<uint64_t>(), eng->d_xs3.as<uint32_t>(),
+                       eng->d_xp3.as<uint32_t>(), eng->d_xf3.as<uint32_t>(),
+                       eng->d_xb3.as<uint32_t>(), d_big.as<uint32_t>());
     hipLaunchKernelGGL(k_x3_flags, dim3(grid_for(1ull << 24)), dim3(kThreads), 0, s,
                        eng->d_xmask1.as<uint32_t>(), eng->d_x2rep.as<uint32_t>(),
                        eng->d_xs3.as<uint32_t>());
     HIP_TRY(hipGetLastError());
-    if (read1(s, d_big.as<uint32_t>())) {
+    const uint2 big = read1(s, d_big.as<uint2>());
+    if (big.y) img.short_reports = true;
+    if (big.x) {
       err = "a 3-gram has 2^30 depth-3 states or more; use a smaller precompute depth";
       return NGAP_ERR_INVALID;
     }
     sz.x2rep = 2048 * 4;
     sz.xs3 = (2ull << 24) * 4;
     sz.xp3 = P3 * 8;
+    sz.xf3 = P3 * 4;
+    sz.xb3 = (1ull << 19) * 4;
   }
   HIP_TRY(hipStreamSynchronize(s));
   return NGAP_OK;

@@ -21,10 +21,11 @@ struct DevImage {
   const uint32_t *beg[kMaxMemoDepth];
   const uint32_t *nrep[kMaxMemoDepth];
   const int32_t *list[kMaxMemoDepth];
+  const uint32_t *filt[kMaxMemoDepth];  // next-byte filter of each list entry
   const uint32_t *sel[kMaxMemoDepth];  // rank tables of depths 2 and 3
   const uint32_t *mask1;     // 16 words per group (layout.h)
   // cross-group root index (layout.h)
-  const uint32_t *xr1, *xe1, *xmask1, *xr2, *xe2, *xsod, *xs3, *xp3, *x2rep;
+  const uint32_t *xr1, *xe1, *xmask1, *xr2, *xe2, *xsod, *xs3, *xp3, *xf3, *xb3, *x2rep;
   uint32_t n_xsod;
 };
 
@@ -54,7 +55,9 @@ struct KParams {
   DevImage img;
   const uint8_t *input;
   uint32_t chunk_len, num_seg, num_groups;
-  uint64_t chunk_magic;    // ceil(2^64 / chunk_len): divisibility test (chunk_len > 0)
+  // divisibility by chunk_len (> 0): its odd part's inverse modulo 2^32, its
+  // power of two, and floor((2^32 - 1) / chunk_len)
+  uint32_t div_inverse, div_shift, div_most;
   // Request runs (chunk_len 0): bit p set when position p is the last of its
   // request, so an item of any request finds its chunk end (nullable: then a
   // wave's current work item gives it)
@@ -67,8 +70,6 @@ struct KParams {
                              // this are busy (--active-threshold)
   int32_t report_off;
   uint32_t ring_cap;       // LDS ring entries per wave (power of two)
-  uint32_t rbuf_cap;       // LDS report buffer entries per wave
-  uint32_t dc_cap;         // LDS dedup cache entries per wave (power of two)
   uint32_t root_batch;     // positions whose roots one step takes (per-group
                            // roots; 1 = NAPgroups' one position at a time)
   unsigned long long *report_count;
@@ -91,6 +92,10 @@ struct KParams {
   uint32_t *task_head;     // kQueues claim counters, kQueueStride words apart
   unsigned long long *task_items;  // nullable, per task
   uint32_t waves_per_block;
+  // k_scan: every work item is an all-group one (scan), and the last input
+  // position an 8-byte load may start at
+  int32_t scan;
+  uint32_t load_last;
   // Root pass (nullable root_items = off): k_roots writes the root items of
   // work item t to root_items[root_off[t] .. root_off[t + 1]), counting them
   // in root_count[t]; the streaming kernel then expands them instead of
@@ -102,8 +107,20 @@ struct KParams {
   unsigned long long *root_count;
 };
 
+inline void set_chunk_len(KParams &P, uint32_t len) {
+  P.chunk_len = len;
+  P.div_shift = (uint32_t)__builtin_ctz(len);
+  const uint32_t odd = len >> P.div_shift;
+  uint32_t x = odd;  // Newton: correct to 3 bits, doubled each time
+  for (int i = 0; i < 4; i++) x *= 2 - odd * x;
+  P.div_inverse = x;
+  P.div_most = 0xFFFFFFFFu / len;
+}
+
 constexpr uint32_t kWave = 64;
 constexpr uint32_t kMaxOpen = 8;  // work items a wave overlaps (k_batched)
+// LDS entries per wave: report buffer, de-duplication cache (power of two)
+constexpr uint32_t kRbuf = 128, kDc = 256;
 // The work queue is split by XCD: workgroup b runs on XCD b % 8, and queue q
 // holds work items q, q + 8, q + 16, ...; each claim counter has its own
 // 128-byte line.  A wave whose queue is empty takes from the next ones.
@@ -149,18 +166,31 @@ NGAP_HD inline Task gen_task(const KParams &P, uint32_t t) {
 // wave: per-work-item traces, or request runs without a last-byte map), 1
 // k_batched_stream of engine runs, 2 k_expand (after the root pass), 3
 // k_batched_stream of request runs (last-byte map), 4 k_batched_stream of
+// generated work items, 5 and 6 k_scan (KParams::scan) of engine runs and of
 // generated work items.
-constexpr int kBatchedKinds = 5;
+constexpr int kBatchedKinds = 7;
 NGAP_HD inline int batched_kind(const KParams &P) {
   if (P.task_items || (!P.chunk_len && !P.last_map)) return 0;
   if (P.root_items) return 2;
   if (!P.chunk_len) return 3;
+  if (P.scan) return P.tasks ? 5 : 6;
   return P.tasks ? 1 : 4;
 }
 
-// LDS bytes per wave for the given capacities
-NGAP_HD inline uint32_t wave_lds_bytes(uint32_t ring, uint32_t rbuf, uint32_t dc) {
-  return ring * 8 + rbuf * 8 + dc * 8 + (65 + 64 + 64 + 64 + 16 + kMaxOpen) * 4 + 4;
-}
+// LDS bytes per wave: what has a fixed size first (so that it lies at constant
+// offsets from one base), then the ring.  Report buffer and de-duplication
+// cache, then: list positions in work (65 + 3 x 64 words), the root masks and
+// the open work items;
+constexpr uint32_t kWaveFixed = (kRbuf + kDc) * 8 + (65 + 3 * kWave + 16 + kMaxOpen + 1) / 2 * 8;
+NGAP_HD inline uint32_t wave_lds_bytes(uint32_t ring) { return kWaveFixed + ring * 8; }
+
+// in k_scan: 64 marks, the waiting 3-grams (a wave's width less one and a search
+// of 128 positions more) and the open work items;
+// the groups' bases lie before all waves.  With 1,024 groups four workgroups
+// fit a CU's 160 KiB.
+constexpr uint32_t kKeyCap = 3 * kWave;
+constexpr uint32_t kScanFixed = (kRbuf + kDc) * 8 + kWave * 4 + kKeyCap * 8 + kMaxOpen * 4;
+NGAP_HD inline uint32_t scan_table_bytes(uint32_t groups) { return (groups * 8 + 15) / 16 * 16; }
+NGAP_HD inline uint32_t scan_wave_bytes(uint32_t ring) { return kScanFixed + ring * 8; }
 
 }  // namespace ngapamd

@@ -46,6 +46,11 @@
 namespace ngapamd {
 
 #define NGAP_DEV __device__ __forceinline__
+// Branch weights: what a wave seldom does goes out of line.  A taken branch
+// costs a lone wave as much as a dozen instructions (the fetch starts over), so
+// the common path falls through.
+#define NGAP_SELDOM(x) __builtin_expect((x) != 0, 0)
+#define NGAP_MOSTLY(x) __builtin_expect((x) != 0, 1)
 
 NGAP_DEV uint32_t lane_id() {
   return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -54,7 +59,17 @@ NGAP_DEV uint32_t mask_rank(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
-NGAP_DEV uint64_t wballot(bool p) { return __ballot(p); }
+NGAP_DEV uint64_t wballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+// A value that every lane is to have from one lane, read into a scalar
+// register.  What steers the wave (claims, queue ends, counts) must come this
+// way and not from a shuffle: a shuffled value is a vector to the compiler, the
+// branches on it are divergent, and every counter that a loop carries through
+// them moves to vector registers and vector instructions.
+NGAP_DEV uint32_t from_first(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+NGAP_DEV uint64_t from_first(uint64_t x) {
+  return (uint64_t)from_first((uint32_t)x) | ((uint64_t)from_first((uint32_t)(x >> 32)) << 32);
+}
+NGAP_DEV uint32_t from_last(uint32_t x) { return __builtin_amdgcn_readlane(x, 63); }
 NGAP_DEV void wsync() { __builtin_amdgcn_wave_barrier(); }
 
 NGAP_DEV uint32_t wave_incl_scan(uint32_t x, uint32_t lane) {
@@ -66,8 +81,34 @@ NGAP_DEV uint32_t wave_incl_scan(uint32_t x, uint32_t lane) {
   return x;
 }
 
+// Inclusive scans over the wave on the DPP network: shifts inside rows of 16
+// lanes, then the last lane of a row broadcast to the rows after it.
+template <int Ctrl, int Rows>
+NGAP_DEV uint32_t dpp(uint32_t x) {  // 0 where the source lane does not exist
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, Ctrl, Rows, 0xF, false);
+}
+template <class Op>
+NGAP_DEV uint32_t dpp_scan(uint32_t x, Op op) {  // op(x, 0) = x
+  x = op(x, dpp<0x111, 0xF>(x));
+  x = op(x, dpp<0x112, 0xF>(x));
+  x = op(x, dpp<0x114, 0xF>(x));
+  x = op(x, dpp<0x118, 0xF>(x));
+  x = op(x, dpp<0x142, 0xA>(x));
+  return op(x, dpp<0x143, 0xC>(x));
+}
+
+// The kernel's parameters read again from memory, for the paths that a wave
+// seldom takes: what only they need does not occupy scalar registers in
+// between.  (Every kernel's only argument is KParams.)
+NGAP_DEV const KParams &cold_params() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const KParams *)p;
+}
+
 // A wave's expanded items, added at its workgroup's lane of the count.
-NGAP_DEV void add_items(const KParams &P, unsigned long long n) {
+NGAP_DEV void add_items(unsigned long long n) {
+  const KParams &P = cold_params();
   atomicAdd(P.items + (blockIdx.x % kItemLanes) * kItemStride, n);
 }
 
@@ -82,9 +123,8 @@ struct WaveState {
   uint32_t *mask1;    // 16: root bytes, then reporting depth-1 bytes (layout.h)
   uint32_t *open;     // kMaxOpen: work items whose items may still be queued
   uint32_t n_open;
-  uint64_t *spill;
   uint32_t head, tail, rn, spill_n;
-  uint32_t lane;
+  uint32_t lane, wave;
   bool overflow;
   unsigned long long items;
   // root pass: the work item's area of root_items and its item count
@@ -147,14 +187,21 @@ NGAP_DEV bool test_hit(bool live, int32_t e, uint32_t t, uint32_t word, uint32_t
 NGAP_DEV void flush_stage(const KParams &P, WaveState &W) {
   if (W.tail == 0) return;
   wsync();
-  unsigned long long base = 0;
+  uint64_t base = 0;
   if (W.lane == 0) base = atomicAdd(W.out_count, (unsigned long long)W.tail);
-  base = __shfl(base, 0, 64);
+  base = from_first(base);
   for (uint32_t i = W.lane; i < W.tail; i += kWave)
     if (base + i < W.out_cap) W.out[base + i] = W.ring[i];
   if (base + W.tail > W.out_cap) W.overflow = true;
   W.tail = 0;
   wsync();
+}
+
+// The wave's spill area and its capacity.
+NGAP_DEV uint64_t *spill_area(const WaveState &W, uint32_t &cap) {
+  const KParams &P = cold_params();
+  cap = P.spill_cap;
+  return P.spill + ((size_t)blockIdx.x * P.waves_per_block + W.wave) * cap;
 }
 
 template <bool Stage = false>
@@ -170,27 +217,36 @@ NGAP_DEV void push(const KParams &P, WaveState &W, bool pred, uint64_t item) {
     wsync();
     return;
   }
-  if (W.tail - W.head + cnt <= P.ring_cap) {
+  // the barriers inside the branches keep the compiler from folding a lane's
+  // condition into the wave's, which would make the counters vectors
+  if (NGAP_MOSTLY(W.tail - W.head + cnt <= P.ring_cap)) {
     if (pred) W.ring[(W.tail + r) & (P.ring_cap - 1)] = item;
+    wsync();
     W.tail += cnt;
-  } else if (W.spill_n + cnt <= P.spill_cap) {
-    if (pred) W.spill[W.spill_n + r] = item;
-    W.spill_n += cnt;
   } else {
-    W.overflow = true;
+    uint32_t cap;
+    uint64_t *spill = spill_area(W, cap);
+    if (W.spill_n + cnt <= cap) {
+      if (pred) spill[W.spill_n + r] = item;
+      wsync();
+      W.spill_n += cnt;
+    } else {
+      W.overflow = true;
+    }
   }
   wsync();
 }
 
-NGAP_DEV void flush_reports(const KParams &P, WaveState &W) {
+NGAP_DEV void flush_reports(WaveState &W) {
   if (W.rn == 0) return;
+  const KParams &P = cold_params();
   wsync();
-  unsigned long long base = 0;
+  uint64_t base = 0;
   if (W.lane == 0) base = atomicAdd(P.report_count, (unsigned long long)W.rn);
-  base = __shfl(base, 0, 64);
+  base = from_first(base);
   if (!P.report_off) {
     for (uint32_t i = W.lane; i < W.rn; i += kWave) {
-      unsigned long long idx = base + i;
+      const uint64_t idx = base + i;
       if (idx < P.report_cap) P.reports[idx] = W.rbuf[i];
     }
   }
@@ -204,14 +260,27 @@ NGAP_DEV void emit(const KParams &P, WaveState &W, bool pred, uint64_t val) {
   uint64_t m = wballot(pred);
   if (m == 0) return;
   uint32_t cnt = __popcll(m);
-  if (W.rn + cnt > P.rbuf_cap) flush_reports(P, W);
+  if (NGAP_SELDOM(W.rn + cnt > kRbuf)) flush_reports(W);
   if (pred) W.rbuf[W.rn + mask_rank(m)] = val;
   W.rn += cnt;
   wsync();
 }
 
+// Queues an item unless its next byte shows that it expands to nothing (its
+// state's next-byte filter, layout.h); such an item is counted as expanded,
+// which is all that expanding it would have done.
+template <bool Stage = false>
+NGAP_DEV void push_filtered(const KParams &P, WaveState &W, bool keep, uint32_t filt,
+                            uint32_t next, uint64_t item) {
+  const bool pass = keep & (((filt >> filter_bit(next)) & 1u) != 0);
+  W.items += __popcll(wballot(keep & !pass));
+  push<Stage>(P, W, pass, item);
+}
+
+NGAP_DEV uint32_t min_u(uint32_t a, uint32_t b) { return a < b ? a : b; }
+
 NGAP_DEV bool dedup_fresh(const KParams &P, WaveState &W, uint64_t key) {
-  uint32_t h = (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> 40) & (P.dc_cap - 1);
+  uint32_t h = (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> 40) & (kDc - 1);
   unsigned long long old = atomicExch((unsigned long long *)&W.dc[h], (unsigned long long)key);
   return old != key;
 }
@@ -220,9 +289,10 @@ NGAP_DEV bool dedup_fresh(const KParams &P, WaveState &W, uint64_t key) {
 NGAP_DEV void refill_from_spill(const KParams &P, WaveState &W) {
   uint32_t room = P.ring_cap - (W.tail - W.head);
   uint32_t k = W.spill_n < room ? W.spill_n : room;
-  uint32_t from = W.spill_n - k;
+  uint32_t from = W.spill_n - k, cap;
+  const uint64_t *spill = spill_area(W, cap);
   for (uint32_t i = W.lane; i < k; i += kWave)
-    W.ring[(W.tail + i) & (P.ring_cap - 1)] = W.spill[from + i];
+    W.ring[(W.tail + i) & (P.ring_cap - 1)] = spill[from + i];
   W.tail += k;
   W.spill_n = from;
   wsync();
@@ -235,21 +305,25 @@ NGAP_DEV void refill_from_spill(const KParams &P, WaveState &W) {
 // position is the chunk's last.
 template <bool Stage = false>
 NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg,
-                      uint32_t pos, uint32_t gtag, const int32_t *list) {
+                      uint32_t pos, uint32_t gtag, const int32_t *list,
+                      const uint32_t *filt) {
+  const uint32_t last = W.cend - 1;
   if (wballot(cnt > 1u) == 0) {
     // at most one entry per lane (the common case): no prefix sum
     const bool ok = cnt == 1u;
     if (wballot(ok) == 0) return;
     const int32_t e = ok ? list[beg & 0x7fffffffu] : 0;
+    const uint32_t f = ok ? filt[beg & 0x7fffffffu] : 0;
+    const uint32_t next = P.input[ok ? min_u(pos + 1, last) : last];
     const uint64_t it = item_of(((uint32_t)e & (uint32_t)kIdMask) | gtag, pos);
     emit(P, W, ok && (e & kFlagReport), it);
     bool keep = ok && !(beg >> 31) && !(e & kFlagDeadEnd) && (pos + 1 < W.cend);
     if (keep && P.dedup && (e & kFlagDedup)) keep = dedup_fresh(P, W, it);
-    push<Stage>(P, W, keep, it);
+    push_filtered<Stage>(P, W, keep, f, next, it);
     return;
   }
   uint32_t incl = wave_incl_scan(cnt, W.lane);
-  uint32_t total = __shfl(incl, 63, 64);
+  uint32_t total = from_last(incl);
   if (total == 0) return;
   W.sh_pref[W.lane] = incl - cnt;
   W.sh_beg[W.lane] = beg;
@@ -261,7 +335,7 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
     uint32_t j = base + W.lane;
     bool ok = j < total;
     int32_t e = 0;
-    uint32_t ppos = 0, tg = 0;
+    uint32_t ppos = 0, tg = 0, f = 0, next = 0;
     bool ronly = true;
     if (ok) {
       int lo = 0, hi = 64;  // largest o with pref[o] <= j (pref[64] = total > j)
@@ -272,15 +346,18 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
       }
       const uint32_t bg = W.sh_beg[lo];
       ronly = bg >> 31;
-      e = list[(bg & 0x7fffffffu) + (j - W.sh_pref[lo])];
+      const uint32_t at = (bg & 0x7fffffffu) + (j - W.sh_pref[lo]);
+      e = list[at];
+      f = filt[at];
       ppos = W.sh_pos[lo];
+      next = P.input[min_u(ppos + 1, last)];
       tg = W.sh_tag[lo];
     }
     const uint32_t u = ((uint32_t)e & (uint32_t)kIdMask) | tg;
     emit(P, W, ok && (e & kFlagReport), item_of(u, ppos));
     bool keep = ok && !ronly && !(e & kFlagDeadEnd) && (ppos + 1 < W.cend);
     if (keep && P.dedup && (e & kFlagDedup)) keep = dedup_fresh(P, W, item_of(u, ppos));
-    push<Stage>(P, W, keep, item_of(u, ppos));
+    push_filtered<Stage>(P, W, keep, f, next, item_of(u, ppos));
   }
   wsync();
 }
@@ -304,8 +381,6 @@ NGAP_DEV int32_t memo_rank(const uint32_t *sel, size_t at, uint32_t bit) {
 // valid address when a lane does not need the value (index 0, or the chunk's
 // last byte), and the value is selected afterwards: the loads of a step then
 // go out together instead of one branch (and one wait) at a time.
-NGAP_DEV uint32_t min_u(uint32_t a, uint32_t b) { return a < b ? a : b; }
-
 template <bool Stage = false>
 NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) {
   const uint8_t *in = P.input;
@@ -323,7 +398,7 @@ NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) 
   if (P.memo_depth < 2) {  // depth 1: all-input states matching b0 become items
     const uint32_t li = W.g * 256u + b0;
     const uint32_t beg = P.img.beg[0][li], end = P.img.beg[0][li + 1];
-    flatten<Stage>(P, W, has ? end - beg : 0u, beg, p, W.gtag, P.img.list[0]);
+    flatten<Stage>(P, W, has ? end - beg : 0u, beg, p, W.gtag, P.img.list[0], P.img.filt[0]);
     return;
   }
   // rank pair of the 2-gram (and the depth-1 reports of rare bytes)
@@ -341,7 +416,7 @@ NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) 
       beg = P.img.beg[0][li] | kReportOnly;
       cnt = P.img.nrep[0][li];
     }
-    flatten<Stage>(P, W, cnt, beg, p, W.gtag, P.img.list[0]);
+    flatten<Stage>(P, W, cnt, beg, p, W.gtag, P.img.list[0], P.img.filt[0]);
   }
   const bool has2 = li2 >= 0;
   if (wballot(has2) == 0) return;
@@ -367,8 +442,9 @@ NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) 
     beg3 = b3;
     cnt3 = li3 >= 0 ? e3 - b3 : 0u;
   }
-  flatten<Stage>(P, W, cnt2, beg2, p + 1, W.gtag, P.img.list[1]);
-  if (wballot(cnt3 != 0)) flatten<Stage>(P, W, cnt3, beg3, p + 2, W.gtag, P.img.list[2]);
+  flatten<Stage>(P, W, cnt2, beg2, p + 1, W.gtag, P.img.list[1], P.img.filt[1]);
+  if (wballot(cnt3 != 0)) 
+    flatten<Stage>(P, W, cnt3, beg3, p + 2, W.gtag, P.img.list[2], P.img.filt[2]);
 }
 
 // Distributes per-lane index ranges [e0, e0 + ecnt) over the wave, 64
@@ -382,7 +458,7 @@ NGAP_DEV void for_entries(const WaveState &W, uint32_t e0, uint32_t ecnt, F &&f)
     return;
   }
   const uint32_t incl = wave_incl_scan(ecnt, W.lane);
-  const uint32_t total = __shfl(incl, 63, 64);
+  const uint32_t total = from_last(incl);
   for (uint32_t base = 0; base < total; base += kWave) {
     const uint32_t j = base + W.lane;
     const bool ok = j < total;
@@ -408,7 +484,7 @@ NGAP_DEV void for_entries2(const WaveState &W, uint32_t a0, uint32_t ac, uint32_
                            uint32_t bc, F &&f) {
   const uint32_t n = ac + bc;
   const uint32_t incl = wave_incl_scan(n, W.lane);
-  const uint32_t total = __shfl(incl, 63, 64);
+  const uint32_t total = from_last(incl);
   for (uint32_t base = 0; base < total; base += kWave) {
     const uint32_t j = base + W.lane;
     const bool ok = j < total;
@@ -431,7 +507,7 @@ NGAP_DEV void for_entries2(const WaveState &W, uint32_t a0, uint32_t ac, uint32_
 
 // Per-lane state of one position in roots_cross.
 struct CrossLane {
-  uint32_t p, k, b0, e0, ec, t0, tc, r0, rc;
+  uint32_t p, k, b0, b3, e0, ec, t0, tc, r0, rc;
 };
 
 // The loads of one position's lookups, in stages shared by both halves of a
@@ -452,6 +528,7 @@ NGAP_DEV void cross_lookup(const KParams &P, const WaveState &W, uint32_t p0, ui
     L[h].b0 = in[pc];
     b1[h] = in[min_u(pc + 1, last)];
     b2[h] = in[min_u(pc + 2, last)];
+    L[h].b3 = in[min_u(pc + 3, last)];
   }
   // Depth 3: the 3-gram slots first.  A slot flags the 3-grams whose first
   // byte or first two bytes begin reporting lists of depth 1 or 2 in some
@@ -498,13 +575,13 @@ NGAP_DEV void cross_lookup(const KParams &P, const WaveState &W, uint32_t p0, ui
 // One entry per lane at most: the entry and its single list item are loaded
 // for both halves before either is emitted.
 template <bool Stage = false>
-NGAP_DEV void emit_one(const KParams &P, WaveState &W, bool ok, int32_t e, bool ronly,
-                       uint32_t pos, uint32_t tag) {
+NGAP_DEV void emit_one(const KParams &P, WaveState &W, bool ok, int32_t e, uint32_t filt,
+                       uint32_t next, uint32_t pos, uint32_t tag) {
   const uint64_t it = item_of(((uint32_t)e & (uint32_t)kIdMask) | tag, pos);
   emit(P, W, ok && (e & kFlagReport), it);
-  bool keep = ok && !ronly && !(e & kFlagDeadEnd) && (pos + 1 < W.cend);
+  bool keep = ok && !(e & kFlagDeadEnd) && (pos + 1 < W.cend);
   if (keep && P.dedup && (e & kFlagDedup)) keep = dedup_fresh(P, W, it);
-  push<Stage>(P, W, keep, it);
+  push_filtered<Stage>(P, W, keep, filt, next, it);
 }
 
 // Roots of every group for positions [p0, pend), pend - p0 <= 128 (cross-
@@ -531,7 +608,7 @@ NGAP_DEV void roots_cross(const KParams &P, WaveState &W, uint32_t p0, uint32_t 
           cnt = P.img.nrep[0][li];
           tag = (li >> 8) << 22;
         }
-        flatten<Stage>(P, W, cnt, beg, pos, tag, P.img.list[0]);
+        flatten<Stage>(P, W, cnt, beg, pos, tag, P.img.list[0], P.img.filt[0]);
       });
     }
     // depth 2: full lists where it is the deepest level, reports otherwise
@@ -549,7 +626,7 @@ NGAP_DEV void roots_cross(const KParams &P, WaveState &W, uint32_t p0, uint32_t 
           cnt = ko == 2 || P.memo_depth == 2 ? e.z - e.y : (e.w & (uint32_t)kIdMask);
           if (!(ko == 2 || P.memo_depth == 2)) beg |= kReportOnly;
         }
-        flatten<Stage>(P, W, cnt, beg, pos + 1, tag, P.img.list[1]);
+        flatten<Stage>(P, W, cnt, beg, pos + 1, tag, P.img.list[1], P.img.filt[1]);
       });
     }
   }
@@ -560,15 +637,19 @@ NGAP_DEV void roots_cross(const KParams &P, WaveState &W, uint32_t p0, uint32_t 
 #pragma unroll
   for (int h = 0; h < 2; h++) {
     const bool inl = (L[h].tc & kSlotInline) != 0;
-    emit_one<Stage>(P, W, inl, (int32_t)L[h].t0, false, L[h].p + 2, (L[h].tc & 1023u) << 22);
+    emit_one<Stage>(P, W, inl, (int32_t)L[h].t0, slot_filter(L[h].t0, L[h].tc), L[h].b3,
+                    L[h].p + 2, (L[h].tc & 1023u) << 22);
     if (inl) L[h].tc = 0;
   }
   if (wballot(L[0].tc != 0 || L[1].tc != 0) == 0) return;
   // some lane has pairs, so pair 0 is a valid stand-in address
+  const uint32_t b3 = L[0].b3 | (L[1].b3 << 8);
   for_entries2(W, L[0].t0, L[0].tc, L[1].t0, L[1].tc,
                [&](bool ok, uint32_t idx, uint32_t o, uint32_t h) {
                  const uint2 e = reinterpret_cast<const uint2 *>(P.img.xp3)[ok ? idx : 0u];
-                 emit_one<Stage>(P, W, ok, (int32_t)e.x, false, p0 + h * kWave + o + 2,
+                 const uint32_t f = P.img.xf3[ok ? idx : 0u];
+                 const uint32_t next = (__shfl(b3, (int)o, 64) >> (8 * h)) & 255u;
+                 emit_one<Stage>(P, W, ok, (int32_t)e.x, f, next, p0 + h * kWave + o + 2,
                                  e.y << 22);
                });
 }
@@ -628,6 +709,11 @@ struct LaneGroup {
 // time (chunk_len, else the wave's one open work item's bounds).
 enum : int { kEndChunkLen = 0, kEndMap = 1, kEndRuntime = 2 };
 
+// The step is written for few instructions, which bound it as much as its two
+// dependent gathers do (with four waves a SIMD, vector instructions took two
+// thirds of the SIMDs' cycles): hits are lane masks first, and reports, the
+// de-duplication cache and successors beyond a lane's first are looked at only
+// when some lane has one.
 template <int End = kEndRuntime>
 NGAP_DEV void expand(const KParams &P, WaveState &W, bool &valid, uint32_t &v,
                      uint32_t &p, int &depth, const LaneGroup &lg) {
@@ -636,7 +722,6 @@ NGAP_DEV void expand(const KParams &P, WaveState &W, bool &valid, uint32_t &v,
   // so the image has a record)
   const uint32_t b = P.input[valid ? p1 : 0u];
   Rec rec = load_rec(P, valid ? lg.rec_base + v : 0u);
-  if (!valid) rec = empty_rec();
   const uint32_t busy = __popcll(wballot(valid));
   W.items += busy;
   // is p1 the last position of its chunk (no successors enabled after it)?
@@ -645,68 +730,89 @@ NGAP_DEV void expand(const KParams &P, WaveState &W, bool &valid, uint32_t &v,
     const uint32_t lw = P.last_map[valid ? p1 >> 5 : 0u];
     last = ((lw >> (p1 & 31)) & 1u) != 0u;
   } else if (End == kEndChunkLen || P.chunk_len) {
-    last = (uint64_t)(p1 + 1) * P.chunk_magic <= P.chunk_magic - 1;
+    // divisible by chunk_len = odd << div_shift: n * (odd's inverse), rotated,
+    // stays small exactly for the multiples (Granlund and Montgomery)
+    const uint32_t n = (p1 + 1) * P.div_inverse;
+    last = __builtin_rotateright32(n, P.div_shift) <= P.div_most;
   } else {
     last = p1 + 1 >= W.cend;
   }
-  bool has_next = false;
-  uint32_t nv = 0;
   // work privatization (kernel_ngap_O4.cu:115-122): a matched successor is
   // expanded by the same lane while more than active_threshold lanes are
   // busy, and otherwise queued for the idle lanes
-  const bool can_priv = (P.priv_limit < 0 || depth < P.priv_limit) &&
-                        (int32_t)busy > P.active_threshold;
+  const bool can_priv = ((P.priv_limit < 0) | (depth < P.priv_limit)) &
+                        ((int32_t)busy > P.active_threshold);
+  bool has_next = false;
+  uint32_t nv = 0;
   bool more = valid;
-  while (wballot(more)) {
-    int32_t link = -1;
+  for (;;) {
     const int32_t es[4] = {rec.ids.x, rec.ids.y, rec.ids.z, rec.ids.w};
     const uint32_t ts[4] = {rec.tests.x, rec.tests.y, rec.tests.z, rec.tests.w};
-    // all loads of this record first: the class words its tests need and the
-    // continuation record, then the wave-wide emits and pushes
-    uint32_t cw[4];
+    // class words of the successors that are not decided by their test word;
+    // successors fill the slots from 0, so the later slots are often empty in
+    // every lane
+    bool need[4], hit[4], keep[4];
+    uint32_t cw[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int s = 0; s < 4; s++) {
-      if (more && es[s] <= -2) link = -(es[s] + 2);
-      const bool need = more && es[s] >= 0 && !(ts[s] & (kTestLiteral | kTestAll));
-      const size_t at =
-          need ? (size_t)(lg.cls_base + ((uint32_t)es[s] & (uint32_t)kIdMask)) * 8 + (b >> 5) : 0;
-      cw[s] = P.img.cls[at];
-    }
-    Rec next = load_rec(P, more && link >= 0 ? (uint32_t)link : 0u);
-    if (!(more && link >= 0)) next = empty_rec();
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      const int32_t e = es[s];
-      // successors fill the slots from 0 (a continuation link needs slots
-      // 0-2 full): once no lane has one in this slot, none has one later
-      if (s < 3 && wballot(more && e >= 0) == 0) break;
-      const uint32_t u = (uint32_t)e & (uint32_t)kIdMask;
-      const bool hit = test_hit(more, e, ts[s], cw[s], b);
-      const uint64_t it = item_of(u | lg.gtag, p1);
-      emit(P, W, hit && (e & kFlagReport), it);
-      bool keep = hit && !(e & kFlagDeadEnd) && !last;
-      if (keep && P.dedup && (e & kFlagDedup)) keep = dedup_fresh(P, W, it);
-      const bool take = keep && !has_next && can_priv;
-      if (take) {
-        has_next = true;
-        nv = u;
+      need[s] = more & (es[s] >= 0) & (ts[s] == 0u);
+      if (wballot(need[s])) {
+        const uint32_t u = (uint32_t)es[s] & (uint32_t)kIdMask;
+        cw[s] = P.img.cls[need[s] ? (size_t)(lg.cls_base + u) * 8 + (b >> 5) : 0];
       }
-      push(P, W, keep && !take, it);
     }
-    more = more && link >= 0;
-    rec = next;
+    bool rep = false, dup = false;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const bool in_class = ((cw[s] >> (b & 31)) & 1u) != 0;
+      hit[s] = more & ((ts[s] == (b | kTestLiteral)) | (ts[s] == kTestAll) | (need[s] & in_class));
+      rep |= hit[s] & ((es[s] & kFlagReport) != 0);
+      keep[s] = hit[s] & ((es[s] & kFlagDeadEnd) == 0) & !last;
+      dup |= keep[s] & ((es[s] & kFlagDedup) != 0);
+    }
+    if (wballot(rep)) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        emit(P, W, hit[s] & ((es[s] & kFlagReport) != 0),
+             item_of(((uint32_t)es[s] & (uint32_t)kIdMask) | lg.gtag, p1));
+    }
+    if (P.dedup && wballot(dup)) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        if (keep[s] & ((es[s] & kFlagDedup) != 0))
+          keep[s] = dedup_fresh(
+              P, W, item_of(((uint32_t)es[s] & (uint32_t)kIdMask) | lg.gtag, p1));
+    }
+    bool queue[4], any = false;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const bool take = keep[s] & !has_next & can_priv;
+      nv = take ? (uint32_t)es[s] & (uint32_t)kIdMask : nv;
+      has_next |= take;
+      queue[s] = keep[s] & !take;
+      any |= queue[s];
+    }
+    if (wballot(any)) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        push(P, W, queue[s], item_of(((uint32_t)es[s] & (uint32_t)kIdMask) | lg.gtag, p1));
+    }
+    // a continuation record (more than four successors)
+    const int32_t e3 = es[3];
+    more = more & (e3 <= -2);
+    if (wballot(more) == 0) break;
+    rec = load_rec(P, more ? (uint32_t)-(e3 + 2) : 0u);
   }
-  if (has_next) {
-    v = nv;
-    p = p1;
-    depth++;
-  } else {
-    valid = false;
-  }
+  // selects, not a branch: a divergent branch that joins at the caller's loop
+  // end would make every counter merged there a vector
+  v = has_next ? nv : v;
+  p = has_next ? p1 : p;
+  depth += has_next ? 1 : 0;
+  valid = has_next;
 }
 
 NGAP_DEV void clear_dedup(const KParams &P, WaveState &W) {
-  for (uint32_t i = W.lane; i < P.dc_cap; i += kWave) W.dc[i] = ~0ull;
+  for (uint32_t i = W.lane; i < kDc; i += kWave) W.dc[i] = ~0ull;
   wsync();
 }
 
@@ -745,19 +851,18 @@ NGAP_DEV void begin_cross(const KParams &P, WaveState &W, uint32_t cstart, uint3
   set_cross(P, W, cstart, cend);
 }
 
-NGAP_DEV void setup_wave(const KParams &P, WaveState &W, unsigned char *base,
-                         uint64_t *spill) {
-  W.ring = reinterpret_cast<uint64_t *>(base);
-  W.rbuf = W.ring + P.ring_cap;
-  W.dc = W.rbuf + P.rbuf_cap;
-  W.sh_pref = reinterpret_cast<uint32_t *>(W.dc + P.dc_cap);
+NGAP_DEV void setup_wave(WaveState &W, unsigned char *base, uint32_t wave) {
+  W.rbuf = reinterpret_cast<uint64_t *>(base);
+  W.dc = W.rbuf + kRbuf;
+  W.sh_pref = reinterpret_cast<uint32_t *>(W.dc + kDc);
   W.sh_beg = W.sh_pref + 65;
   W.sh_pos = W.sh_beg + 64;
   W.sh_tag = W.sh_pos + 64;
   W.mask1 = W.sh_tag + 64;
   W.open = W.mask1 + 16;
+  W.ring = reinterpret_cast<uint64_t *>(base + kWaveFixed);
+  W.wave = wave;
   W.n_open = 0;
-  W.spill = spill;
   W.out = nullptr;
   W.out_count = nullptr;
   W.out_cap = 0;
@@ -834,12 +939,12 @@ NGAP_DEV uint32_t claim_task(const KParams &P, const WaveState &W, uint32_t &q) 
   for (uint32_t tries = 0; tries < kQueues; tries++) {
     uint32_t j = 0;
     if (W.lane == 0) j = atomicAdd(P.task_head + q * kQueueStride, 1u);
-    j = __shfl(j, 0, 64);
+    j = from_first(j);
     const uint64_t t = (uint64_t)j * kQueues + q;
     if (t < P.num_tasks) return (uint32_t)t;
     uint32_t m = 0;
     if (W.lane == 0) m = atomicOr(empty, 1u << q);
-    known |= __shfl(m, 0, 64) | (1u << q);
+    known |= from_first(m) | (1u << q);
     if (known == (1u << kQueues) - 1) return P.num_tasks;
     uint32_t d = 1;
     while ((known >> ((q + d) % kQueues)) & 1u) d++;
@@ -915,10 +1020,11 @@ struct TaskStream {
 // All queued items are done: the open work items are complete, and each is
 // marked for the overflow fallback when the wave dropped an item since they
 // opened.
-NGAP_DEV void close_open(const KParams &P, WaveState &W) {
+NGAP_DEV void close_open(WaveState &W) {
   if (W.n_open == 0) return;
   wsync();
   if (W.overflow) {
+    const KParams &P = cold_params();
     if (W.lane < W.n_open) atomicOr(&P.overflow[W.open[W.lane]], kSpillOverflow);
     if (W.lane == 0) atomicAdd(P.overflow_count, W.n_open);
   }
@@ -984,13 +1090,360 @@ NGAP_DEV void drain_stream(const KParams &P, WaveState &W) {
     wsync();
     if (wballot(valid) == 0) {
       if (W.tail == W.head && W.spill_n == 0) {
-        close_open(P, W);
+        close_open(W);
         if (!more) break;
       }
       continue;
     }
     expand<End>(P, W, valid, v, p, depth, lg);
   }
+}
+
+// x of another lane.
+NGAP_DEV uint32_t from_lane(uint32_t x, uint32_t lane) {
+  return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(lane << 2), (int)x);
+}
+
+// A load at a 32-bit byte offset from a wave-uniform base.
+template <class T>
+NGAP_DEV T load_at(const void *base, uint32_t byte_offset) {
+  return *reinterpret_cast<const T *>(static_cast<const char *>(base) + byte_offset);
+}
+
+// ---- all-group scan at memo depth 3 (k_scan) ----
+// The engine's main path: every work item scans a window for all groups,
+// memo depth 3, and no list of depth 1 or 2 reports in any group (patterns of
+// three or more symbols), so a position's 3-gram slot holds all there is to do
+// there.  A kernel of its own: without the other levels' index arrays its
+// scalar state fits the scalar registers (the general kernel spills over a
+// hundred of them into vector lanes, and moving them back and forth is vector
+// work), and the roots need a third of the instructions.  Before it (one kernel
+// for all levels, a slot read and both tables for every position, successors
+// without filters) and now: 400,000 states over 16 MiB 0.213 and 0.152 ms,
+// 1,024 automata over 8 MiB 0.272 and 0.206, over 64 MiB 1.77 and 1.31, eight
+// automata of short words over 4 MiB of text 0.139 and 0.126.  What bounds it is
+// the latency of its gathers (slot, pairs, records: 4 MiB of L2 per XCD against
+// 128 MiB of slots) and, at the end of a run, of the last chains' steps.
+
+// A 3-gram that some group's depth-3 list has, waiting for its slot: the key
+// in bits 0-23, the filter bit of the byte after it in 24-28, bit 29 set when
+// the 3-gram ends its chunk, the position of its last byte in the upper word.
+constexpr uint32_t kKeyLast = 1u << 29;
+
+struct ScanLds {
+  uint32_t *mark;       // [kWave]
+  uint64_t *keys;       // [kKeyCap], `n_keys` of them waiting
+  const uint2 *bases;   // (record, class) bases of every group
+  uint32_t n_keys;
+};
+
+// The 3-grams at positions [a, b), b - a <= 128, that have a list in some
+// group, by the presence bitmap (2 MiB: it stays in L2, where the 128 MiB of
+// slots do not).  Two neighbouring positions a lane, from one 8-byte load of
+// the input (at most P.load_last, so that it stays inside the input).  The
+// slots are read by whole waves of present 3-grams (take_keys).  Against a slot
+// read at every position: 0.153 and 0.184 ms where the lists cover one 3-gram in
+// 28 (400,000 states, 16 MiB), 1.31 and 1.27 where they cover nearly half (1,024
+// automata, 64 MiB).
+NGAP_DEV void find_keys(const KParams &P, WaveState &W, ScanLds &S, uint32_t a, uint32_t b) {
+  const uint32_t p = a + 2 * W.lane;
+  // 3-grams end before the chunk does
+  const uint32_t lim = b + 2 <= W.cend ? b : W.cend - (W.cend < 2 ? W.cend : 2);
+  const uint32_t at = min_u(p, P.load_last);
+  uint64_t bytes;
+  __builtin_memcpy(&bytes, P.input + at, 8);
+  bytes >>= 8 * min_u(p - at, 7);
+  const uint32_t lo = (uint32_t)bytes, hi = (uint32_t)(bytes >> 32);
+  const uint32_t key[2] = {__builtin_amdgcn_perm(hi, lo, 0x0c000102u),
+                           __builtin_amdgcn_perm(hi, lo, 0x0c010203u)};
+  const uint32_t next[2] = {lo >> 24, hi & 255u};
+  uint32_t word[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) word[h] = load_at<uint32_t>(P.img.xb3, (key[h] >> 5) << 2);
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const bool has = (p + h < lim) & (((word[h] >> (key[h] & 31)) & 1u) != 0);
+    const uint64_t m = wballot(has);
+    const uint32_t low = key[h] | (filter_bit(next[h]) << 24) |
+                         (p + h + 3 >= W.cend ? kKeyLast : 0u);
+    if (has) S.keys[S.n_keys + mask_rank(m)] = ((uint64_t)(p + h + 2) << 32) | low;
+    wsync();
+    S.n_keys += __popcll(m);
+  }
+}
+
+// Roots from the slots of up to 64 waiting 3-grams, one a lane.
+NGAP_DEV void take_keys(const KParams &P, WaveState &W, ScanLds &S) {
+  const uint32_t count = min_u(S.n_keys, kWave);
+  S.n_keys -= count;
+  const bool have = W.lane < count;
+  const uint64_t entry = S.keys[S.n_keys + (have ? W.lane : 0u)];
+  const uint32_t key = (uint32_t)entry, pos = (uint32_t)(entry >> 32);
+  const uint2 slot = load_at<uint2>(P.img.xs3, (key & 0xFFFFFFu) << 3);
+  const uint32_t bit = (key >> 24) & 31;
+  // an inline state: the one entry, in the slot itself
+  const bool inl = have & ((int32_t)slot.y < 0);
+  {
+    bool keep = inl & ((slot.x & (uint32_t)kFlagDeadEnd) == 0) & ((key & kKeyLast) == 0);
+    const uint64_t it = item_of((slot.x & (uint32_t)kIdMask) | (slot.y << 22), pos);
+    if (NGAP_SELDOM(wballot(inl & ((slot.x & (uint32_t)(kFlagReport | kFlagDedup)) != 0)))) {
+      emit(P, W, inl & ((slot.x & (uint32_t)kFlagReport) != 0), it);
+      if (P.dedup && (keep & ((slot.x & (uint32_t)kFlagDedup) != 0)))
+        keep = dedup_fresh(P, W, it);
+      wsync();
+    }
+    const bool pass = keep & (((slot_filter(slot.x, slot.y) >> bit) & 1u) != 0);
+    W.items += __popcll(wballot(keep & !pass));
+    push(P, W, pass, it);
+  }
+  // the other slots' pairs, spread over the wave: owners mark where their
+  // entries start and a running maximum finds each entry's owner
+  const uint32_t cnt = (have & !inl) ? slot.y : 0u;
+  if (wballot(cnt != 0) == 0) return;
+  const uint32_t incl = dpp_scan(cnt, [](uint32_t x, uint32_t y) { return x + y; });
+  const uint32_t excl = incl - cnt, total = from_last(incl);
+  // entry j of the wave's flat index space is its owner's pair j + at
+  const uint32_t at = slot.x - excl;
+  uint32_t carry = 0;  // owner of the entries before this round's first mark, plus 1
+  for (uint32_t base = 0; base < total; base += kWave) {
+    S.mark[W.lane] = W.lane == 0 ? carry : 0u;
+    wsync();
+    if ((cnt != 0) & (excl - base < kWave)) S.mark[excl - base] = W.lane + 1;
+    wsync();
+    const uint32_t own =
+        dpp_scan(S.mark[W.lane], [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+    carry = from_last(own);
+    const uint32_t j = base + W.lane;
+    const bool ok = j < total;
+    const uint32_t wat = from_lane(at, own - 1), wkey = from_lane(key, own - 1),
+                   wpos = from_lane(pos, own - 1);
+    const uint32_t idx = ok ? j + wat : 0u;
+    const uint2 e = reinterpret_cast<const uint2 *>(P.img.xp3)[idx];
+    const uint32_t f = P.img.xf3[idx];
+    const uint64_t it = item_of((e.x & (uint32_t)kIdMask) | (e.y << 22), wpos);
+    bool k = ok & ((e.x & (uint32_t)kFlagDeadEnd) == 0) & ((wkey & kKeyLast) == 0);
+    if (NGAP_SELDOM(wballot(ok & ((e.x & (uint32_t)(kFlagReport | kFlagDedup)) != 0)))) {
+      emit(P, W, ok & ((e.x & (uint32_t)kFlagReport) != 0), it);
+      if (P.dedup && (k & ((e.x & (uint32_t)kFlagDedup) != 0))) k = dedup_fresh(P, W, it);
+      wsync();
+    }
+    const bool pass = k & (((f >> ((wkey >> 24) & 31)) & 1u) != 0);
+    W.items += __popcll(wballot(k & !pass));
+    push(P, W, pass, it);
+  }
+  wsync();
+}
+
+// The item a lane expands: its position (kNoItem: none), byte offsets of its
+// state's record and of its group's first record and class, its group's tag.
+struct ScanItem {
+  uint32_t pos, rec, rec_base, cls_base, gtag;
+};
+constexpr uint32_t kNoItem = ~0u;  // (+ 1 = 0: an idle lane's loads hit position and record 0)
+
+// expand() for k_scan: the same step with 32-bit byte offsets (the image's
+// records and classes are below 4 GiB each, scan_image).  A chain of steps is
+// bound by the instructions of each and above all by its branches: a step of
+// a lone chain over random states took 1,050 ns in the general kernel's first
+// form and takes 580 here, with 60,000 states in the cache.  So the common step
+// has few branches: one to skip the slots that no lane fills, one to skip everything that
+// most steps do not have (a report, a state with several predecessors, a second
+// matched successor, a continuation record).
+NGAP_DEV void expand_scan(const KParams &P, WaveState &W, ScanItem &I, int &depth) {
+  const bool valid = I.pos != kNoItem;
+  const uint32_t p1 = I.pos + 1;
+  const uint32_t b = load_at<uint8_t>(P.input, p1);
+  int4 ids = load_at<int4>(P.img.succ4, I.rec);
+  uint4 tests = load_at<uint4>(P.img.succ4, I.rec + 16);
+  const uint32_t busy = __popcll(wballot(valid));
+  W.items += busy;
+  const uint32_t n = (p1 + 1) * P.div_inverse;
+  const bool last = __builtin_rotateright32(n, P.div_shift) <= P.div_most;
+  const bool can_priv = ((P.priv_limit < 0) | (depth < P.priv_limit)) &
+                        ((int32_t)busy > P.active_threshold);
+  const uint32_t lit = b | kTestLiteral;
+  const uint32_t cls = I.cls_base + ((b >> 5) << 2);
+  bool has_next = false;
+  uint32_t nv = 0;
+  bool more = valid;
+  for (;;) {
+    const int32_t es[4] = {ids.x, ids.y, ids.z, ids.w};
+    const uint32_t ts[4] = {tests.x, tests.y, tests.z, tests.w};
+    bool need[4], hit[4] = {false, false, false, false}, keep[4];
+    uint32_t cw[4];
+    auto fetch = [&](int s) {
+      need[s] = more & (es[s] >= 0) & (ts[s] == 0u);
+      cw[s] = load_at<uint32_t>(
+          P.img.cls, need[s] ? cls + (((uint32_t)es[s] & (uint32_t)kIdMask) << 5) : 0u);
+    };
+    auto test = [&](int s) {
+      hit[s] = (more & ((ts[s] == lit) | (ts[s] == kTestAll))) |
+               (need[s] & (((cw[s] >> (b & 31)) & 1u) != 0));
+    };
+    // successors fill the slots from 0 (a continuation link is in the last)
+    fetch(0);
+    uint32_t all = 0;  // the hit successors' tags together
+    if (wballot(more & (es[1] >= 0))) {
+      fetch(1);
+      if (wballot(more & (es[2] >= 0))) {
+        fetch(2);
+        fetch(3);
+        test(2);
+        test(3);
+        all = (hit[2] ? (uint32_t)es[2] : 0u) | (hit[3] ? (uint32_t)es[3] : 0u);
+      }
+      test(1);
+      all |= hit[1] ? (uint32_t)es[1] : 0u;
+    }
+    test(0);
+    all |= hit[0] ? (uint32_t)es[0] : 0u;
+    bool any = false, several = false;
+    uint32_t first = 0;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      keep[s] = hit[s] & ((es[s] & kFlagDeadEnd) == 0) & !last;
+      several |= keep[s] & any;
+      first = (keep[s] & !any) ? (uint32_t)es[s] : first;
+      any |= keep[s];
+    }
+    if (NGAP_MOSTLY(wballot(((all & (uint32_t)(kFlagReport | kFlagDedup)) != 0) | several |
+                            (any & (has_next | !can_priv)) | (more & (es[3] <= -2))) == 0)) {
+      nv = any ? first : nv;
+      has_next |= any;
+      break;
+    }
+    if (wballot((all & (uint32_t)kFlagReport) != 0)) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        emit(P, W, hit[s] & ((es[s] & kFlagReport) != 0),
+             item_of(((uint32_t)es[s] & (uint32_t)kIdMask) | I.gtag, p1));
+    }
+    if (P.dedup && wballot((all & (uint32_t)kFlagDedup) != 0)) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        if (keep[s] & ((es[s] & kFlagDedup) != 0))
+          keep[s] =
+              dedup_fresh(P, W, item_of(((uint32_t)es[s] & (uint32_t)kIdMask) | I.gtag, p1));
+      wsync();
+    }
+    bool queue[4];
+    any = false;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const bool take = keep[s] & !has_next & can_priv;
+      nv = take ? (uint32_t)es[s] : nv;
+      has_next |= take;
+      queue[s] = keep[s] & !take;
+      any |= queue[s];
+    }
+    if (wballot(any)) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        push(P, W, queue[s], item_of(((uint32_t)es[s] & (uint32_t)kIdMask) | I.gtag, p1));
+    }
+    // a continuation record (more than four successors)
+    more &= es[3] <= -2;
+    if (wballot(more) == 0) break;
+    const uint32_t link = more ? (uint32_t)-(es[3] + 2) << 5 : 0u;
+    ids = load_at<int4>(P.img.succ4, link);
+    tests = load_at<uint4>(P.img.succ4, link + 16);
+  }
+  I.pos = has_next ? p1 : kNoItem;
+  I.rec = has_next ? I.rec_base + ((nv & (uint32_t)kIdMask) << 5) : 0u;
+  depth += 1;
+}
+
+template <bool Gen>
+__global__ void __launch_bounds__(kBlockThreads) k_scan(KParams P) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const uint32_t wave = from_first(threadIdx.x / kWave);
+  uint2 *bases = reinterpret_cast<uint2 *>(lds);
+  for (uint32_t g = threadIdx.x; g < P.num_groups; g += kBlockThreads)
+    bases[g] = *reinterpret_cast<const uint2 *>(&P.img.meta[g]);
+  WaveState W;
+  unsigned char *mine = lds + scan_table_bytes(P.num_groups) +
+                        wave * scan_wave_bytes(P.ring_cap);
+  setup_wave(W, mine, wave);
+  W.ring = reinterpret_cast<uint64_t *>(mine + kScanFixed);
+  ScanLds S;
+  S.mark = reinterpret_cast<uint32_t *>(W.dc + kDc);
+  S.bases = bases;
+  S.keys = reinterpret_cast<uint64_t *>(S.mark + kWave);
+  S.n_keys = 0;
+  W.open = reinterpret_cast<uint32_t *>(S.keys + kKeyCap);
+  clear_dedup(P, W);
+  __syncthreads();
+
+  uint32_t q = blockIdx.x % kQueues, cur = 0, end = 0;
+  bool more = true;
+  ScanItem I = {};
+  I.pos = kNoItem;
+  int depth = 0;
+  for (;;) {
+    // Below `low` queued items something comes before the next expansion:
+    // spilled items come back; else, while half the ring is still queued (so
+    // that the expansions after it find items for every idle lane), roots: of
+    // a wave's width of waiting 3-grams, or of what is left of them when no
+    // position can be searched any more.
+    const uint32_t qn = W.tail - W.head;
+    const bool search = (cur < end) | (more & (W.n_open < kMaxOpen));
+    const uint32_t low = W.spill_n ? kWave : (search | (S.n_keys != 0)) ? P.ring_cap / 2 : 0u;
+    if (qn < low) {
+      if (NGAP_SELDOM(W.spill_n)) {
+        refill_from_spill(P, W);
+        continue;
+      }
+      if ((S.n_keys >= kWave) | !search) {
+        take_keys(P, W, S);
+        continue;
+      }
+      if (NGAP_SELDOM(cur >= end)) {
+        const KParams &Q = cold_params();
+        const uint32_t t = claim_task(Q, W, q);
+        if (t >= Q.num_tasks) {
+          more = false;
+          continue;
+        }
+        const Task T = Gen ? gen_task(Q, t) : Q.tasks[t];
+        if (W.lane == 0) W.open[W.n_open] = t;
+        W.n_open++;
+        W.cstart = T.cstart;
+        W.cend = T.cend;
+        if ((T.flags & kTaskSeedStart) && Q.img.n_xsod) seed_start_all(Q, W);
+        cur = T.begin;
+        end = T.end;
+      }
+      const uint32_t stop = min_u(cur + 2 * kWave, end);
+      find_keys(P, W, S, cur, stop);
+      cur = stop;
+      continue;
+    }
+    const uint64_t idle = wballot(I.pos == kNoItem);
+    const uint32_t take = min_u(__popcll(idle), qn);
+    if (take) {
+      const uint32_t r = mask_rank(idle);
+      if ((I.pos == kNoItem) & (r < take)) {
+        const uint64_t it = W.ring[(W.head + r) & (P.ring_cap - 1)];
+        const uint32_t tagged = (uint32_t)it;
+        const uint2 base = S.bases[tagged >> 22];
+        I.pos = (uint32_t)(it >> 32);
+        I.gtag = tagged & ~(uint32_t)kIdMask;
+        I.rec_base = base.x << 5;
+        I.cls_base = base.y << 5;
+        I.rec = I.rec_base + ((tagged & (uint32_t)kIdMask) << 5);
+        depth = 0;
+      }
+      wsync();
+      W.head += take;
+    } else if (NGAP_SELDOM(idle == ~0ull)) {  // nothing queued, nothing in the lanes
+      close_open(W);
+      if (!more) break;
+      continue;
+    }
+    expand_scan(P, W, I, depth);
+  }
+  flush_reports(W);
+  if (W.lane == 0) add_items(W.items);
 }
 
 // Plain schedule: the cursor over a (group, chunk) unit shared by the block's
@@ -1001,7 +1454,7 @@ struct SharedCursor {
   NGAP_DEV bool next(const WaveState &W, uint32_t &a, uint32_t &b) {
     uint32_t x = 0;
     if (W.lane == 0) x = atomicAdd(cursor, batch);
-    x = __shfl(x, 0, 64);
+    x = from_first(x);
     if (x >= end) return false;
     a = x;
     b = x + batch < end ? x + batch : end;
@@ -1023,14 +1476,13 @@ struct LocalCursor {
 
 __global__ void __launch_bounds__(kBlockThreads) k_plain(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t wave = from_first(threadIdx.x / kWave);
   const uint32_t unit = blockIdx.x;
   const uint32_t g = unit % P.num_groups, c = unit / P.num_groups;
   uint32_t *cursor = reinterpret_cast<uint32_t *>(lds);
-  const uint32_t wbytes = wave_lds_bytes(P.ring_cap, P.rbuf_cap, P.dc_cap);
+  const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
-  setup_wave(P, W, lds + 16 + wave * wbytes,
-             P.spill + ((size_t)unit * P.waves_per_block + wave) * P.spill_cap);
+  setup_wave(W, lds + 16 + wave * wbytes, wave);
   begin_unit(P, W, g, c * P.chunk_len, (c + 1) * P.chunk_len);
   if (threadIdx.x == 0) *cursor = W.cstart;
   __syncthreads();
@@ -1040,20 +1492,19 @@ __global__ void __launch_bounds__(kBlockThreads) k_plain(KParams P) {
   }
   SharedCursor src{cursor, W.cend, P.root_batch};
   drain<false>(P, W, src);
-  flush_reports(P, W);
+  flush_reports(W);
   if (W.lane == 0) {
     if (W.overflow && atomicOr(&P.overflow[unit], 1u) == 0u) atomicAdd(P.overflow_count, 1u);
-    add_items(P, W.items);
+    add_items(W.items);
   }
 }
 
 __global__ void __launch_bounds__(kBlockThreads) k_batched(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t wave = threadIdx.x / kWave;
-  const uint32_t wbytes = wave_lds_bytes(P.ring_cap, P.rbuf_cap, P.dc_cap);
+  const uint32_t wave = from_first(threadIdx.x / kWave);
+  const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
-  setup_wave(P, W, lds + 16 + wave * wbytes,
-             P.spill + ((size_t)blockIdx.x * P.waves_per_block + wave) * P.spill_cap);
+  setup_wave(W, lds + 16 + wave * wbytes, wave);
   uint32_t q = blockIdx.x % kQueues;
   for (;;) {
     const uint32_t t = claim_task(P, W, q);
@@ -1083,8 +1534,8 @@ __global__ void __launch_bounds__(kBlockThreads) k_batched(KParams P) {
       if (P.task_items) P.task_items[ti] = W.items - items0;
     }
   }
-  flush_reports(P, W);
-  if (W.lane == 0) add_items(P, W.items);
+  flush_reports(W);
+  if (W.lane == 0) add_items(W.items);
 }
 
 // The batched engine without per-work-item traces: each wave overlaps its
@@ -1095,30 +1546,28 @@ __global__ void __launch_bounds__(kBlockThreads) k_batched(KParams P) {
 template <int End, bool Gen>
 __global__ void __launch_bounds__(kBlockThreads) k_batched_stream(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t wave = threadIdx.x / kWave;
-  const uint32_t wbytes = wave_lds_bytes(P.ring_cap, P.rbuf_cap, P.dc_cap);
+  const uint32_t wave = from_first(threadIdx.x / kWave);
+  const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
-  setup_wave(P, W, lds + 16 + wave * wbytes,
-             P.spill + ((size_t)blockIdx.x * P.waves_per_block + wave) * P.spill_cap);
+  setup_wave(W, lds + 16 + wave * wbytes, wave);
   clear_dedup(P, W);
   drain_stream<false, End, Gen>(P, W);
-  flush_reports(P, W);
-  if (W.lane == 0) add_items(P, W.items);
+  flush_reports(W);
+  if (W.lane == 0) add_items(W.items);
 }
 
 // The streaming kernel after a root pass (k_roots): its work items' roots
 // are read from root_items, so it holds only the expansion's registers.
 __global__ void __launch_bounds__(kBlockThreads) k_expand(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t wave = threadIdx.x / kWave;
-  const uint32_t wbytes = wave_lds_bytes(P.ring_cap, P.rbuf_cap, P.dc_cap);
+  const uint32_t wave = from_first(threadIdx.x / kWave);
+  const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
-  setup_wave(P, W, lds + 16 + wave * wbytes,
-             P.spill + ((size_t)blockIdx.x * P.waves_per_block + wave) * P.spill_cap);
+  setup_wave(W, lds + 16 + wave * wbytes, wave);
   clear_dedup(P, W);
   drain_stream<true, kEndChunkLen, false>(P, W);
-  flush_reports(P, W);
-  if (W.lane == 0) add_items(P, W.items);
+  flush_reports(W);
+  if (W.lane == 0) add_items(W.items);
 }
 
 // Root pass of an engine run: one wave per piece of a work item (a non-
@@ -1128,12 +1577,12 @@ __global__ void __launch_bounds__(kBlockThreads) k_expand(KParams P) {
 // k_batched_stream then expands the items.
 __global__ void __launch_bounds__(kBlockThreads) k_roots(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t wave = from_first(threadIdx.x / kWave);
   const uint32_t piece = blockIdx.x * P.waves_per_block + wave;
   if (piece >= P.num_pieces) return;  // wave-uniform; no block barrier follows
-  const uint32_t wbytes = wave_lds_bytes(P.ring_cap, P.rbuf_cap, P.dc_cap);
+  const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
-  setup_wave(P, W, lds + 16 + wave * wbytes, nullptr);
+  setup_wave(W, lds + 16 + wave * wbytes, wave);
   const RootPiece R = P.pieces[piece];
   const Task T = P.tasks[R.task];
   const uint64_t o0 = P.root_off[R.task];
@@ -1155,7 +1604,8 @@ __global__ void __launch_bounds__(kBlockThreads) k_roots(KParams P) {
       roots<true>(P, W, a, min_u(a + kWave, R.end));
   }
   flush_stage(P, W);
-  flush_reports(P, W);
+  flush_reports(W);
+  if (W.lane == 0 && W.items) add_items(W.items);  // the filtered ones
   if (W.lane == 0 && W.overflow && atomicOr(&P.overflow[R.task], kRootOverflow) == 0u)
     atomicAdd(P.overflow_count, 1u);
 }
@@ -1171,7 +1621,7 @@ NGAP_DEV void block_append(const KParams &P, WaveState &W, uint32_t *count, uint
   if (m == 0) return;
   uint32_t base = 0;
   if (W.lane == 0) base = atomicAdd(count, (uint32_t)__popcll(m));
-  base = __shfl(base, 0, 64);
+  base = from_first(base);
   const uint32_t slot = base + mask_rank(m);
   if (pred) {
     if (slot < P.spill_cap) buf[slot] = u;
@@ -1181,13 +1631,13 @@ NGAP_DEV void block_append(const KParams &P, WaveState &W, uint32_t *count, uint
 
 __global__ void __launch_bounds__(kBlockThreads) k_blocking(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t wave = from_first(threadIdx.x / kWave);
   const uint32_t unit = blockIdx.x;
   const uint32_t g = unit % P.num_groups, c = unit / P.num_groups;
   uint32_t *count = reinterpret_cast<uint32_t *>(lds);  // [0] current, [1] next
-  const uint32_t wbytes = wave_lds_bytes(P.ring_cap, P.rbuf_cap, P.dc_cap);
+  const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
-  setup_wave(P, W, lds + 16 + wave * wbytes, nullptr);
+  setup_wave(W, lds + 16 + wave * wbytes, wave);
   begin_unit(P, W, g, c * P.chunk_len, (c + 1) * P.chunk_len);
   uint32_t *front = reinterpret_cast<uint32_t *>(P.spill) + (size_t)unit * 2 * P.spill_cap;
   const GroupMeta gm = P.img.meta[g];
@@ -1269,10 +1719,10 @@ __global__ void __launch_bounds__(kBlockThreads) k_blocking(KParams P) {
     if (threadIdx.x == 0) count[sel] = 0;
     __syncthreads();
   }
-  flush_reports(P, W);
+  flush_reports(W);
   if (W.lane == 0) {
     if (W.overflow && atomicOr(&P.overflow[unit], 1u) == 0u) atomicAdd(P.overflow_count, 1u);
-    add_items(P, W.items);
+    add_items(W.items);
   }
 }
 
@@ -1331,6 +1781,8 @@ static const void *batched_kernel(int kind) {
     case 2: return reinterpret_cast<const void *>(k_expand);
     case 3: return reinterpret_cast<const void *>(k_batched_stream<kEndMap, false>);
     case 4: return reinterpret_cast<const void *>(k_batched_stream<kEndChunkLen, true>);
+    case 5: return reinterpret_cast<const void *>(k_scan<false>);
+    case 6: return reinterpret_cast<const void *>(k_scan<true>);
     default: return reinterpret_cast<const void *>(k_batched);
   }
 }
@@ -1352,6 +1804,12 @@ hipError_t launch_batched(hipStream_t s, const KParams &P, uint32_t blocks, uint
     case 4:
       hipLaunchKernelGGL((k_batched_stream<kEndChunkLen, true>), dim3(blocks),
                          dim3(kBlockThreads), lds, s, P);
+      break;
+    case 5:
+      hipLaunchKernelGGL(k_scan<false>, dim3(blocks), dim3(kBlockThreads), lds, s, P);
+      break;
+    case 6:
+      hipLaunchKernelGGL(k_scan<true>, dim3(blocks), dim3(kBlockThreads), lds, s, P);
       break;
     default:
       hipLaunchKernelGGL(k_batched, dim3(blocks), dim3(kBlockThreads), lds, s, P);

@@ -19,6 +19,7 @@ ImageSizes sizes_of(const Image &img) {
     z.beg[d] = img.memo[d].beg.size() * 4;
     z.nrep[d] = img.memo[d].nrep.size() * 4;
     z.list[d] = img.memo[d].list.size() * 4;
+    z.filt[d] = img.memo[d].filt.size() * 4;
     z.sel[d] = img.memo[d].sel.size() * 4;
   }
   z.mask1 = img.mask1.size() * 4;
@@ -30,6 +31,8 @@ ImageSizes sizes_of(const Image &img) {
   z.xsod = img.xsod.size() * 4;
   z.xs3 = img.xs3.size() * 4;
   z.xp3 = img.xp3.size() * 4;
+  z.xf3 = img.xf3.size() * 4;
+  z.xb3 = img.xb3.size() * 4;
   z.x2rep = img.x2rep.size() * 4;
   return z;
 }
@@ -48,7 +51,8 @@ inline bool has_byte(const uint32_t *sets, int v, int b) {
 }
 
 // Appends one list (reporting entries first, each part in id order).
-void push_list(MemoLevel &m, std::vector<int32_t> &ids, const std::vector<int32_t> &tag) {
+void push_list(MemoLevel &m, std::vector<int32_t> &ids, const std::vector<int32_t> &tag,
+               const std::vector<uint32_t> &filt) {
   std::sort(ids.begin(), ids.end(), [&](int32_t a, int32_t b) {
     bool ra = tag[a] & kFlagReport, rb = tag[b] & kFlagReport;
     if (ra != rb) return ra;
@@ -58,6 +62,7 @@ void push_list(MemoLevel &m, std::vector<int32_t> &ids, const std::vector<int32_
   for (int32_t v : ids) {
     if (tag[v] & kFlagReport) nrep++;
     m.list.push_back(tag[v]);
+    m.filt.push_back(filt[v]);
   }
   m.nrep.push_back(nrep);
   m.beg.push_back((uint32_t)m.list.size());
@@ -122,7 +127,12 @@ bool build_part(const HostGroup &hg, int32_t g, int memo_depth, GroupPart &P) {
     for (int u : succ[v]) indeg[u]++;
   }
   std::vector<int32_t> tag(n);
+  std::vector<uint32_t> filt(n, 0);  // next-byte filters
   for (int v = 0; v < n; v++) {
+    uint32_t any = 0;
+    for (int u : succ[v])
+      for (int w = 0; w < 8; w++) any |= hg.sets[(size_t)u * 8 + w];
+    filt[v] = filter_of(any);
     int32_t t = v;
     if (hg.attrs[v] & 2) t |= kFlagReport;
     if (succ[v].empty()) t |= kFlagDeadEnd;
@@ -184,7 +194,7 @@ bool build_part(const HostGroup &hg, int32_t g, int memo_depth, GroupPart &P) {
     std::sort(l1[b].begin(), l1[b].end());
     l1[b].erase(std::unique(l1[b].begin(), l1[b].end()), l1[b].end());
     if (!l1[b].empty()) P.mask1[b / 32] |= 1u << (b % 32);
-    push_list(P.memo[0], l1[b], tag);
+    push_list(P.memo[0], l1[b], tag, filt);
     if (P.memo[0].nrep.back()) P.mask1[8 + b / 32] |= 1u << (b % 32);
   }
   // deeper levels, each list's successors split by the next byte
@@ -215,7 +225,7 @@ bool build_part(const HostGroup &hg, int32_t g, int memo_depth, GroupPart &P) {
           if (d == 2) P.key2.push_back(((uint32_t)li << 8) | (uint32_t)b);
           else P.key3.push_back((P.key2[li] << 8) | (uint32_t)b);
           cur_lists.push_back(bucket[b]);
-          push_list(m, bucket[b], tag);
+          push_list(m, bucket[b], tag, filt);
         }
       }
     }
@@ -291,6 +301,7 @@ bool build_image(const HostGroup *groups, int32_t num_groups, int32_t memo_depth
       for (size_t i = 1; i < pm.beg.size(); i++) m.beg.push_back(list_base + pm.beg[i]);
       m.nrep.insert(m.nrep.end(), pm.nrep.begin(), pm.nrep.end());
       m.list.insert(m.list.end(), pm.list.begin(), pm.list.end());
+      m.filt.insert(m.filt.end(), pm.filt.begin(), pm.filt.end());
       const size_t s0 = m.sel.size();
       m.sel.insert(m.sel.end(), pm.sel.begin(), pm.sel.end());
       for (size_t i = s0 + 1; i < m.sel.size(); i += 2) m.sel[i] += key_base;
@@ -351,15 +362,18 @@ bool build_image(const HostGroup *groups, int32_t num_groups, int32_t memo_depth
       for (size_t i = 0; i < key3.size(); i++) order[at[key3[i]]++] = (uint32_t)i;
     }
     img.xs3.assign(2u << 24, 0);
+    img.xb3.assign(1u << 19, 0);
     img.xp3.reserve(m3.list.size() * 2);
     for (uint32_t k = 0; k < (1u << 24); k++) {
       const uint32_t n = start[k + 1] - start[k];
       if (n == 0) continue;
+      img.xb3[k >> 5] |= 1u << (k & 31);
       const uint32_t li0 = order[start[k]];
       if (n == 1 && m3.beg[li0 + 1] - m3.beg[li0] == 1) {
         // one group, one state: the slot holds the state itself
-        img.xs3[2 * (size_t)k] = (uint32_t)m3.list[m3.beg[li0]];
-        img.xs3[2 * (size_t)k + 1] = kSlotInline | grp3[li0];
+        const uint32_t f = m3.filt[m3.beg[li0]];
+        img.xs3[2 * (size_t)k] = (uint32_t)m3.list[m3.beg[li0]] | slot_filter_low(f);
+        img.xs3[2 * (size_t)k + 1] = kSlotInline | grp3[li0] | slot_filter_high(f);
         continue;
       }
       const size_t first = img.xp3.size() / 2;
@@ -368,6 +382,7 @@ bool build_image(const HostGroup *groups, int32_t num_groups, int32_t memo_depth
         for (uint32_t i = m3.beg[li]; i < m3.beg[li + 1]; i++) {
           img.xp3.push_back((uint32_t)m3.list[i]);
           img.xp3.push_back(grp3[li]);
+          img.xf3.push_back(m3.filt[i]);
         }
       }
       if (img.xp3.size() / 2 >= (1ull << 31)) {
@@ -393,6 +408,8 @@ bool build_image(const HostGroup *groups, int32_t num_groups, int32_t memo_depth
     }
   }
   img.n_xsod = img.xsod.size() / 2;
+  for (int d = 0; d < 2; d++)
+    for (uint32_t r : img.memo[d].nrep) img.short_reports |= r != 0;
   for (auto &m : img.memo)
     if (m.list.size() >= (1ull << 31)) {
       err = "memo tables too large (2^31 entries); use a smaller precompute depth";

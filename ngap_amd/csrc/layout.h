@@ -51,6 +51,36 @@ constexpr uint32_t kSlotInline = 1u << 31;    // 3-gram slot holds its one state
 // first two bytes a reporting depth-2 list, in some group
 constexpr uint32_t kSlotPrefixReports = 1u << 30;
 
+// Next-byte filter of a state: which bytes can match one of its (non-all-
+// input) successors, folded to 27 bits: byte b counts at bit b % 32, the last
+// bit for 26..31 too.  A byte whose bit is clear matches no successor, so an
+// item whose next byte fails its state's filter expands to nothing and need
+// not be queued.  A literal successor passes one byte in 27, a class of 17
+// random bytes about half of them; the letters of either case have bits of
+// their own.
+#if defined(__HIPCC__)
+#define NGAP_LHD __host__ __device__
+#else
+#define NGAP_LHD
+#endif
+constexpr uint32_t kFilterTop = 26;
+NGAP_LHD inline uint32_t filter_bit(uint32_t b) {
+  const uint32_t x = b & 31;
+  return x < kFilterTop ? x : kFilterTop;
+}
+NGAP_LHD inline uint32_t filter_of(uint32_t words_or) {  // the class's eight words, or-ed
+  return (words_or & ((1u << kFilterTop) - 1)) | ((words_or >> kFilterTop) ? 1u << kFilterTop : 0u);
+}
+// The filter of an inline 3-gram slot's state lies in the slot's spare bits:
+// 25-31 of its first word (the tagged state) and 10-29 of the second (the
+// group).
+constexpr int kSlotFilterLow = 7;  // filter bits in the first word
+NGAP_LHD inline uint32_t slot_filter(uint32_t w0, uint32_t w1) {
+  return (w0 >> 25) | (((w1 >> 10) & 0xFFFFFu) << kSlotFilterLow);
+}
+NGAP_LHD inline uint32_t slot_filter_low(uint32_t f) { return f << 25; }
+NGAP_LHD inline uint32_t slot_filter_high(uint32_t f) { return (f >> kSlotFilterLow) << 10; }
+
 struct HostGroup {  // what the C ABI hands in for one group
   int32_t num_states = 0;
   const int32_t *row = nullptr;
@@ -87,6 +117,7 @@ struct MemoLevel {            // one depth for all groups
   std::vector<uint32_t> nrep;  // reporting entries at the head of each list
   std::vector<uint32_t> sel;   // d >= 2: rank table, (word, rank) pairs
   std::vector<int32_t> list;   // tagged state ids
+  std::vector<uint32_t> filt;  // the next-byte filter of each list entry's state
   uint64_t keys() const { return nrep.size(); }
 };
 
@@ -111,19 +142,24 @@ struct Image {
   //   xsod: (tagged id, group) pairs of every group's start-of-data states.
   //   x3 (depth 3): 3-gram k -> every group's depth-3 list, through the
   //       8-byte slot xs3[2k], xs3[2k+1]: (0, 0) when no group has one;
-  //       (tagged state, kSlotInline | group) when exactly one group has one
-  //       and it holds one state (the common case: one load, no list);
+  //       (tagged state, kSlotInline | group), with the state's next-byte
+  //       filter in the spare bits, when exactly one group has one and it
+  //       holds one state (the common case: one load, no list);
   //       otherwise (first pair, pair count) into xp3, whose 8-byte pairs
   //       (tagged state, group) are the states of every group's list, group
   //       by group in list order: a lookup reads the slot, then its pairs,
-  //       with no list indirection.  Bit 30 of the second word
+  //       with no list indirection; xf3 holds each pair's next-byte filter.
+  //       Bit 30 of the second word
   //       (kSlotPrefixReports) flags the 3-grams whose first byte has a
   //       reporting depth-1 list or whose first two bytes have a reporting
   //       depth-2 list in some group (the count is the word without it).
+  //       xb3 has a bit per 3-gram that some group has a list for (bit k % 32
+  //       of word k / 32).
   //       x2rep marks the 2-grams that have a reporting depth-2 list (2048
   //       words).
-  std::vector<uint32_t> xr1, xe1, xmask1, xr2, xe2, xsod, xs3, xp3, x2rep;
+  std::vector<uint32_t> xr1, xe1, xmask1, xr2, xe2, xsod, xs3, xp3, xf3, xb3, x2rep;
   uint64_t n_xsod = 0;          // (state, group) pairs in xsod
+  bool short_reports = false;   // some depth-1 or depth-2 list has a reporting entry
   uint64_t total_states = 0;
 };
 
@@ -132,13 +168,14 @@ struct Image {
 struct ImageSizes {
   uint64_t meta = 0, succ4 = 0, cls = 0, sod = 0;
   uint64_t beg[kMaxMemoDepth] = {0, 0, 0}, nrep[kMaxMemoDepth] = {0, 0, 0},
-           list[kMaxMemoDepth] = {0, 0, 0}, sel[kMaxMemoDepth] = {0, 0, 0};
+           list[kMaxMemoDepth] = {0, 0, 0}, filt[kMaxMemoDepth] = {0, 0, 0},
+           sel[kMaxMemoDepth] = {0, 0, 0};
   uint64_t mask1 = 0, xr1 = 0, xe1 = 0, xmask1 = 0, xr2 = 0, xe2 = 0, xsod = 0, xs3 = 0,
-           xp3 = 0, x2rep = 0;
+           xp3 = 0, xf3 = 0, xb3 = 0, x2rep = 0;
   uint64_t total() const {
     uint64_t t = meta + succ4 + cls + sod + mask1 + xr1 + xe1 + xmask1 + xr2 + xe2 + xsod + xs3 +
-                 xp3 + x2rep;
-    for (int d = 0; d < kMaxMemoDepth; d++) t += beg[d] + nrep[d] + list[d] + sel[d];
+                 xp3 + xf3 + xb3 + x2rep;
+    for (int d = 0; d < kMaxMemoDepth; d++) t += beg[d] + nrep[d] + list[d] + filt[d] + sel[d];
     return t;
   }
 };

@@ -10,6 +10,7 @@
 // the kernel from their index, so nothing is uploaded.  Every run on a device
 // shares that device's array: runs that overlap on one device race, and the
 // counters and flags are cleared by a kernel at the start of every run.
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 
@@ -85,16 +86,19 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     KParams P = base_params(eng, mp, o);
     P.ring_cap = ring_of(o);
     P.input = d_input;
-    P.chunk_len = (uint32_t)chunk_len;
-    P.chunk_magic = ~0ull / P.chunk_len + 1;
+    set_chunk_len(P, (uint32_t)chunk_len);
     P.num_seg = num_seg;
     // the schedule: all-group windows (depth >= 2) or one group per work item,
     // windows of about two work items per wave, on a grid sized to the job
     const uint32_t G = (uint32_t)eng->img.num_groups;
     P.gen_cross = mp.memo_depth >= 2 && o.cross_groups != 0;
-    const uint64_t work = (uint64_t)num_seg * chunk_len * (P.gen_cross ? 1 : G);
+    const uint64_t total = (uint64_t)num_seg * chunk_len;
+    const uint64_t work = total * (P.gen_cross ? 1 : G);
+    P.scan = P.gen_cross && scan_image(eng, mp, total);
+    P.load_last = (uint32_t)(total - std::min<uint64_t>(total, 8));
+    const int kind = P.scan ? 6 : 4;  // of generated work items
     uint32_t blocks = 0;
-    int rc = persistent_blocks(eng, o.persistent_blocks, &blocks, P.ring_cap, 4);  // generated work items
+    int rc = persistent_blocks(eng, o.persistent_blocks, &blocks, P.ring_cap, kind);
     if (rc) return rc;
     if (!o.persistent_blocks) blocks = job_blocks(blocks, P.waves_per_block, work);
     const uint64_t waves = (uint64_t)blocks * P.waves_per_block;
@@ -135,7 +139,7 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     HIP_TRY(launch_reset(ctx.stream, P.report_count, P.items, P.task_head, P.overflow,
                          P.num_tasks, P.overflow_count, 0, nullptr));
     HIP_TRY(hipEventRecord(ctx.ev0, ctx.stream));
-    HIP_TRY(launch_batched(ctx.stream, P, blocks, lds_bytes(P.ring_cap)));
+    HIP_TRY(launch_batched(ctx.stream, P, blocks, batched_lds(P.ring_cap, kind, G)));
     HIP_TRY(hipEventRecord(ctx.ev1, ctx.stream));
     HIP_TRY(hipMemcpyAsync(ctx.host_cnt, counters, kCounterBytes, hipMemcpyDeviceToHost,
                            ctx.stream));

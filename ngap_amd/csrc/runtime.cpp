@@ -162,7 +162,12 @@ void RunCtx::drop_graph() {
 }
 
 uint32_t lds_bytes(uint32_t ring) {
-  return 16 + (kBlockThreads / kWave) * wave_lds_bytes(ring, kRbuf, kDc);
+  return 16 + (kBlockThreads / kWave) * wave_lds_bytes(ring);
+}
+
+uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups) {
+  if (kind < 5) return lds_bytes(ring);
+  return scan_table_bytes(groups) + (kBlockThreads / kWave) * scan_wave_bytes(ring);
 }
 
 // ring_capacity option -> LDS ring entries (0 = default); 0 when invalid
@@ -229,6 +234,7 @@ KParams base_params(const ngap_engine *eng, const Mapping &mp, const ngap_run_op
     P.img.beg[d] = eng->d_beg[d].as<uint32_t>();
     P.img.nrep[d] = eng->d_nrep[d].as<uint32_t>();
     P.img.list[d] = eng->d_list[d].as<int32_t>();
+    P.img.filt[d] = eng->d_filt[d].as<uint32_t>();
     P.img.sel[d] = eng->d_sel[d].as<uint32_t>();
   }
   P.img.mask1 = eng->d_mask1.as<uint32_t>();
@@ -240,6 +246,8 @@ KParams base_params(const ngap_engine *eng, const Mapping &mp, const ngap_run_op
   P.img.xsod = eng->d_xsod.as<uint32_t>();
   P.img.xs3 = eng->d_xs3.as<uint32_t>();
   P.img.xp3 = eng->d_xp3.as<uint32_t>();
+  P.img.xf3 = eng->d_xf3.as<uint32_t>();
+  P.img.xb3 = eng->d_xb3.as<uint32_t>();
   P.img.x2rep = eng->d_x2rep.as<uint32_t>();
   P.img.n_xsod = (uint32_t)eng->img.n_xsod;
   P.num_groups = (uint32_t)eng->img.num_groups;
@@ -250,8 +258,6 @@ KParams base_params(const ngap_engine *eng, const Mapping &mp, const ngap_run_op
   P.active_threshold = o.active_threshold;
   P.report_off = o.report_off;
   P.ring_cap = o.schedule == NGAP_SCHED_BATCHED && ring_of(o) ? ring_of(o) : kRing;
-  P.rbuf_cap = kRbuf;
-  P.dc_cap = kDc;
   P.root_batch = (uint32_t)mp.root_batch;
   P.waves_per_block = kBlockThreads / kWave;
   return P;
@@ -269,15 +275,24 @@ void attach_ctx(KParams &P, RunCtx &ctx) {
 }
 
 // Kernel kind an engine run of o launches: 0 k_batched (traces), 1
-// k_batched_stream, 2 k_expand (after the root pass).
-int engine_kind(const ngap_run_opts &o) { return o.task_traces ? 0 : o.root_pass ? 2 : 1; }
+// k_batched_stream, 2 k_expand (after the root pass), 5 k_scan.
+int engine_kind(const ngap_run_opts &o, bool scan) {
+  return o.task_traces ? 0 : o.root_pass ? 2 : scan ? 5 : 1;
+}
+
+bool scan_image(const ngap_engine *eng, const Mapping &mp, uint64_t input_len) {
+  // 32-bit byte offsets into records and classes: at most 2^27 of each
+  return mp.memo_depth == 3 && !eng->img.short_reports && input_len >= 8 &&
+         eng->img_sizes.succ4 < (1ull << 32) && eng->img_sizes.cls < (1ull << 32);
+}
 
 int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *blocks,
                       uint32_t ring, int kind) {
   const int slot = kBatchedKinds * (31 - __builtin_clz(ring)) + kind;  // ring in [64, 2048]
   int per_cu = eng->batched_per_cu[slot];
   if (per_cu == 0) {
-    HIP_TRY(batched_occupancy(&per_cu, lds_bytes(ring), kind));
+    HIP_TRY(batched_occupancy(&per_cu, batched_lds(ring, kind, (uint32_t)eng->img.num_groups),
+                              kind));
     const_cast<ngap_engine *>(eng)->batched_per_cu[slot] = per_cu;
   }
   if (per_cu < 1) per_cu = 1;
@@ -344,7 +359,8 @@ static int root_areas(const ngap_engine *eng, RunCtx &ctx, const std::vector<Tas
 static int launch_batched_ctx(RunCtx &ctx, const KParams &P, uint32_t blocks, uint32_t n_flags,
                               bool keep_reports, bool use_graph, hipEvent_t begin,
                               hipEvent_t end) {
-  const uint32_t lds = lds_bytes(P.ring_cap);
+  const uint32_t lds = batched_lds(P.ring_cap, batched_kind(P), P.num_groups);
+  const uint32_t root_lds = lds_bytes(P.ring_cap);
   HIP_TRY(launch_reset(ctx.stream, P.report_count, P.items, P.task_head, P.overflow, n_flags,
                        P.overflow_count, keep_reports, P.root_count));
   if (use_graph) {
@@ -354,7 +370,7 @@ static int launch_batched_ctx(RunCtx &ctx, const KParams &P, uint32_t blocks, ui
     if (!ctx.gexec || key != ctx.gkey) {
       ctx.drop_graph();
       HIP_TRY(hipStreamBeginCapture(ctx.stream, hipStreamCaptureModeThreadLocal));
-      hipError_t e4 = P.root_items ? launch_roots(ctx.stream, P, lds) : hipSuccess;
+      hipError_t e4 = P.root_items ? launch_roots(ctx.stream, P, root_lds) : hipSuccess;
       hipError_t e2 = launch_batched(ctx.stream, P, blocks, lds);
       hipGraph_t g = nullptr;
       hipError_t e3 = hipStreamEndCapture(ctx.stream, &g);
@@ -371,7 +387,7 @@ static int launch_batched_ctx(RunCtx &ctx, const KParams &P, uint32_t blocks, ui
     return NGAP_OK;
   }
   HIP_TRY(hipEventRecord(begin, ctx.stream));
-  if (P.root_items) HIP_TRY(launch_roots(ctx.stream, P, lds));
+  if (P.root_items) HIP_TRY(launch_roots(ctx.stream, P, root_lds));
   HIP_TRY(launch_batched(ctx.stream, P, blocks, lds));
   HIP_TRY(hipEventRecord(end, ctx.stream));
   return NGAP_OK;
@@ -776,7 +792,7 @@ int ngap_create(int32_t device, ngap_engine **out) {
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, device));
     e->num_cus = prop.multiProcessorCount;
-    HIP_TRY(set_lds_limit(lds_bytes(kMaxRing)));
+    HIP_TRY(set_lds_limit(std::max(lds_bytes(kMaxRing), batched_lds(kMaxRing, 5, 1024))));
     rc = noalloc_attach(device, &e->scratch);  // this device's scratch array (noalloc.cpp)
     if (rc) return rc;
     *out = e.release();
@@ -901,11 +917,14 @@ int ngap_load_groups_ex(ngap_engine *eng, const ngap_group_desc *groups, int32_t
       HIP_TRY(eng->d_xsod.upload(im.xsod));
       HIP_TRY(eng->d_xs3.upload(im.xs3));
       HIP_TRY(eng->d_xp3.upload(im.xp3));
+      HIP_TRY(eng->d_xf3.upload(im.xf3));
+      HIP_TRY(eng->d_xb3.upload(im.xb3));
       HIP_TRY(eng->d_x2rep.upload(im.x2rep));
       for (int d = 0; d < kMaxMemoDepth; d++) {
         HIP_TRY(eng->d_beg[d].upload(im.memo[d].beg));
         HIP_TRY(eng->d_nrep[d].upload(im.memo[d].nrep));
         HIP_TRY(eng->d_list[d].upload(im.memo[d].list));
+        HIP_TRY(eng->d_filt[d].upload(im.memo[d].filt));
         HIP_TRY(eng->d_sel[d].upload(im.memo[d].sel));
       }
       eng->img_sizes = sizes_of(im);
@@ -916,10 +935,12 @@ int ngap_load_groups_ex(ngap_engine *eng, const ngap_group_desc *groups, int32_t
       kept.meta.swap(im.meta);
       kept.mask1.swap(im.mask1);
       kept.n_xsod = im.n_xsod;
+      kept.short_reports = im.short_reports;
       kept.total_states = im.total_states;
       im = std::move(kept);
     }
     if (const int rc = pack_image(eng)) return rc;
+    for (int &n : eng->batched_per_cu) n = 0;  // k_scan's LDS depends on the groups
     eng->built_on_device = build == NGAP_BUILD_DEVICE;
     eng->build_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -969,7 +990,10 @@ int ngap_image_array(ngap_engine *eng, const char *name, void *out, uint64_t cap
         {"beg3", &eng->d_beg[2], z.beg[2]},   {"nrep1", &eng->d_nrep[0], z.nrep[0]},
         {"nrep2", &eng->d_nrep[1], z.nrep[1]}, {"nrep3", &eng->d_nrep[2], z.nrep[2]},
         {"list1", &eng->d_list[0], z.list[0]}, {"list2", &eng->d_list[1], z.list[1]},
-        {"list3", &eng->d_list[2], z.list[2]}, {"sel2", &eng->d_sel[1], z.sel[1]},
+        {"list3", &eng->d_list[2], z.list[2]}, {"filt1", &eng->d_filt[0], z.filt[0]},
+        {"filt2", &eng->d_filt[1], z.filt[1]}, {"filt3", &eng->d_filt[2], z.filt[2]},
+        {"xf3", &eng->d_xf3, z.xf3},          {"xb3", &eng->d_xb3, z.xb3},
+        {"sel2", &eng->d_sel[1], z.sel[1]},
         {"sel3", &eng->d_sel[2], z.sel[2]},   {"mask1", &eng->d_mask1, z.mask1},
         {"xr1", &eng->d_xr1, z.xr1},          {"xe1", &eng->d_xe1, z.xe1},
         {"xmask1", &eng->d_xmask1, z.xmask1}, {"xr2", &eng->d_xr2, z.xr2},
@@ -1071,8 +1095,7 @@ int ngap_run(ngap_engine *eng, const ngap_run_opts *opts, ngap_run_stats *st) {
     ctx.report_cap = o.report_off ? 0 : cap;
     KParams P = base_params(eng, mp, o);
     P.input = eng->d_input.as<uint8_t>();
-    P.chunk_len = (uint32_t)eng->chunk_len;
-    P.chunk_magic = ~0ull / P.chunk_len + 1;  // wraps to 0 for 1-byte chunks, as the test needs
+    set_chunk_len(P, (uint32_t)eng->chunk_len);
     P.num_seg = eng->num_seg;
     if (st) st->num_units = (uint32_t)units;
     if (o.schedule == NGAP_SCHED_PLAIN || o.algorithm == NGAP_ALGO_BLOCKING)
@@ -1084,24 +1107,31 @@ int ngap_run(ngap_engine *eng, const ngap_run_opts *opts, ngap_run_stats *st) {
     // one group included: a 3-gram slot per position replaces the group's
     // rank-table lookups (regex20k: 0.185 ms against 0.217)
     const int kind = o.tasks ? 0 : (mp.memo_depth >= 2 && o.cross_groups != 0) ? 1 : 2;
+    const uint64_t total = (uint64_t)eng->num_seg * eng->chunk_len;
+    bool scan = kind != 2 && scan_image(eng, mp, total);
+    for (uint32_t i = 0; kind == 0 && scan && i < o.num_tasks; i++)
+      scan = o.tasks[i].group == NGAP_ALL_GROUPS;
+    P.scan = scan;
+    P.load_last = (uint32_t)(total - std::min<uint64_t>(total, 8));
     // the default grid, sized to the job
     if (o.persistent_blocks == 0) {
       uint32_t full = 0;
-      int rc = persistent_blocks(eng, 0, &full, P.ring_cap, engine_kind(o));
+      int rc = persistent_blocks(eng, 0, &full, P.ring_cap, engine_kind(o, scan));
       if (rc) return rc;
       uint64_t work = 0;
       if (kind == 0) {
         for (uint32_t i = 0; i < o.num_tasks; i++)
           work += o.tasks[i].end > o.tasks[i].begin ? o.tasks[i].end - o.tasks[i].begin : 0;
       } else {
-        work = (uint64_t)eng->num_seg * eng->chunk_len * (kind == 2 ? eng->img.num_groups : 1);
+        work = total * (kind == 2 ? eng->img.num_groups : 1);
       }
       o.persistent_blocks = job_blocks(full, P.waves_per_block, work);
     }
     uint32_t waves = 0;
     if (kind != 0) {
       uint32_t blocks = 0;
-      int rc = persistent_blocks(eng, o.persistent_blocks, &blocks, P.ring_cap, engine_kind(o));
+      int rc = persistent_blocks(eng, o.persistent_blocks, &blocks, P.ring_cap,
+                                 engine_kind(o, scan));
       if (rc) return rc;
       waves = blocks * P.waves_per_block;
     }
@@ -1150,6 +1180,11 @@ int ngap_autotune(ngap_engine *eng, const ngap_run_opts *base, int32_t max_runs,
     o.tasks = nullptr;
     o.num_tasks = 0;
     const uint32_t L = (uint32_t)eng->chunk_len;
+    Mapping mp;
+    std::string err;
+    const bool scan = map_algorithm(o.algorithm, o.precompute_depth, eng->img.memo_depth, mp, err) &&
+                      o.cross_groups != 0 &&
+                      scan_image(eng, mp, eng->chunk_len * eng->num_seg);
     int runs = 0;
     double best_t = 1e300;
     ngap_run_opts cur = o;
@@ -1178,7 +1213,7 @@ int ngap_autotune(ngap_engine *eng, const ngap_run_opts *base, int32_t max_runs,
       if (axis == 2) {
         ngap_run_opts f = cur;
         f.persistent_blocks = 0;
-        int rc2 = persistent_blocks(eng, 0, &full, ring_of(f), engine_kind(f));
+        int rc2 = persistent_blocks(eng, 0, &full, ring_of(f), engine_kind(f, scan));
         if (rc2) return rc2;
       }
       const std::vector<uint32_t> grids = {full / 4, full / 2, (full * 3) / 4};
@@ -1235,7 +1270,9 @@ int ngap_batched_grid(ngap_engine *eng, uint32_t ring_capacity, uint32_t *blocks
     const uint32_t ring = ring_of(o);
     if (!ring) return ngap_fail(NGAP_ERR_INVALID, "ring_capacity must be a power of two in [64, 2048]");
     HIP_TRY(hipSetDevice(eng->device));
-    int rc = persistent_blocks(eng, 0, blocks, ring, engine_kind(o));
+    // the grid of all-group work items at the loaded depth
+    int rc = persistent_blocks(eng, 0, blocks, ring,
+                               engine_kind(o, scan_image(eng, {eng->img.memo_depth, 0, 0}, 8)));
     if (rc) return rc;
     *waves_per_block = kBlockThreads / kWave;
     return NGAP_OK;

@@ -29,8 +29,8 @@ int ngap_fail(int code, const std::string &msg);
 
 namespace ngapamd {
 
-// LDS capacities per wave (entries)
-constexpr uint32_t kRing = 256, kRbuf = 128, kDc = 256;
+// LDS ring entries per wave, by default
+constexpr uint32_t kRing = 256;
 constexpr uint32_t kMinRing = 64, kMaxRing = 2048;  // batched ring_capacity range
 
 // Device memory for one load: the builder's temporaries and the arrays it
@@ -177,6 +177,8 @@ struct Mapping {
 
 bool map_algorithm(int algorithm, int depth_req, int loaded_depth, Mapping &m, std::string &err);
 uint32_t lds_bytes(uint32_t ring = kRing);
+// LDS of a launch of the batched kernel `kind` over `groups` groups.
+uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups);
 
 // Sorts ctx's last n reports (offsets below 2^offset_bits) on the device and
 // encodes them (reports.hip): into ctx.host_reports[1..] up to kSmallReports,
@@ -202,20 +204,23 @@ hipError_t set_lds_limit(uint32_t lds);
 struct ngap_engine {
   int device = 0;
   int num_cus = 0;
-  // blocks per CU by (log2(ring), batched kernel kind), 0 = not queried
+  // blocks per CU by (log2(ring), batched kernel kind) for the loaded groups,
+  // 0 = not queried
   int batched_per_cu[12 * ngapamd::kBatchedKinds] = {0};
   ngapamd::Image img;
   bool loaded = false;
   ngapamd::Slab build_slab;  // the device builder's memory while a load runs
   ngapamd::DevBuf d_meta, d_succ4, d_cls, d_sod, d_mask1;
   ngapamd::DevBuf d_beg[ngapamd::kMaxMemoDepth], d_nrep[ngapamd::kMaxMemoDepth],
-      d_list[ngapamd::kMaxMemoDepth], d_sel[ngapamd::kMaxMemoDepth];
-  ngapamd::DevBuf d_xr1, d_xe1, d_xmask1, d_xr2, d_xe2, d_xsod, d_xs3, d_xp3, d_x2rep;
-  std::array<ngapamd::DevBuf *, 26> image_arrays() {
-    return {&d_succ4, &d_cls, &d_xs3, &d_xp3, &d_list[0], &d_list[1], &d_list[2], &d_sel[0],
-            &d_sel[1], &d_sel[2], &d_beg[0], &d_beg[1], &d_beg[2], &d_nrep[0], &d_nrep[1],
-            &d_nrep[2], &d_xr1, &d_xe1, &d_xmask1, &d_xr2, &d_xe2, &d_xsod, &d_x2rep, &d_meta,
-            &d_sod, &d_mask1};
+      d_list[ngapamd::kMaxMemoDepth], d_filt[ngapamd::kMaxMemoDepth],
+      d_sel[ngapamd::kMaxMemoDepth];
+  ngapamd::DevBuf d_xr1, d_xe1, d_xmask1, d_xr2, d_xe2, d_xsod, d_xs3, d_xp3, d_xf3, d_xb3,
+      d_x2rep;
+  std::array<ngapamd::DevBuf *, 31> image_arrays() {
+    return {&d_succ4, &d_cls, &d_xs3, &d_xp3, &d_xf3, &d_xb3, &d_list[0], &d_list[1],
+            &d_list[2], &d_filt[0], &d_filt[1], &d_filt[2], &d_sel[0], &d_sel[1], &d_sel[2],
+            &d_beg[0], &d_beg[1], &d_beg[2], &d_nrep[0], &d_nrep[1], &d_nrep[2], &d_xr1,
+            &d_xe1, &d_xmask1, &d_xr2, &d_xe2, &d_xsod, &d_x2rep, &d_meta, &d_sod, &d_mask1};
   }
   // one allocation holding every image array above (they are views into it)
   ngapamd::DevBuf d_arena;
@@ -247,7 +252,14 @@ struct ngap_engine {
 namespace ngapamd {
 KParams base_params(const ngap_engine *eng, const Mapping &mp, const ngap_run_opts &o);
 void attach_ctx(KParams &P, RunCtx &ctx);
-int engine_kind(const ngap_run_opts &o);
+int engine_kind(const ngap_run_opts &o, bool scan);
+// Whether all-group work items of this engine's runs take k_scan: memo depth
+// 3, no depth-1 or depth-2 reports in the image, records and classes below
+// 4 GiB each, and an input that holds an 8-byte load.  It was the faster one
+// wherever it can run: at equal windows of 1,024 positions 0.149 against 0.199 ms
+// (400,000 states, 16 MiB), 0.205 / 0.234 (1,024 automata, 8 MiB), 1.09 / 1.12
+// (64 MiB), 0.107 / 0.128 (short words in text).
+bool scan_image(const ngap_engine *eng, const Mapping &mp, uint64_t input_len);
 // Persistent grid of the batched kernel `kind` (batched_occupancy) for ring.
 int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *blocks,
                       uint32_t ring = kRing, int kind = 1);

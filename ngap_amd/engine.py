@@ -51,8 +51,9 @@ class Engine:
         self.max_depth = max(1, int(max_precompute_depth))
 
     IMAGE_ARRAYS = ("meta", "succ4", "cls", "sod", "beg1", "beg2", "beg3", "nrep1", "nrep2",
-                    "nrep3", "list1", "list2", "list3", "sel2", "sel3", "mask1", "xr1", "xe1",
-                    "xmask1", "xr2", "xe2", "xsod", "xs3", "xp3", "x2rep")
+                    "nrep3", "list1", "list2", "list3", "filt1", "filt2", "filt3", "sel2", "sel3",
+                    "mask1", "xr1", "xe1", "xmask1", "xr2", "xe2", "xsod", "xs3", "xp3", "xf3",
+                    "xb3", "x2rep")
 
     def image_info(self):
         info = _lib.ImageInfo()
