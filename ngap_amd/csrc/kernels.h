@@ -89,6 +89,7 @@ struct KParams {
   int32_t gen_cross;
   const uint32_t *task_order;  // nullable
   uint32_t num_tasks;
+  int32_t even;            // the work items cost about the same (all-group windows)
   uint32_t *task_head;     // kQueues claim counters, kQueueStride words apart
   unsigned long long *task_items;  // nullable, per task
   uint32_t waves_per_block;
@@ -121,23 +122,21 @@ constexpr uint32_t kWave = 64;
 constexpr uint32_t kMaxOpen = 8;  // work items a wave overlaps (k_batched)
 // LDS entries per wave: report buffer, de-duplication cache (power of two)
 constexpr uint32_t kRbuf = 128, kDc = 256;
-// The work queue is split by XCD: workgroup b runs on XCD b % 8, and queue q
-// holds work items q, q + 8, q + 16, ...; each claim counter has its own
-// 128-byte line.  A wave whose queue is empty takes from the next ones.
+// The work items that are no workgroup's own are split by XCD: workgroup b runs
+// on XCD b % 8, and queue q holds every eighth of them; each claim counter has
+// its own 128-byte line.
 constexpr uint32_t kQueues = 8, kQueueStride = 32;
 constexpr uint32_t kBlockThreads = 256;
 // Counters of a run (one buffer per run context, cleared by k_reset): bytes
 // 0-31 hold the report count and the count of overflowed work items (word
-// 3), byte 128 on the queue claim counters, then one mask per XCD of the
-// queues its waves found empty (one line each), then kItemLanes lines of
+// 3), byte 128 on the queue claim counters, then kItemLanes lines of
 // expanded-item counts, one 64-bit word at the start of each line:
 // the waves of workgroup b add theirs at lane b % kItemLanes and the host
 // sums the lanes.  A single count that every wave adds to as it ends costs
 // 5-8 % of a launch of the streaming kernel: atomics on one address
 // serialise.
 constexpr uint32_t kItemLanes = 32, kItemStride = 16;  // stride in 64-bit words
-constexpr uint32_t kEmptyMasks = kQueues * kQueueStride;  // task_head word of XCD 0's mask
-constexpr uint32_t kItemsWord = (128 + 2 * kQueues * kQueueStride * 4) / 8;
+constexpr uint32_t kItemsWord = (128 + kQueues * kQueueStride * 4) / 8;
 constexpr uint32_t kCounterBytes = (kItemsWord + kItemLanes * kItemStride) * 8;
 NGAP_HD inline unsigned long long items_sum(const unsigned long long *counters) {
   unsigned long long n = 0;

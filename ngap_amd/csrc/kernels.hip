@@ -925,33 +925,76 @@ NGAP_DEV void drain(const KParams &P, WaveState &W, Src &src) {
   }
 }
 
-// Claims the next work item for this wave: from the queue of its XCD first,
-// then from the others.  Returns P.num_tasks when all are empty.  `q` is the
-// wave's current queue (advanced when one runs dry).  A wave that finds a
-// queue empty adds it to its XCD's mask of empty queues and gets back what
-// the XCD's other waves found, so it claims only from queues not known to be
-// empty (a queue found empty stays empty): at the end of a run a wave learns
-// that every queue is empty from two atomics, not from a failed claim on each
-// of the eight counters, which thousands of waves would hit at once.
-NGAP_DEV uint32_t claim_task(const KParams &P, const WaveState &W, uint32_t &q) {
-  uint32_t *empty = P.task_head + kEmptyMasks + (blockIdx.x % kQueues) * kQueueStride;
-  uint32_t known = 0;
-  for (uint32_t tries = 0; tries < kQueues; tries++) {
-    uint32_t j = 0;
-    if (W.lane == 0) j = atomicAdd(P.task_head + q * kQueueStride, 1u);
-    j = from_first(j);
-    const uint64_t t = (uint64_t)j * kQueues + q;
-    if (t < P.num_tasks) return (uint32_t)t;
-    uint32_t m = 0;
-    if (W.lane == 0) m = atomicOr(empty, 1u << q);
-    known |= from_first(m) | (1u << q);
-    if (known == (1u << kQueues) - 1) return P.num_tasks;
-    uint32_t d = 1;
-    while ((known >> ((q + d) % kQueues)) & 1u) d++;
-    q = (q + d) % kQueues;
+// A wave's claims of work items.  A workgroup's own items (item i * workgroups +
+// workgroup is its i-th) are taken by its waves with an LDS counter, the others
+// are in one queue an XCD, from which a wave claims by an atomic in memory.  Such
+// an atomic is a round trip of 2 us, and those of thousands of waves on one address
+// take 20 ns each, one after the other: 2 MiB scanned in two items a wave took
+// 0.086 ms with all claimed so (the queues' ends found by two more atomics a wave)
+// and takes 0.056 with none.  So items of about the same cost (P.even) are all the
+// workgroups' own up to kOwnItems a wave, which is enough to even out the waves'
+// times within a workgroup, and three quarters of them above, where the rest evens
+// out the workgroups' (1,024 automata, 64 MiB, 16 items a wave: 1.12 ms with all
+// owned, 1.09 so).  Of other items only a wave's first is its own.
+constexpr uint32_t kOwnItems = 6;
+struct Claims {
+  uint32_t *word;    // LDS: the workgroup's items taken; its queue is empty
+  uint32_t per;      // its items
+  uint32_t queues, q;
+  uint32_t ahead;    // lane 0: what an early claim returned
+  bool first, own, asked, dry;
+  // all of the workgroup's threads; two words of LDS
+  NGAP_DEV void start(const KParams &P, uint32_t *lds) {
+    const uint32_t waves = P.waves_per_block, wgs = gridDim.x;
+    const uint64_t all = (uint64_t)waves * wgs;
+    per = P.num_tasks <= all * (P.even ? kOwnItems : 1)
+              ? (P.num_tasks + wgs - 1) / wgs
+              : P.even ? (uint32_t)((uint64_t)P.num_tasks * 3 / 4 / wgs) : waves;
+    word = lds;
+    if (threadIdx.x == 0) {
+      word[0] = waves;  // a wave's first item is its own
+      word[1] = 0;
+    }
+    __syncthreads();
+    queues = min_u(kQueues, wgs);
+    q = blockIdx.x % kQueues;
+    ahead = 0;
+    first = own = true;
+    asked = false;
+    dry = (uint64_t)per * wgs + q >= P.num_tasks;
   }
-  return P.num_tasks;
-}
+  // claims from the queue early
+  NGAP_DEV void ask(const KParams &P, const WaveState &W) {
+    if (asked | own | dry) return;
+    dry = from_first(word[1]) != 0;
+    if (dry) return;
+    if (W.lane == 0) ahead = atomicAdd(P.task_head + q * kQueueStride, 1u);
+    asked = true;
+  }
+  // the next work item, or P.num_tasks when there is none
+  NGAP_DEV uint32_t claim(const KParams &P, const WaveState &W) {
+    if (own) {
+      uint32_t i = W.wave;
+      if (!first) {
+        i = 0;
+        if (W.lane == 0) i = atomicAdd(word, 1u);
+        i = from_first(i);
+      }
+      first = false;
+      const uint64_t t = (uint64_t)i * gridDim.x + blockIdx.x;
+      if ((i < per) & (t < P.num_tasks)) return (uint32_t)t;
+      own = false;
+    }
+    ask(P, W);
+    if (!asked) return P.num_tasks;
+    asked = false;
+    const uint64_t t = (uint64_t)per * gridDim.x + (uint64_t)from_first(ahead) * queues + q;
+    if (t < P.num_tasks) return (uint32_t)t;
+    dry = true;
+    if (W.lane == 0) word[1] = 1;
+    return P.num_tasks;
+  }
+};
 
 // Batched schedule, engine runs: the wave's stream of work items.  A wave
 // starts the next work item as soon as the current one has no positions left
@@ -964,13 +1007,12 @@ struct TaskStream {
   uint64_t rbase = 0;       // root pass: the work item's first root item
   bool cross = false;
   bool cross_mask = false;  // LDS holds the cross-group report mask
-  uint32_t q = 0;           // the wave's queue
-  NGAP_DEV void start(const KParams &P, const WaveState &W) { q = blockIdx.x % kQueues; }
+  Claims claims;
   template <bool RootItems, bool Gen>
   NGAP_DEV int next(const KParams &P, WaveState &W, uint32_t &a, uint32_t &b) {
     if (cur >= end) {
       if (W.n_open >= kMaxOpen) return 1;
-      const uint32_t t = claim_task(P, W, q);
+      const uint32_t t = claims.claim(P, W);
       if (t >= P.num_tasks) return 2;
       const uint32_t ti = P.task_order ? P.task_order[t] : t;
       const Task T = Gen ? gen_task(P, ti) : P.tasks[ti];
@@ -1044,9 +1086,9 @@ NGAP_DEV void take_roots(const KParams &P, WaveState &W, uint64_t from, uint32_t
 // drain() over a TaskStream: items of several work items (and groups) share
 // the queue, so a lane looks up its item's group bases when it takes one.
 template <bool RootItems, int End, bool Gen>
-NGAP_DEV void drain_stream(const KParams &P, WaveState &W) {
+NGAP_DEV void drain_stream(const KParams &P, WaveState &W, uint32_t *word) {
   TaskStream src;
-  src.start(P, W);
+  src.claims.start(P, word);
   bool valid = false;
   uint32_t v = 0, p = 0;
   int depth = 0;
@@ -1357,11 +1399,11 @@ template <bool Gen>
 __global__ void __launch_bounds__(kBlockThreads) k_scan(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
   const uint32_t wave = from_first(threadIdx.x / kWave);
-  uint2 *bases = reinterpret_cast<uint2 *>(lds);
+  uint2 *bases = reinterpret_cast<uint2 *>(lds + 16);
   for (uint32_t g = threadIdx.x; g < P.num_groups; g += kBlockThreads)
     bases[g] = *reinterpret_cast<const uint2 *>(&P.img.meta[g]);
   WaveState W;
-  unsigned char *mine = lds + scan_table_bytes(P.num_groups) +
+  unsigned char *mine = lds + 16 + scan_table_bytes(P.num_groups) +
                         wave * scan_wave_bytes(P.ring_cap);
   setup_wave(W, mine, wave);
   W.ring = reinterpret_cast<uint64_t *>(mine + kScanFixed);
@@ -1372,9 +1414,10 @@ __global__ void __launch_bounds__(kBlockThreads) k_scan(KParams P) {
   S.n_keys = 0;
   W.open = reinterpret_cast<uint32_t *>(S.keys + kKeyCap);
   clear_dedup(P, W);
-  __syncthreads();
 
-  uint32_t q = blockIdx.x % kQueues, cur = 0, end = 0;
+  Claims claims;
+  claims.start(P, reinterpret_cast<uint32_t *>(lds));
+  uint32_t cur = 0, end = 0;
   bool more = true;
   ScanItem I = {};
   I.pos = kNoItem;
@@ -1399,7 +1442,7 @@ __global__ void __launch_bounds__(kBlockThreads) k_scan(KParams P) {
       }
       if (NGAP_SELDOM(cur >= end)) {
         const KParams &Q = cold_params();
-        const uint32_t t = claim_task(Q, W, q);
+        const uint32_t t = claims.claim(Q, W);
         if (t >= Q.num_tasks) {
           more = false;
           continue;
@@ -1416,6 +1459,8 @@ __global__ void __launch_bounds__(kBlockThreads) k_scan(KParams P) {
       const uint32_t stop = min_u(cur + 2 * kWave, end);
       find_keys(P, W, S, cur, stop);
       cur = stop;
+      // the next work item is claimed with one step of this one left
+      if (end - cur <= 2 * kWave) claims.ask(cold_params(), W);
       continue;
     }
     const uint64_t idle = wballot(I.pos == kNoItem);
@@ -1505,9 +1550,10 @@ __global__ void __launch_bounds__(kBlockThreads) k_batched(KParams P) {
   const uint32_t wbytes = wave_lds_bytes(P.ring_cap);
   WaveState W;
   setup_wave(W, lds + 16 + wave * wbytes, wave);
-  uint32_t q = blockIdx.x % kQueues;
+  Claims claims;
+  claims.start(P, reinterpret_cast<uint32_t *>(lds));
   for (;;) {
-    const uint32_t t = claim_task(P, W, q);
+    const uint32_t t = claims.claim(P, W);
     if (t >= P.num_tasks) break;
     const uint32_t ti = P.task_order ? P.task_order[t] : t;
     const Task T = P.tasks[ti];
@@ -1551,7 +1597,7 @@ __global__ void __launch_bounds__(kBlockThreads) k_batched_stream(KParams P) {
   WaveState W;
   setup_wave(W, lds + 16 + wave * wbytes, wave);
   clear_dedup(P, W);
-  drain_stream<false, End, Gen>(P, W);
+  drain_stream<false, End, Gen>(P, W, reinterpret_cast<uint32_t *>(lds));
   flush_reports(W);
   if (W.lane == 0) add_items(W.items);
 }
@@ -1565,7 +1611,7 @@ __global__ void __launch_bounds__(kBlockThreads) k_expand(KParams P) {
   WaveState W;
   setup_wave(W, lds + 16 + wave * wbytes, wave);
   clear_dedup(P, W);
-  drain_stream<true, kEndChunkLen, false>(P, W);
+  drain_stream<true, kEndChunkLen, false>(P, W, reinterpret_cast<uint32_t *>(lds));
   flush_reports(W);
   if (W.lane == 0) add_items(W.items);
 }
@@ -1736,7 +1782,7 @@ __global__ void k_reset(unsigned long long *report_count, unsigned long long *it
   if (i == 0) {
     if (!keep_reports) *report_count = 0;
     for (uint32_t k = 0; k < kItemLanes; k++) items[k * kItemStride] = 0;
-    for (uint32_t k = 0; k < 2 * kQueues; k++) task_head[k * kQueueStride] = 0;
+    for (uint32_t k = 0; k < kQueues; k++) task_head[k * kQueueStride] = 0;
     *overflow_count = 0;
   }
   for (; i < n_overflow; i += gridDim.x * blockDim.x) {

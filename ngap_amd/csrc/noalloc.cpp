@@ -89,12 +89,13 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     set_chunk_len(P, (uint32_t)chunk_len);
     P.num_seg = num_seg;
     // the schedule: all-group windows (depth >= 2) or one group per work item,
-    // windows of about two work items per wave, on a grid sized to the job
+    // windows as ngap_run's, on a grid sized to the job
     const uint32_t G = (uint32_t)eng->img.num_groups;
     P.gen_cross = mp.memo_depth >= 2 && o.cross_groups != 0;
     const uint64_t total = (uint64_t)num_seg * chunk_len;
     const uint64_t work = total * (P.gen_cross ? 1 : G);
     P.scan = P.gen_cross && scan_image(eng, mp, total);
+    P.even = P.gen_cross;
     P.load_last = (uint32_t)(total - std::min<uint64_t>(total, 8));
     const int kind = P.scan ? 6 : 4;  // of generated work items
     uint32_t blocks = 0;
@@ -103,7 +104,10 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     if (!o.persistent_blocks) blocks = job_blocks(blocks, P.waves_per_block, work);
     const uint64_t waves = (uint64_t)blocks * P.waves_per_block;
     uint32_t win = o.window;
-    if (!win) {
+    if (!win && P.gen_cross) {
+      win = cross_window(work, waves);
+      while (win < 65536 && (total / win + num_seg) * 4 > kScratchFlags) win *= 2;
+    } else if (!win) {
       win = 256;
       while (win < 65536 && (double)win * 1.41421356 < (double)work / (2.0 * waves)) win *= 2;
     }

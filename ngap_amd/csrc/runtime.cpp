@@ -167,7 +167,7 @@ uint32_t lds_bytes(uint32_t ring) {
 
 uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups) {
   if (kind < 5) return lds_bytes(ring);
-  return scan_table_bytes(groups) + (kBlockThreads / kWave) * scan_wave_bytes(ring);
+  return 16 + scan_table_bytes(groups) + (kBlockThreads / kWave) * scan_wave_bytes(ring);
 }
 
 // ring_capacity option -> LDS ring entries (0 = default); 0 when invalid
@@ -296,7 +296,9 @@ int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *bloc
     const_cast<ngap_engine *>(eng)->batched_per_cu[slot] = per_cu;
   }
   if (per_cu < 1) per_cu = 1;
-  *blocks = requested ? requested : (uint32_t)(per_cu * eng->num_cus);
+  // never more than can be resident: a wave's work items are partly its own
+  const uint32_t full = (uint32_t)(per_cu * eng->num_cus);
+  *blocks = requested ? std::min(requested, full) : full;
   return NGAP_OK;
 }
 
@@ -304,6 +306,16 @@ uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t wor
   const uint64_t per_block = kMinWavePositions * std::max<uint32_t>(1, waves_per_block);
   const uint64_t want = (work + per_block - 1) / per_block;
   return (uint32_t)std::min<uint64_t>(full_blocks, std::max<uint64_t>(64, want));
+}
+
+// Work-item length of all-group windows: four a wave, between two steps' worth
+// of positions and 1,024.  Fewer even out the waves' times too little (1,024
+// automata, 8 MiB: one a wave 0.207 ms, two 0.215, four 0.188), longer ones above
+// 4,096 positions a wave too (64 MiB: windows of 8,192 positions 1.35 ms, 4,096
+// 1.16, 1,024 1.09, 256 1.15); shorter ones cost their set-up.
+uint32_t cross_window(uint64_t positions, uint64_t waves) {
+  const uint64_t per = (positions + 4 * waves - 1) / std::max<uint64_t>(1, 4 * waves);
+  return (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(128, (per + 63) / 64 * 64));
 }
 
 // Root pass set-up for the resident work items: each work item's area of
@@ -622,7 +634,7 @@ std::vector<Task> static_schedule(const ngap_engine *eng, uint32_t window, bool 
 std::vector<Task> cross_schedule(const ngap_engine *eng, uint32_t window, bool is_dup,
                                  uint32_t waves) {
   const uint32_t S = eng->num_seg, L = (uint32_t)eng->chunk_len;
-  uint32_t win = window ? window : auto_window((uint64_t)S * L, waves);
+  uint32_t win = window ? window : cross_window((uint64_t)S * L, waves);
   if (win > L) win = L;
   std::vector<Task> tasks;
   for (uint32_t c = 0; c < S; c++)
@@ -1112,6 +1124,7 @@ int ngap_run(ngap_engine *eng, const ngap_run_opts *opts, ngap_run_stats *st) {
     for (uint32_t i = 0; kind == 0 && scan && i < o.num_tasks; i++)
       scan = o.tasks[i].group == NGAP_ALL_GROUPS;
     P.scan = scan;
+    P.even = kind == 1;
     P.load_last = (uint32_t)(total - std::min<uint64_t>(total, 8));
     // the default grid, sized to the job
     if (o.persistent_blocks == 0) {

@@ -265,10 +265,11 @@ int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *bloc
                       uint32_t ring = kRing, int kind = 1);
 // The default persistent grid for a job of `work` positions (summed over the
 // groups each work item scans): the full grid, or fewer workgroups when that
-// would leave a wave fewer than kMinWavePositions positions.  A small job on
-// the full grid spends its time on the waves' own set-up and claims
-// (literal64, 1 MiB: 0.079 ms on 384 workgroups against 0.132 on 1,280).
-constexpr uint64_t kMinWavePositions = 640;
+// would leave a wave fewer than kMinWavePositions positions, one search step of
+// k_scan (DNA literals: 1 MiB 0.026 ms on the full grid, 0.031 on 384 workgroups;
+// 64 KiB 0.017 on 128, 0.019 on 64).
+constexpr uint64_t kMinWavePositions = 128;
+uint32_t cross_window(uint64_t positions, uint64_t waves);
 uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t work);
 uint32_t ring_of(const ngap_run_opts &o);
 // Runs tasks on ctx (batched kernel), with the overflow fallback of o.

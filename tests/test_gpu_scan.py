@@ -55,3 +55,35 @@ def test_scan_edges(engine, chunk, shortest):
                     assert np.array_equal(got, want), (got.size, want.size)
             got, _ = run_noalloc(engine, opts, np.frombuffer(data, np.uint8), chunk)
             assert np.array_equal(got, want), (got.size, want.size)
+
+
+@pytest.mark.parametrize("blocks", [1, 3, 8, 9])  # below, at and above a queue an XCD
+def test_work_item_claims(engine, blocks):
+    # items a wave: below one, one, up to the last count that is all the
+    # workgroups' own (six), just above it and far above
+    r = random.Random(blocks)
+    groups = [chain_rules(r, 4, 3), chain_rules(r, 2, 2), fan_rules()]
+    chunk, chunks, waves = 997, 3, 4 * blocks
+    data = bytes(r.choice(ALPHA) for _ in range(chunk * chunks))
+    want, _ = oracle.run(groups, data, chunk, chunks)
+    for depth in (2, 3):
+        engine.load_groups(groups, max_precompute_depth=depth)
+        engine.set_input(data, chunk, chunks)
+        for items in (1, waves - 1, waves, waves + 1, 6 * waves - 1, 6 * waves, 6 * waves + 1,
+                      40 * waves):
+            window = max(1, -(-chunk // max(1, items // chunks)))
+            for cross in (0, 2):
+                print("[case] claims", blocks, depth, items, window, cross, flush=True)
+                opts = engine.options(schedule="batched", precompute_depth=depth,
+                                      cross_groups=cross, window=window,
+                                      persistent_blocks=blocks)
+                engine.run(opts)
+                assert np.array_equal(engine.reports(), want)
+                got, _ = run_noalloc(engine, opts, np.frombuffer(data, np.uint8), chunk)
+                assert np.array_equal(got, want)
+        # the program's own work items, of very different sizes
+        cuts = [0] + sorted(r.sample(range(1, chunk), 5 * waves)) + [chunk]
+        tasks = [(-1, c, a, b) for c in range(chunks) for a, b in zip(cuts, cuts[1:])]
+        engine.run(schedule="batched", precompute_depth=depth, tasks=tasks,
+                   persistent_blocks=blocks)
+        assert np.array_equal(engine.reports(), want)
