@@ -186,6 +186,32 @@ uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups);
 // ctx.sorted_on_host.
 hipError_t sort_reports_device(RunCtx &ctx, uint64_t n, uint32_t offset_bits);
 
+// What the device needs to set up a request launch (requests.hip): the requests
+// in the order of their bytes in the input, each with its first 16-byte unit, and
+// in the order of the work items, longest first, each with its first work item.
+struct RequestSpan {
+  const uint8_t *src;  // pinned, 16-byte aligned, readable to a multiple of 16
+  uint32_t base, len, group, first;
+};
+struct RequestTasks {
+  uint32_t first, request;
+};
+struct RequestBatch {
+  const RequestSpan *spans;
+  const RequestTasks *order;
+  uint32_t count, units, bytes, window, num_tasks, map_words;
+  uint8_t *input;
+  uint32_t *map;
+  Task *tasks;
+  uint32_t *overflow, *task_head;
+  unsigned long long *counters, *items;
+};
+hipError_t launch_gather(hipStream_t s, const RequestBatch &B);
+// counters[0..3] and the first min(count, cap, kSmallReports) reports, to pinned memory
+hipError_t launch_results(hipStream_t s, const unsigned long long *counters,
+                          const uint64_t *reports, uint64_t cap, unsigned long long *to_counters,
+                          uint64_t *to_reports);
+
 // Kernel launchers (kernels.hip).  launch_reset clears the run's counters
 // and n per-work-item flags (and root counts, when given); launch_roots runs
 // the root pass (k_roots) over P.pieces.

@@ -30,7 +30,7 @@ double now_ms() {
 }
 
 // Pinned host buffers for request bytes, reused by size class (a power of
-// two): the host-to-device copy of a launch is an asynchronous DMA from them.
+// two, 64 KiB at least): a launch's first kernel reads them.
 struct PinnedPool {
   std::multimap<size_t, uint8_t *> free_;
   std::vector<uint8_t *> all;
@@ -74,18 +74,18 @@ struct Slot {
   RunCtx ctx;
   DevBuf input;
   DevBuf last_map;              // bit per input byte: the last byte of a request
-  Task *task_host = nullptr;    // pinned staging of the work items (async upload)
-  size_t task_cap = 0;
-  uint32_t *map_host = nullptr; // pinned staging of last_map
-  size_t map_cap = 0;
+  DevBuf about;                 // the launch's requests (RequestSpan, RequestTasks)
+  uint8_t *about_host = nullptr;  // pinned staging of it
+  size_t about_cap = 0;
   ~Slot() {
-    if (task_host) (void)hipHostFree(task_host);
-    if (map_host) (void)hipHostFree(map_host);
+    if (about_host) (void)hipHostFree(about_host);
   }
   bool busy = false;
   std::vector<uint64_t> ids;
   std::vector<uint32_t> base;   // request start offsets in the slot input
-  std::vector<Task> tasks;
+  std::vector<RequestSpan> spans;
+  std::vector<RequestTasks> order;
+  uint32_t window = 0;
   uint64_t bytes = 0;           // HBM held while in flight
   KParams P;
   uint32_t blocks = 0;
@@ -98,6 +98,7 @@ struct Slot {
   void release() {
     input.release();
     last_map.release();
+    about.release();
     ctx.reports.release();
     ctx.spill.release();
     ctx.tasks.release();
@@ -223,7 +224,6 @@ bool fits_budget(ngap_server *s, Slot &sl, LaunchSize &z) {
 int launch_slot(ngap_server *s, Slot &sl) {
   sl.ids.clear();
   sl.base.clear();
-  sl.tasks.clear();
   const uint32_t wpb = kBlockThreads / kWave;
   const uint64_t waves = (uint64_t)s->blocks_per_launch * wpb;
   // continuous batching: a launch takes its share of what is queued (split
@@ -271,57 +271,49 @@ int launch_slot(ngap_server *s, Slot &sl) {
   }
   if (sl.ids.empty()) return NGAP_OK;
   const uint32_t win = serve_window(total, waves);
-  // last-byte map: bit p set when p is the last byte of its request (the
-  // streaming kernel's chunk-end test for items of any request)
-  const size_t map_words = total / 32 + 2;
-  if (sl.map_cap < map_words) {
-    if (sl.map_host) HIP_TRY(hipHostFree(sl.map_host));
-    sl.map_host = nullptr;
-    sl.map_cap = 0;
-    const size_t cap = std::max<size_t>(4096, map_words * 2);
-    HIP_TRY(hipHostMalloc((void **)&sl.map_host, cap * 4, hipHostMallocDefault));
-    sl.map_cap = cap;
+  // the requests, in the order of their bytes, and longest first: the order of
+  // the work items
+  const size_t n = sl.ids.size();
+  sl.window = win;
+  sl.spans.clear();
+  sl.order.clear();
+  uint32_t units = 0;
+  for (size_t i = 0; i < n; i++) {
+    const Request &r = s->reqs[sl.ids[i]];
+    sl.spans.push_back({r.data, sl.base[i], (uint32_t)r.len, (uint32_t)r.group, units});
+    sl.order.push_back({0, (uint32_t)i});
+    units += (uint32_t)((r.len + 15) / 16);
   }
-  memset(sl.map_host, 0, map_words * 4);
-  for (size_t i = 0; i < sl.ids.size(); i++) {
-    Request &r = s->reqs[sl.ids[i]];
-    const uint32_t cs = sl.base[i], ce = cs + (uint32_t)r.len;
-    sl.map_host[(ce - 1) >> 5] |= 1u << ((ce - 1) & 31);
-    for (uint32_t a = cs; a < ce; a += win) {
-      const uint32_t b = std::min<uint32_t>(a + win, ce);
-      sl.tasks.push_back({(uint32_t)r.group, cs, ce, a, b, a == cs ? kTaskSeedStart : 0u});
-    }
+  std::stable_sort(sl.order.begin(), sl.order.end(),
+                   [&](const RequestTasks &x, const RequestTasks &y) {
+                     return sl.spans[x.request].len > sl.spans[y.request].len;
+                   });
+  uint32_t ntasks = 0;
+  for (RequestTasks &q : sl.order) {
+    q.first = ntasks;
+    ntasks += (sl.spans[q.request].len - 1) / win + 1;
   }
   // the actual work items are no more than the admission bound: the launch
   // needs no more than what was admitted
-  LaunchSize z = launch_size(total, sl.tasks.size(), s->blocks_per_launch, wpb);
+  LaunchSize z = launch_size(total, ntasks, s->blocks_per_launch, wpb);
   z.blocks = std::min(z.blocks, adm_blocks);
   HIP_TRY(sl.input.reserve(z.input));
   HIP_TRY(sl.last_map.reserve(z.map));
-  for (size_t i = 0; i < sl.ids.size(); i++) {
-    Request &r = s->reqs[sl.ids[i]];
-    HIP_TRY(hipMemcpyAsync(sl.input.as<uint8_t>() + sl.base[i], r.data, r.len,
-                           hipMemcpyHostToDevice, sl.ctx.stream));
-    r.state = 1;
+  const size_t order_at = n * sizeof(RequestSpan), about = order_at + n * sizeof(RequestTasks);
+  if (sl.about_cap < about) {
+    if (sl.about_host) HIP_TRY(hipHostFree(sl.about_host));
+    sl.about_host = nullptr;
+    sl.about_cap = 0;
+    const size_t cap = std::max<size_t>(16384, about * 2);
+    HIP_TRY(hipHostMalloc((void **)&sl.about_host, cap, hipHostMallocDefault));
+    sl.about_cap = cap;
   }
-  HIP_TRY(hipMemcpyAsync(sl.last_map.p, sl.map_host, map_words * 4, hipMemcpyHostToDevice,
-                         sl.ctx.stream));
-  // longest requests first inside the launch
-  std::stable_sort(sl.tasks.begin(), sl.tasks.end(), [](const Task &x, const Task &y) {
-    return (x.cend - x.cstart) > (y.cend - y.cstart);
-  });
-  if (sl.task_cap < sl.tasks.size()) {
-    if (sl.task_host) HIP_TRY(hipHostFree(sl.task_host));
-    sl.task_host = nullptr;
-    sl.task_cap = 0;
-    const size_t cap = std::max<size_t>(4096, sl.tasks.size() * 2);
-    HIP_TRY(hipHostMalloc((void **)&sl.task_host, cap * sizeof(Task), hipHostMallocDefault));
-    sl.task_cap = cap;
-  }
-  std::copy(sl.tasks.begin(), sl.tasks.end(), sl.task_host);
+  HIP_TRY(sl.about.reserve(sl.about_cap));
+  memcpy(sl.about_host, sl.spans.data(), order_at);
+  memcpy(sl.about_host + order_at, sl.order.data(), about - order_at);
+  HIP_TRY(hipMemcpyAsync(sl.about.p, sl.about_host, about, hipMemcpyHostToDevice, sl.ctx.stream));
+  for (uint64_t id : sl.ids) s->reqs[id].state = 1;
   HIP_TRY(sl.ctx.tasks.reserve(z.tasks));
-  HIP_TRY(hipMemcpyAsync(sl.ctx.tasks.p, sl.task_host, sl.tasks.size() * sizeof(Task),
-                         hipMemcpyHostToDevice, sl.ctx.stream));
   sl.ctx.tasks_resident = false;
   HIP_TRY(sl.ctx.overflow.reserve(z.overflow));
   HIP_TRY(sl.ctx.reports.reserve(z.reports));
@@ -333,7 +325,7 @@ int launch_slot(ngap_server *s, Slot &sl) {
   P.num_seg = 0;
   P.last_map = sl.last_map.as<uint32_t>();
   P.tasks = sl.ctx.tasks.as<Task>();
-  P.num_tasks = (uint32_t)sl.tasks.size();
+  P.num_tasks = ntasks;
   P.overflow = sl.ctx.overflow.as<uint32_t>();
   P.spill = sl.ctx.spill.as<uint64_t>();
   P.spill_cap = kServeSpill;
@@ -342,13 +334,28 @@ int launch_slot(ngap_server *s, Slot &sl) {
   // a small launch takes only the workgroups its work items can feed, so
   // short requests do not pay for a full persistent grid
   sl.blocks = z.blocks;
-  HIP_TRY(launch_reset(sl.ctx.stream, P.report_count, P.items, P.task_head, P.overflow,
-                       P.num_tasks, P.overflow_count, 0, nullptr));
+  RequestBatch B;
+  B.spans = sl.about.as<RequestSpan>();
+  B.order = reinterpret_cast<const RequestTasks *>(sl.about.as<uint8_t>() + order_at);
+  B.count = (uint32_t)n;
+  B.units = units;
+  B.bytes = (uint32_t)total;
+  B.window = win;
+  B.num_tasks = ntasks;
+  B.map_words = (uint32_t)(total / 32 + 2);
+  B.input = sl.input.as<uint8_t>();
+  B.map = sl.last_map.as<uint32_t>();
+  B.tasks = sl.ctx.tasks.as<Task>();
+  B.overflow = P.overflow;
+  B.task_head = P.task_head;
+  B.counters = P.report_count;
+  B.items = P.items;
+  HIP_TRY(launch_gather(sl.ctx.stream, B));
   HIP_TRY(launch_batched(sl.ctx.stream, P, sl.blocks, lds_bytes(P.ring_cap)));
-  // the counters follow the launch into pinned memory: retiring reads them
-  // without another copy
-  HIP_TRY(hipMemcpyAsync(sl.ctx.host_cnt, sl.ctx.counters.p, 32, hipMemcpyDeviceToHost,
-                         sl.ctx.stream));
+  // the counters and the first reports follow the launch into pinned memory:
+  // retiring reads them without another copy
+  HIP_TRY(launch_results(sl.ctx.stream, P.report_count, P.reports, P.report_cap,
+                         sl.ctx.host_cnt, sl.ctx.host_reports));
   HIP_TRY(hipEventRecord(sl.ctx.ev1, sl.ctx.stream));
   sl.bytes = z.total();
   s->inflight_bytes += sl.bytes;
@@ -384,7 +391,16 @@ int retire_slot(ngap_server *s, Slot &sl) {
       sl.ctx.report_cap = cnt + 1;
     }
     s->redone++;
-    int rc = run_tasks(s->eng, sl.ctx, P, sl.tasks, 0, o, nullptr);
+    std::vector<Task> tasks;
+    tasks.reserve(P.num_tasks);
+    for (const RequestTasks &q : sl.order) {
+      const RequestSpan &x = sl.spans[q.request];
+      const uint32_t end = x.base + x.len;
+      for (uint32_t a = x.base; a < end; a += sl.window)
+        tasks.push_back({x.group, x.base, end, a, std::min(a + sl.window, end),
+                         a == x.base ? kTaskSeedStart : 0u});
+    }
+    int rc = run_tasks(s->eng, sl.ctx, P, tasks, 0, o, nullptr);
     s->peak_held = std::max(s->peak_held, s->held());
     if (rc) {
       for (uint64_t id : sl.ids) fail_request(s, s->reqs[id]);
@@ -396,8 +412,13 @@ int retire_slot(ngap_server *s, Slot &sl) {
     sl.ctx.last_count = cnt;
   }
   std::vector<uint64_t> v;
-  int rc = sorted_reports(sl.ctx, v);
-  if (rc) return rc;
+  if (!redo && cnt <= kSmallReports) {
+    v.assign(sl.ctx.host_reports, sl.ctx.host_reports + cnt);
+    std::sort(v.begin(), v.end());
+    v.erase(std::unique(v.begin(), v.end()), v.end());
+  } else if (const int rc = sorted_reports(sl.ctx, v)) {
+    return rc;
+  }
   // split by request: device reports are (offset << 32) | id, offsets global
   // in the slot input; requests are contiguous and sorted by base
   std::vector<size_t> order(sl.ids.size());
