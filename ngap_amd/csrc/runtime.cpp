@@ -145,11 +145,24 @@ int RunCtx::init() {
 
 int RunCtx::finish(float *ms, unsigned long long cnt[4], bool record_end) {
   if (record_end) HIP_TRY(hipEventRecord(ev1, stream));
-  HIP_TRY(hipMemcpyAsync(host_cnt, counters.p, kCounterBytes, hipMemcpyDeviceToHost, stream));
+  HIP_TRY(launch_finish(stream, counters.as<unsigned long long>(), host_cnt));
   HIP_TRY(hipStreamSynchronize(stream));
   HIP_TRY(hipEventElapsedTime(ms, ev0, ev1));
   memcpy(cnt, host_cnt, 32);
-  cnt[1] = items_sum(host_cnt);
+  counters_zero = (uint32_t)cnt[3] == 0;
+  return NGAP_OK;
+}
+
+int RunCtx::begin(const KParams &P, uint32_t n, bool keep_reports) {
+  const bool zero = counters_zero && !keep_reports && !P.root_count && zero_flags == overflow.p &&
+                    zero_cap == overflow.n && n <= zero_n;
+  counters_zero = false;
+  if (zero) return NGAP_OK;
+  HIP_TRY(launch_reset(stream, P.report_count, P.items, P.task_head, P.overflow, n,
+                       P.overflow_count, keep_reports, P.root_count));
+  zero_flags = overflow.p;
+  zero_cap = overflow.n;
+  zero_n = n;
   return NGAP_OK;
 }
 
@@ -373,8 +386,7 @@ static int launch_batched_ctx(RunCtx &ctx, const KParams &P, uint32_t blocks, ui
                               hipEvent_t end) {
   const uint32_t lds = batched_lds(P.ring_cap, batched_kind(P), P.num_groups);
   const uint32_t root_lds = lds_bytes(P.ring_cap);
-  HIP_TRY(launch_reset(ctx.stream, P.report_count, P.items, P.task_head, P.overflow, n_flags,
-                       P.overflow_count, keep_reports, P.root_count));
+  if (const int rc = ctx.begin(P, n_flags, keep_reports)) return rc;
   if (use_graph) {
     std::vector<unsigned char> key(sizeof P + 4);
     memcpy(key.data(), &P, sizeof P);
@@ -733,8 +745,7 @@ int run_plain(ngap_engine *eng, RunCtx &ctx, KParams P, const ngap_run_opts &o,
   HIP_TRY(ctx.overflow.reserve((size_t)units * 4));
   P.overflow = ctx.overflow.as<uint32_t>();
   attach_ctx(P, ctx);
-  HIP_TRY(launch_reset(ctx.stream, P.report_count, P.items, P.task_head, P.overflow, units,
-                       P.overflow_count, 0, nullptr));
+  if (const int rc = ctx.begin(P, units, false)) return rc;
   HIP_TRY(hipEventRecord(ctx.ev0, ctx.stream));  // times the matching kernel alone
   if (blocking) HIP_TRY(launch_blocking(ctx.stream, P, units, lds_bytes()));
   else HIP_TRY(launch_plain(ctx.stream, P, units, lds_bytes()));

@@ -162,8 +162,16 @@ struct RunCtx {
   ~RunCtx();
   int init();
   void drop_graph();
+  // Whether the counters and the first n words of `overflow` are known to be
+  // zero: the last finish() on them left them so.  Each launch takes it back.
+  bool counters_zero = false;
+  const void *zero_flags = nullptr;
+  size_t zero_cap = 0;
+  uint32_t zero_n = 0;
+  // Clears P's counters and n flags on the stream, where they are not zero yet.
+  int begin(const KParams &P, uint32_t n, bool keep_reports);
   // Ends a timed launch begun with ev0: records ev1 (unless the launch
-  // recorded it), queues the copy of the run counters into host_cnt behind
+  // recorded it), queues k_finish (the run counters into host_cnt) behind
   // it and waits for the stream once.  *ms = ev0..ev1; cnt = reports, items
   // (the lanes summed), -, overflowed units.
   int finish(float *ms, unsigned long long cnt[4], bool record_end);
@@ -218,6 +226,7 @@ hipError_t launch_results(hipStream_t s, const unsigned long long *counters,
 hipError_t launch_reset(hipStream_t s, unsigned long long *rc, unsigned long long *items,
                         uint32_t *head, uint32_t *ovf, uint32_t n, uint32_t *ovf_count,
                         int keep_reports, unsigned long long *root_count);
+hipError_t launch_finish(hipStream_t s, unsigned long long *counters, unsigned long long *to);
 hipError_t launch_plain(hipStream_t s, const KParams &P, uint32_t units, uint32_t lds);
 hipError_t launch_blocking(hipStream_t s, const KParams &P, uint32_t units, uint32_t lds);
 hipError_t launch_roots(hipStream_t s, const KParams &P, uint32_t lds);

@@ -350,6 +350,7 @@ int launch_slot(ngap_server *s, Slot &sl) {
   B.task_head = P.task_head;
   B.counters = P.report_count;
   B.items = P.items;
+  sl.ctx.counters_zero = false;
   HIP_TRY(launch_gather(sl.ctx.stream, B));
   HIP_TRY(launch_batched(sl.ctx.stream, P, sl.blocks, lds_bytes(P.ring_cap)));
   // the counters and the first reports follow the launch into pinned memory:

@@ -334,3 +334,31 @@ def test_server_rejects_report_off(engine):
     engine.load_groups(groups, 2)
     with pytest.raises(NgapError):
         Server(engine, report_off=True, algorithm="nonblockingallgroups", precompute_depth=2)
+
+
+@pytest.mark.parametrize("schedule", ["plain", "batched"])
+def test_counters_between_runs(engine, schedule):
+    # a run leaves its counters and flags at zero for the next one, whatever ran
+    # before: more and fewer work items, an overflow, a fallback, a root pass
+    g = synth.regex_group(np.random.default_rng(3), 3000, dotstar=True)
+    data = synth.zipf_bytes(np.random.default_rng(4), 1 << 16, 0.8)
+    want, _ = oracle.run([g], data, 1 << 12)
+    engine.load_groups([g], 3)
+    engine.set_input(data, 1 << 12)
+    first = {}
+    steps = [dict(), dict(window=100), dict(), dict(spill_capacity=64, ring_capacity=64, over=True),
+             dict(), dict(spill_capacity=64, ring_capacity=64, fallback=True), dict(window=100),
+             dict(root_pass=True), dict(), dict(is_dup=False, precompute_depth=2), dict()]
+    for k, kw in enumerate(steps):
+        kw = dict(dict(precompute_depth=3), **kw)
+        over = kw.pop("over", False)
+        say("counters", schedule, k, kw)
+        try:
+            st = engine.run(algorithm="nonblockinggroups", schedule=schedule, **kw)
+        except NgapError as e:
+            assert over and e.code == 4
+            continue
+        assert np.array_equal(engine.reports(), want)
+        key = tuple(sorted(kw.items()))
+        raw, items = first.setdefault(key, (st["reports_raw"], st["items"]))
+        assert st["reports_raw"] == raw and st["items"] == items
