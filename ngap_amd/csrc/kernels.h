@@ -127,6 +127,7 @@ constexpr uint32_t kRbuf = 128, kDc = 256;
 // its own 128-byte line.
 constexpr uint32_t kQueues = 8, kQueueStride = 32;
 constexpr uint32_t kBlockThreads = 256;
+constexpr uint32_t kPlainWaves = 16;  // of a unit in k_plain, at most
 // Counters of a run (one buffer per run context, cleared by k_reset): bytes
 // 0-31 hold the report count and the count of overflowed work items (word
 // 3), byte 128 on the queue claim counters, then kItemLanes lines of

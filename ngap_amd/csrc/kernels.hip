@@ -1519,7 +1519,8 @@ struct LocalCursor {
   }
 };
 
-__global__ void __launch_bounds__(kBlockThreads) k_plain(KParams P) {
+// A unit's waves share its cursor, so their number is free (run_plain).
+__global__ void __launch_bounds__(kPlainWaves * kWave) k_plain(KParams P) {
   extern __shared__ __align__(16) unsigned char lds[];
   const uint32_t wave = from_first(threadIdx.x / kWave);
   const uint32_t unit = blockIdx.x;
@@ -1835,7 +1836,7 @@ hipError_t launch_reset(hipStream_t s, unsigned long long *rc, unsigned long lon
 }
 
 hipError_t launch_plain(hipStream_t s, const KParams &P, uint32_t units, uint32_t lds) {
-  hipLaunchKernelGGL(k_plain, dim3(units), dim3(kBlockThreads), lds, s, P);
+  hipLaunchKernelGGL(k_plain, dim3(units), dim3(P.waves_per_block * kWave), lds, s, P);
   return hipGetLastError();
 }
 
