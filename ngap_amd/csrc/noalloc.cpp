@@ -101,7 +101,15 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     uint32_t blocks = 0;
     int rc = persistent_blocks(eng, o.persistent_blocks, &blocks, P.ring_cap, kind);
     if (rc) return rc;
-    if (!o.persistent_blocks) blocks = job_blocks(blocks, P.waves_per_block, work);
+    // a grid as asked for has to leave each wave a worklist
+    if (o.persistent_blocks &&
+        kScratchSpill / ((uint64_t)o.persistent_blocks * P.waves_per_block * 8) < kWave)
+      return ngap_fail(NGAP_ERR_INVALID, "grid too large for the scratch array's worklists");
+    uint32_t fewer = blocks;  // the grid that gives each wave a larger worklist
+    if (!o.persistent_blocks) {
+      fewer = job_blocks(blocks, P.waves_per_block, work, kSpillPositions);
+      blocks = job_blocks(blocks, P.waves_per_block, work);
+    }
     const uint64_t waves = (uint64_t)blocks * P.waves_per_block;
     uint32_t win = o.window;
     if (!win && P.gen_cross) {
@@ -123,12 +131,6 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     P.tasks = nullptr;
     P.num_tasks = (uint32_t)T;
     P.task_items = nullptr;
-    // spill areas: what the scratch array holds for this grid, at most the
-    // requested capacity
-    const uint64_t fit = kScratchSpill / (waves * 8);
-    if (fit < kWave)
-      return ngap_fail(NGAP_ERR_INVALID, "grid too large for the scratch array's worklists");
-    P.spill_cap = (uint32_t)std::min<uint64_t>(o.spill_capacity ? o.spill_capacity : fit, fit);
     unsigned char *base = static_cast<unsigned char *>(eng->scratch);
     unsigned long long *counters = reinterpret_cast<unsigned long long *>(base);
     P.report_count = counters + 0;
@@ -140,19 +142,32 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     P.reports = d_reports;
     P.report_cap = report_cap;
     RunCtx &ctx = eng->ctx;
-    HIP_TRY(launch_reset(ctx.stream, P.report_count, P.items, P.task_head, P.overflow,
-                         P.num_tasks, P.overflow_count, 0, nullptr));
-    HIP_TRY(hipEventRecord(ctx.ev0, ctx.stream));
-    HIP_TRY(launch_batched(ctx.stream, P, blocks, batched_lds(P.ring_cap, kind, G)));
-    HIP_TRY(hipEventRecord(ctx.ev1, ctx.stream));
-    HIP_TRY(hipMemcpyAsync(ctx.host_cnt, counters, kCounterBytes, hipMemcpyDeviceToHost,
-                           ctx.stream));
-    HIP_TRY(hipStreamSynchronize(ctx.stream));
-    float ms = 0;
-    HIP_TRY(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
+    float ms = 0, all_ms = 0;
     unsigned long long cnt[4];
-    memcpy(cnt, ctx.host_cnt, 32);
-    cnt[1] = items_sum(ctx.host_cnt);
+    for (;;) {
+      // spill areas: what the scratch array holds for this grid, at most the
+      // requested capacity
+      const uint64_t fit = kScratchSpill / ((uint64_t)blocks * P.waves_per_block * 8);
+      if (fit < kWave)
+        return ngap_fail(NGAP_ERR_INVALID, "grid too large for the scratch array's worklists");
+      P.spill_cap = (uint32_t)std::min<uint64_t>(o.spill_capacity ? o.spill_capacity : fit, fit);
+      HIP_TRY(launch_reset(ctx.stream, P.report_count, P.items, P.task_head, P.overflow,
+                           P.num_tasks, P.overflow_count, 0, nullptr));
+      HIP_TRY(hipEventRecord(ctx.ev0, ctx.stream));
+      HIP_TRY(launch_batched(ctx.stream, P, blocks, batched_lds(P.ring_cap, kind, G)));
+      HIP_TRY(hipEventRecord(ctx.ev1, ctx.stream));
+      HIP_TRY(hipMemcpyAsync(ctx.host_cnt, counters, kCounterBytes, hipMemcpyDeviceToHost,
+                             ctx.stream));
+      HIP_TRY(hipStreamSynchronize(ctx.stream));
+      HIP_TRY(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
+      all_ms += ms;
+      memcpy(cnt, ctx.host_cnt, 32);
+      cnt[1] = items_sum(ctx.host_cnt);
+      // what a worklist of the larger grid could not hold, the smaller grid's may
+      if ((uint32_t)cnt[3] == 0 || blocks <= fewer) break;
+      blocks = fewer;
+    }
+    ms = all_ms;
     if (st) {
       st->kernel_ms = ms;
       st->reports_raw = cnt[0];

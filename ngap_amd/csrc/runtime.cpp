@@ -315,8 +315,9 @@ int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *bloc
   return NGAP_OK;
 }
 
-uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t work) {
-  const uint64_t per_block = kMinWavePositions * std::max<uint32_t>(1, waves_per_block);
+uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t work,
+                    uint64_t per_wave) {
+  const uint64_t per_block = per_wave * std::max<uint32_t>(1, waves_per_block);
   const uint64_t want = (work + per_block - 1) / per_block;
   return (uint32_t)std::min<uint64_t>(full_blocks, std::max<uint64_t>(64, want));
 }
@@ -466,17 +467,27 @@ int run_tasks(ngap_engine *eng, RunCtx &ctx, KParams P, const std::vector<Task> 
   // root pass), the others the per-work-item kernel (launch_batched)
   rc = persistent_blocks(eng, o.persistent_blocks, &blocks, P.ring_cap, batched_kind(P));
   if (rc) return rc;
-  P.spill_cap = o.spill_capacity ? o.spill_capacity : 65536;
-  HIP_TRY(ctx.spill.reserve((size_t)blocks * P.waves_per_block * P.spill_cap * 8));
-  P.spill = ctx.spill.as<uint64_t>();
-  attach_ctx(P, ctx);
-
-  rc = launch_batched_ctx(ctx, P, blocks, T, false, o.use_graph != 0, ctx.ev0, ctx.ev1);
-  if (rc) return rc;
-  float ms = 0;
+  // default worklists: 64K items a wave, less where a small job takes more waves
+  // than its positions fill (ngap_run); what those cannot hold is run again with
+  // the former, and so is this context's next run
+  const uint32_t most = o.spill_capacity ? o.spill_capacity : 65536;
+  if (o.spill_capacity || !P.spill_cap || P.root_items || ctx.spill_most) P.spill_cap = most;
+  float ms = 0, all_ms = 0;
   unsigned long long cnt[4] = {0, 0, 0, 0};
-  rc = ctx.finish(&ms, cnt, false);
-  if (rc) return rc;
+  for (;;) {
+    HIP_TRY(ctx.spill.reserve((size_t)blocks * P.waves_per_block * P.spill_cap * 8));
+    P.spill = ctx.spill.as<uint64_t>();
+    attach_ctx(P, ctx);
+    rc = launch_batched_ctx(ctx, P, blocks, T, false, o.use_graph != 0, ctx.ev0, ctx.ev1);
+    if (rc) return rc;
+    rc = ctx.finish(&ms, cnt, false);
+    if (rc) return rc;
+    all_ms += ms;
+    if ((uint32_t)cnt[3] == 0 || P.spill_cap >= most) break;
+    P.spill_cap = most;
+    ctx.spill_most = true;
+  }
+  ms = all_ms;
   std::vector<uint32_t> bad;
   bool spill_over = false;  // some work item lost items (not only its root area)
   if ((uint32_t)cnt[3] && T) {  // per-item flags only when some work item overflowed
@@ -1172,6 +1183,8 @@ int ngap_run(ngap_engine *eng, const ngap_run_opts *opts, ngap_run_stats *st) {
         work = total * (kind == 2 ? eng->img.num_groups : 1);
       }
       o.persistent_blocks = job_blocks(full, P.waves_per_block, work);
+      P.spill_cap = (uint32_t)(65536ull * job_blocks(full, P.waves_per_block, work, kSpillPositions) /
+                               o.persistent_blocks);
     }
     uint32_t waves = 0;
     if (kind != 0) {

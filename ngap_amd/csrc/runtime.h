@@ -137,6 +137,7 @@ struct RunCtx {
   // offsets (items), the areas and the per-work-item counts
   DevBuf pieces, root_off, root_items, root_count;
   uint32_t num_pieces = 0;
+  bool spill_most = false;      // a smaller worklist than the default overflowed
   uint32_t root_factor = 0;     // items per position the resident areas were sized for
   uint32_t root_boost = 1;      // doubles (up to 64x) after a root area overflowed,
   uint64_t root_gen = 0;        // for this engine generation (groups and input)
@@ -305,7 +306,13 @@ int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *bloc
 // 64 KiB 0.017 on 128, 0.019 on 64).
 constexpr uint64_t kMinWavePositions = 128;
 uint32_t cross_window(uint64_t positions, uint64_t waves);
-uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t work);
+uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t work,
+                    uint64_t per_wave = kMinWavePositions);
+// Positions for which a wave's default worklist (64K items) was sized: a job on
+// more waves than one per so many has smaller ones, so that the grids of small
+// jobs cost no more memory (1 MiB of DNA, the first run of an engine 0.69 ms with
+// 2 GiB to allocate, 0.39 so).
+constexpr uint64_t kSpillPositions = 640;
 uint32_t ring_of(const ngap_run_opts &o);
 // Runs tasks on ctx (batched kernel), with the overflow fallback of o.
 int run_tasks(ngap_engine *eng, RunCtx &ctx, KParams P, const std::vector<Task> &tasks,

@@ -42,3 +42,20 @@ def test_plain_backlog_of_one_wave(engine):
     st = engine.run(algorithm="nonblockinggroups", schedule="plain")
     assert st["reports_raw"] == n and st["overflow_units"] == 0
     assert [int(x) for x in engine.reports()] == [((n + 1) << 32) | 4]
+
+
+def test_batched_backlog_of_one_wave(engine):
+    # the same on the batched schedule, whose small jobs have smaller worklists
+    n = 40000
+    g = make_group(n + 2, [(0, 1 + i) for i in range(n)] + [(1 + i, n + 1) for i in range(n)],
+                   [[97]] + [[98]] * n + [[99]], all_input=[0], reporting=[n + 1])
+    data = b"x" * 150000 + b"abc" + b"x" * 50000
+    for depth in (1, 2, 3):
+        engine.load_groups([g], depth)
+        engine.set_input(data, len(data))
+        print("[case] batched backlog", depth, flush=True)
+        for _ in range(2):
+            st = engine.run(algorithm="nonblockinggroups", schedule="batched",
+                            precompute_depth=depth)
+            assert st["reports_raw"] == n and st["overflow_units"] == 0
+            assert [int(x) for x in engine.reports()] == [((n + 1) << 32) | 150002]
