@@ -12,7 +12,9 @@
 //    one launch.  Equal keys get the same place, which leaves the repeats'
 //    slots empty: the second launch closes the gaps, swaps the halves and
 //    writes the result straight to pinned host memory.
-//  * Above: rocPRIM's radix sort and unique, in place in the report buffer.
+//  * Above: rocPRIM's radix sort and unique, in place in the report buffer
+//    (reports_large.hip, a module of its own: a process's first use of rocPRIM's
+//    kernels loads them, 4 ms that few reports need not wait for).
 // The line between them: two ngap_get_reports calls (count, then copy) over
 // 2,048 reports take 25 us, over 4,096 31, 8,192 44, 16,384 70 by rank; 16,385
 // by radix (10 launches, the copy by hipMemcpy) 141, 131,072 558.  One 1,024-
@@ -22,11 +24,6 @@
 // 154,507 (207 now).  The rank kernel is bound by its 64-bit comparisons: 14k
 // keys in 59 us with a scalar load per key, 39 with one per eight.
 #include <hip/hip_runtime.h>
-
-#include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_select.hpp>
-
-#include <algorithm>
 
 #include "runtime.h"
 
@@ -107,47 +104,10 @@ __global__ void __launch_bounds__(kSortThreads)
   if (threadIdx.x == kSortThreads - 1) out[0] = before + total;
 }
 
-__global__ void k_encode(uint64_t *keys, const uint64_t *count) {
-  const uint64_t n = *count;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    keys[i] = encode(keys[i]);
-}
-
-// The radix path: reports[0, n) -> sorted, unique, encoded in place.
-// hipErrorOutOfMemory when its work area cannot be allocated.
-hipError_t sort_large(RunCtx &ctx, uint64_t n, uint32_t bits) {
-  uint64_t *keys = ctx.reports.as<uint64_t>();
-  size_t sort_bytes = 0, uniq_bytes = 0;
-  hipError_t e = rocprim::radix_sort_keys(nullptr, sort_bytes, keys, keys, n, 0, bits, ctx.stream);
-  if (e != hipSuccess) return e;
-  e = rocprim::unique(nullptr, uniq_bytes, keys, keys, keys, n, rocprim::equal_to<uint64_t>(),
-                      ctx.stream);
-  if (e != hipSuccess) return e;
-  const size_t tmp = (std::max(sort_bytes, uniq_bytes) + 255) / 256 * 256;
-  if ((e = ctx.sort_area.reserve(tmp + n * 8 + 8)) != hipSuccess) return e;
-  uint64_t *sorted = reinterpret_cast<uint64_t *>(ctx.sort_area.as<char>() + tmp);
-  uint64_t *kept = sorted + n;
-  e = rocprim::radix_sort_keys(ctx.sort_area.p, sort_bytes, keys, sorted, n, 0, bits, ctx.stream);
-  if (e != hipSuccess) return e;
-  e = rocprim::unique(ctx.sort_area.p, uniq_bytes, sorted, keys, kept, n,
-                      rocprim::equal_to<uint64_t>(), ctx.stream);
-  if (e != hipSuccess) return e;
-  const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + 255) / 256, 2048);
-  hipLaunchKernelGGL(k_encode, dim3(blocks), dim3(256), 0, ctx.stream, keys, kept);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = hipMemcpyAsync(ctx.host_reports, kept, 8, hipMemcpyDeviceToHost, ctx.stream)) !=
-      hipSuccess)
-    return e;
-  if ((e = hipStreamSynchronize(ctx.stream)) == hipSuccess)
-    ctx.unique_reports = ctx.host_reports[0];
-  return e;
-}
-
 }  // namespace
 
 hipError_t sort_reports_device(RunCtx &ctx, uint64_t n, uint32_t offset_bits) {
-  if (n > kSmallReports) return sort_large(ctx, n, 32 + offset_bits);
+  if (n > kSmallReports) return sort_reports_large(ctx, n, 32 + offset_bits);
   hipLaunchKernelGGL(k_rank_reports, dim3(((uint32_t)n + kWave - 1) / kWave), dim3(kSortThreads),
                      0, ctx.stream, ctx.reports.as<uint64_t>(), (uint32_t)n,
                      ctx.report_slots);

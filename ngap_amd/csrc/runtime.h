@@ -194,6 +194,7 @@ uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups);
 // else in place in ctx.reports.  Sets ctx.unique_reports and
 // ctx.sorted_on_host.
 hipError_t sort_reports_device(RunCtx &ctx, uint64_t n, uint32_t offset_bits);
+hipError_t sort_reports_large(RunCtx &ctx, uint64_t n, uint32_t bits);
 
 // What the device needs to set up a request launch (requests.hip): the requests
 // in the order of their bytes in the input, each with its first 16-byte unit, and
