@@ -49,6 +49,17 @@ constexpr uint64_t kKeyStateMask = (1ull << 22) - 1;
 // device error flags (bits)
 constexpr uint32_t kErrRowOrder = 1, kErrColRange = 2, kErrAasRange = 4, kErrSodRange = 8;
 
+// Bits that hold every value up to n (so that no value below n is all ones: the
+// sentinel stays the largest key).  A sort takes a pass per 8 bits of its keys:
+// with the bits that can differ, and lists, whose indices come in order, by their
+// d-gram alone, a load of 128 automata of up to 50,000 states takes 5.13 ms, with
+// all bits 5.4.
+inline int bits_of(uint64_t n) {
+  int b = 1;
+  while (b < 64 && (n >> b)) b++;
+  return b;
+}
+
 inline uint32_t grid_for(uint64_t n) {
   uint64_t b = (n + kThreads - 1) / kThreads;
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(b, 1u << 20));
@@ -508,13 +519,14 @@ struct Prim {
   hipStream_t s;
   DevBuf tmp;
   Prim(hipStream_t stream, Slab &slab) : s(stream), tmp(slab) {}
-  hipError_t sort(const uint64_t *in, uint64_t *out, uint64_t n, int bits) {
+  // by the bits [from, to) (a stable sort: keys in order by the bits below stay so)
+  hipError_t sort(const uint64_t *in, uint64_t *out, uint64_t n, int from, int to) {
     if (n == 0) return hipSuccess;
     size_t bytes = 0;
-    hipError_t e = rocprim::radix_sort_keys(nullptr, bytes, in, out, n, 0, bits, s);
+    hipError_t e = rocprim::radix_sort_keys(nullptr, bytes, in, out, n, from, to, s);
     if (e != hipSuccess) return e;
     if ((e = tmp.reserve(bytes)) != hipSuccess) return e;
-    return rocprim::radix_sort_keys(tmp.p, bytes, in, out, n, 0, bits, s);
+    return rocprim::radix_sort_keys(tmp.p, bytes, in, out, n, from, to, s);
   }
   // out[i] = in[0] + ... + in[i-1], n + 1 entries (out[n] = total; in[n] is
   // read, whatever it holds)
@@ -731,7 +743,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     err = "CSR column index out of range";
     return NGAP_ERR_INVALID;
   }
-  HIP_TRY(prim.sort(d_ekeys.as<uint64_t>(), d_esorted.as<uint64_t>(), E, 64));
+  HIP_TRY(prim.sort(d_ekeys.as<uint64_t>(), d_esorted.as<uint64_t>(), E, 0, 22 + bits_of(N)));
   uint64_t D = 0;
   HIP_TRY(d_dkeys.reserve(E * 8 + 8));
   HIP_TRY(prim.unique(d_esorted.as<uint64_t>(), d_dkeys.as<uint64_t>(), E, &D, d_cnt8));
@@ -818,6 +830,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
   sz.meta = (uint64_t)G * sizeof(GroupMeta);
 
   // memo level 1
+  const int key_bits = kKeyGroupShift + bits_of((uint64_t)G);
   static_assert(kMaxMemoDepth == 3, "one buffer a level");
   DevBuf d_cnt(slab), d_off(slab), d_keys(slab), d_sorted(slab);
   DevBuf d_ent[kMaxMemoDepth] = {DevBuf(slab), DevBuf(slab), DevBuf(slab)};
@@ -835,7 +848,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
                      d_sb.as<uint32_t>(), attrs, sets, (uint32_t)G, A, d_off.as<uint64_t>(),
                      nullptr, d_keys.as<uint64_t>());
   HIP_TRY(hipGetLastError());
-  HIP_TRY(prim.sort(d_keys.as<uint64_t>(), d_sorted.as<uint64_t>(), T, 57));
+  HIP_TRY(prim.sort(d_keys.as<uint64_t>(), d_sorted.as<uint64_t>(), T, 0, key_bits));
   HIP_TRY(d_ent[0].reserve(T * 8 + 8));
   HIP_TRY(prim.unique(d_sorted.as<uint64_t>(), d_ent[0].as<uint64_t>(), T, &nent[0], d_cnt8));
   {
@@ -911,7 +924,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
                        d_sb.as<uint32_t>(), d_soff.as<uint64_t>(), d_dkeys.as<uint64_t>(), attrs,
                        sets, d_off.as<uint64_t>(), nullptr, d_keys.as<uint64_t>());
     HIP_TRY(hipGetLastError());
-    HIP_TRY(prim.sort(d_keys.as<uint64_t>(), d_sorted.as<uint64_t>(), T, 57));
+    HIP_TRY(prim.sort(d_keys.as<uint64_t>(), d_sorted.as<uint64_t>(), T, 0, key_bits));
     HIP_TRY(d_ent[d - 1].reserve(T * 8 + 8));
     HIP_TRY(prim.unique(d_sorted.as<uint64_t>(), d_ent[d - 1].as<uint64_t>(), T, &nent[d - 1],
                         d_cnt8));
@@ -992,7 +1005,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(prim.inscan(d_c.as<uint32_t>(), eng->d_xr2.as<uint32_t>(), 65537));
     hipLaunchKernelGGL(k_sort_keys_of_lists, dim3(grid_for(L2)), dim3(kThreads), 0, s,
                        d_lgram[1].as<uint32_t>(), L2, d_k.as<uint64_t>());
-    HIP_TRY(prim.sort(d_k.as<uint64_t>(), d_o.as<uint64_t>(), L2, 48));
+    HIP_TRY(prim.sort(d_k.as<uint64_t>(), d_o.as<uint64_t>(), L2, 32, 48));
     HIP_TRY(eng->d_xe2.reserve(L2 * 16 + 16));
     hipLaunchKernelGGL(k_xe2, dim3(grid_for(L2)), dim3(kThreads), 0, s, d_o.as<uint64_t>(), L2,
                        eng->d_beg[1].as<uint32_t>(), eng->d_nrep[1].as<uint32_t>(),
@@ -1019,7 +1032,7 @@ int build_image_device(ngap_engine *eng, const HostGroup *hg, int32_t G, int32_t
     HIP_TRY(d_xpos.reserve((L3 + 1) * 8));
     hipLaunchKernelGGL(k_sort_keys_of_lists, dim3(grid_for(L3)), dim3(kThreads), 0, s,
                        d_lgram[2].as<uint32_t>(), L3, d_k.as<uint64_t>());
-    HIP_TRY(prim.sort(d_k.as<uint64_t>(), d_o.as<uint64_t>(), L3, 56));
+    HIP_TRY(prim.sort(d_k.as<uint64_t>(), d_o.as<uint64_t>(), L3, 32, 56));
     hipLaunchKernelGGL(k_x3_runs, dim3(grid_for(L3)), dim3(kThreads), 0, s, d_o.as<uint64_t>(),
                        L3, eng->d_beg[2].as<uint32_t>(), d_start.as<uint32_t>(),
                        d_contrib.as<uint64_t>());
