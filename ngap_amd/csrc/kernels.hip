@@ -362,14 +362,6 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
   wsync();
 }
 
-// Rank-table lookup: pair `at` covers 32 consecutive keys; returns the
-// key's list index, or -1 when bit `bit` of the pair's word is clear.
-NGAP_DEV int32_t memo_rank(const uint32_t *sel, size_t at, uint32_t bit) {
-  const uint2 w = reinterpret_cast<const uint2 *>(sel)[at];
-  if (!((w.x >> bit) & 1u)) return -1;
-  return (int32_t)(w.y + __popc(w.x & ((1u << bit) - 1u)));
-}
-
 // Roots for positions [p0, pend): one lane per position.  A position whose
 // byte starts no root costs one load and one bit test.  A lane uses the
 // deepest memo level that fits before the chunk end (kernel_ngap_OA.cu:243-

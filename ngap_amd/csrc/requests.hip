@@ -8,8 +8,9 @@
 // device does the rest:
 //  * k_gather reads the requests' bytes straight from the pinned buffers, 16
 //    bytes a lane and four loads in flight, which is what the link takes (7.5 MB in
-//    0.135 ms, 55 GB/s, where no other launch reads); the same kernel clears the run's counters and flags, sets the map of the
-//    requests' last bytes and lists the work items.
+//    0.135 ms, 55 GB/s, where no other launch reads); the same kernel clears the
+//    run's counters and flags, sets the map of the requests' last bytes and lists
+//    the work items.
 //  * k_results writes the counters and the first reports to pinned memory, where
 //    retiring the launch finds them without another copy.
 #include <hip/hip_runtime.h>
@@ -126,7 +127,8 @@ hipError_t launch_gather(hipStream_t s, const RequestBatch &B) {
   const uint64_t units = ((uint64_t)B.units + kUnitsPerLane - 1) / kUnitsPerLane;
   // a lane for every four units, and enough for the work items and the map
   const uint64_t want = std::max<uint64_t>(units, std::max(B.num_tasks, B.map_words / 4));
-  const uint32_t blocks = (uint32_t)((std::max<uint64_t>(want, kItemLanes) + kThreads - 1) / kThreads);
+  const uint32_t blocks =
+      (uint32_t)((std::max<uint64_t>(want, kItemLanes) + kThreads - 1) / kThreads);
   hipLaunchKernelGGL(k_gather, dim3(blocks), dim3(kThreads), 0, s, B);
   return hipGetLastError();
 }
