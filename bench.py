@@ -272,16 +272,16 @@ def roofline_of(groups, data, chunk, depth, kern_ms, engine_label, workload, tra
         f"input byte ({ss['per_group']:.1f} group by group, {ss['reference']:.1f} for the "
         f"reference algorithm, floor {ss['floor']:.4f}); {ss['stats']}")
     achieved = model * total / (kern_ms * 1e-3) / 1e9
-    traffic = None
+    traffic, kernel = None, "k_scan" if depth >= 3 else "k_batched_stream"
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     if os.path.exists(tpath):
         t = json.load(open(tpath)).get(traffic_key)
         if t and t.get("engine") == engine_label and t.get("precompute_depth") == depth:
-            traffic = t["bytes_per_launch"]
+            traffic, kernel = t["bytes_per_launch"], t["kernel"]
     return dict(bound="hbm", achieved=round(achieved, 2), peak=HBM_PEAK_GBS, unit="GB/s",
                 frac=round(achieved / HBM_PEAK_GBS, 5), traffic=traffic,
                 traffic_gbs=round(traffic / (kern_ms * 1e-3) / 1e9, 1) if traffic else None,
-                kernel="k_batched_stream", kernel_ms=round(kern_ms, 4),
+                kernel=kernel, kernel_ms=round(kern_ms, 4),
                 work_items="all-group" if cross else "per-group",
                 algorithmic_bytes_per_input_byte=round(model, 3),
                 floor_bytes_per_input_byte=round(ss["floor"], 5),
