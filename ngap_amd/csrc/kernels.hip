@@ -302,8 +302,8 @@ NGAP_DEV void refill_from_spill(const KParams &P, WaveState &W) {
 // space (prefix sum over the wave), 64 entries per step.  Every entry that
 // reports is emitted; entries are also pushed as items unless the lane's
 // list is report-only (bit 31 of beg), the state has no successors, or the
-// position is the chunk's last.
-template <bool Stage = false>
+// position is the chunk's last, or (Filter) its next byte cannot match.
+template <bool Stage = false, bool Filter = true>
 NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg,
                       uint32_t pos, uint32_t gtag, const int32_t *list,
                       const uint32_t *filt) {
@@ -313,13 +313,17 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
     const bool ok = cnt == 1u;
     if (wballot(ok) == 0) return;
     const int32_t e = ok ? list[beg & 0x7fffffffu] : 0;
-    const uint32_t f = ok ? filt[beg & 0x7fffffffu] : 0;
-    const uint32_t next = P.input[ok ? min_u(pos + 1, last) : last];
+    uint32_t f = 0, next = 0;
+    if (Filter) {
+      f = ok ? filt[beg & 0x7fffffffu] : 0;
+      next = P.input[ok ? min_u(pos + 1, last) : last];
+    }
     const uint64_t it = item_of(((uint32_t)e & (uint32_t)kIdMask) | gtag, pos);
     emit(P, W, ok && (e & kFlagReport), it);
     bool keep = ok && !(beg >> 31) && !(e & kFlagDeadEnd) && (pos + 1 < W.cend);
     if (keep && P.dedup && (e & kFlagDedup)) keep = dedup_fresh(P, W, it);
-    push_filtered<Stage>(P, W, keep, f, next, it);
+    if (Filter) push_filtered<Stage>(P, W, keep, f, next, it);
+    else push<Stage>(P, W, keep, it);
     return;
   }
   uint32_t incl = wave_incl_scan(cnt, W.lane);
@@ -348,16 +352,19 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
       ronly = bg >> 31;
       const uint32_t at = (bg & 0x7fffffffu) + (j - W.sh_pref[lo]);
       e = list[at];
-      f = filt[at];
       ppos = W.sh_pos[lo];
-      next = P.input[min_u(ppos + 1, last)];
+      if (Filter) {
+        f = filt[at];
+        next = P.input[min_u(ppos + 1, last)];
+      }
       tg = W.sh_tag[lo];
     }
     const uint32_t u = ((uint32_t)e & (uint32_t)kIdMask) | tg;
     emit(P, W, ok && (e & kFlagReport), item_of(u, ppos));
     bool keep = ok && !ronly && !(e & kFlagDeadEnd) && (ppos + 1 < W.cend);
     if (keep && P.dedup && (e & kFlagDedup)) keep = dedup_fresh(P, W, item_of(u, ppos));
-    push_filtered<Stage>(P, W, keep, f, next, item_of(u, ppos));
+    if (Filter) push_filtered<Stage>(P, W, keep, f, next, item_of(u, ppos));
+    else push<Stage>(P, W, keep, item_of(u, ppos));
   }
   wsync();
 }
@@ -373,7 +380,12 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
 // valid address when a lane does not need the value (index 0, or the chunk's
 // last byte), and the value is selected afterwards: the loads of a step then
 // go out together instead of one branch (and one wait) at a time.
-template <bool Stage = false>
+// Deep: the lists of depth 2 and 3 with their entries' filters.  Where a unit's
+// waves take their positions one batch after the other (drain) they spare a step
+// too seldom: 1,024 automata, 2 MiB, depth 3 5.9 ms without and 6.05 with them, while
+// work items whose roots and expansions overlap (drain_stream) take 6.25 and 6.12.
+// At depth 1 they always pay: 11.1 and 8.7 ms, 10.9 and 8.1.
+template <bool Stage = false, bool Deep = true>
 NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) {
   const uint8_t *in = P.input;
   const uint32_t p = p0 + W.lane;
@@ -434,9 +446,9 @@ NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) 
     beg3 = b3;
     cnt3 = li3 >= 0 ? e3 - b3 : 0u;
   }
-  flatten<Stage>(P, W, cnt2, beg2, p + 1, W.gtag, P.img.list[1], P.img.filt[1]);
+  flatten<Stage, Deep>(P, W, cnt2, beg2, p + 1, W.gtag, P.img.list[1], P.img.filt[1]);
   if (wballot(cnt3 != 0)) 
-    flatten<Stage>(P, W, cnt3, beg3, p + 2, W.gtag, P.img.list[2], P.img.filt[2]);
+    flatten<Stage, Deep>(P, W, cnt3, beg3, p + 2, W.gtag, P.img.list[2], P.img.filt[2]);
 }
 
 // Distributes per-lane index ranges [e0, e0 + ecnt) over the wave, 64
@@ -885,7 +897,7 @@ NGAP_DEV void drain(const KParams &P, WaveState &W, Src &src) {
       uint32_t a, b;
       if (!src.next(W, a, b)) roots_left = false;
       else if (Cross) roots_cross(P, W, a, b);
-      else roots(P, W, a, b);
+      else roots<false, false>(P, W, a, b);
       continue;
     }
     const uint64_t idle = wballot(!valid);
