@@ -260,7 +260,11 @@ int ngap_get_tasks(ngap_engine *eng, ngap_task *out, uint64_t cap, uint64_t *n_o
  * No counterpart in the reference (one input per process there).  A request
  * (group, bytes) is scanned as one chunk.  Requests queue; whenever one of
  * max_inflight launch slots is free and the HBM budget allows, all queued
- * requests that fit are packed into one launch on that slot's stream. */
+ * requests that fit are packed into one launch on that slot's stream.
+ * Loading other groups first completes the launches in flight, on the groups
+ * they were started with; requests still queued are scanned with the new groups
+ * (one whose group no longer exists fails).  While no groups are loaded (a load
+ * failed) nothing is launched: NGAP_ERR_STATE, and the requests stay queued. */
 typedef struct ngap_server ngap_server;
 
 /* opts: algorithm / precompute depth / unique as for ngap_run (report_off is

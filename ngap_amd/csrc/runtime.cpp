@@ -938,6 +938,7 @@ int ngap_load_groups_ex(ngap_engine *eng, const ngap_group_desc *groups, int32_t
       hg[i].sod = groups[i].start_states;
     }
     std::string err;
+    if (const int rc = settle_servers(eng)) return rc;  // (the loaded groups stay)
     eng->loaded = false;
     eng->generation++;
     eng->ctx.have_run = false;

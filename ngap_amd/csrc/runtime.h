@@ -222,6 +222,16 @@ hipError_t launch_results(hipStream_t s, const unsigned long long *counters,
                           const uint64_t *reports, uint64_t cap, unsigned long long *to_counters,
                           uint64_t *to_reports);
 
+// The request servers of an engine (ngap_server_create adds, ngap_server_destroy
+// removes; shared, since either may be destroyed first).
+struct ServerList {
+  std::vector<ngap_server *> all;
+};
+// Retires every launch in flight on the engine's servers, re-runs of overflowed
+// ones included.  Their kernels hold raw pointers into the image, whose memory
+// the next load reuses, so a load begins with this.
+int settle_servers(ngap_engine *eng);
+
 // Kernel launchers (kernels.hip).  launch_reset clears the run's counters
 // and n per-work-item flags (and root counts, when given); launch_roots runs
 // the root pass (k_roots) over P.pieces.
@@ -246,6 +256,7 @@ struct ngap_engine {
   int batched_per_cu[12 * ngapamd::kBatchedKinds] = {0};
   ngapamd::Image img;
   bool loaded = false;
+  std::shared_ptr<ngapamd::ServerList> servers = std::make_shared<ngapamd::ServerList>();
   ngapamd::Slab build_slab;  // the device builder's memory while a load runs
   ngapamd::DevBuf d_meta, d_succ4, d_cls, d_sod, d_mask1;
   ngapamd::DevBuf d_beg[ngapamd::kMaxMemoDepth], d_nrep[ngapamd::kMaxMemoDepth],

@@ -161,6 +161,7 @@ LaunchSize launch_size(uint64_t bytes, uint64_t ntasks, uint32_t max_blocks,
 
 struct ngap_server {
   ngap_engine *eng = nullptr;
+  std::shared_ptr<ServerList> peers;  // the engine's servers, this one among them
   uint64_t budget = 0;
   ngap_run_opts opts;
   Mapping mp;
@@ -175,6 +176,11 @@ struct ngap_server {
   uint64_t peak_held = 0, peak_inflight = 0, launches = 0, rejected = 0, redone = 0;
   PinnedPool pinned;  // freed by ngap_server_destroy after every launch completed
   std::unique_ptr<HostPool> copier;  // staging copies of large requests
+  ~ngap_server() {
+    if (!peers) return;
+    auto &v = peers->all;
+    v.erase(std::remove(v.begin(), v.end(), this), v.end());
+  }
   uint64_t held() const {
     uint64_t h = 0;
     for (auto &x : slots) h += x->held();
@@ -222,6 +228,13 @@ bool fits_budget(ngap_server *s, Slot &sl, LaunchSize &z) {
 }
 
 int launch_slot(ngap_server *s, Slot &sl) {
+  // the groups may be others than when the server was created or the requests
+  // were submitted
+  std::string err;
+  if (!s->eng->loaded) return ngap_fail(NGAP_ERR_STATE, "no groups loaded");
+  if (!map_algorithm(s->opts.algorithm, s->opts.precompute_depth, s->eng->img.memo_depth, s->mp,
+                     err))
+    return ngap_fail(NGAP_ERR_INVALID, err);
   sl.ids.clear();
   sl.base.clear();
   const uint32_t wpb = kBlockThreads / kWave;
@@ -243,6 +256,13 @@ int launch_slot(ngap_server *s, Slot &sl) {
   while (!s->queue.empty()) {
     const uint64_t id = s->queue.front();
     Request &r = s->reqs[id];
+    if (r.group >= s->eng->img.num_groups) {  // its group is gone
+      s->queue.pop_front();
+      s->queued_bytes -= r.len;
+      fail_request(s, r);
+      share = share_now();
+      continue;
+    }
     const uint64_t need = total + r.len;
     if (!sl.ids.empty() && (need >= (1ull << 31) || total >= share)) break;
     // the window only grows with the launch's bytes: 256-position work items
@@ -449,6 +469,16 @@ int retire_slot(ngap_server *s, Slot &sl) {
 
 }  // namespace
 
+int ngapamd::settle_servers(ngap_engine *eng) {
+  for (ngap_server *s : eng->servers->all)
+    for (auto &sl : s->slots) {
+      if (!sl->busy) continue;
+      const int rc = retire_slot(s, *sl);
+      if (sl->busy) return rc;  // (a launch that ended in an error has failed its requests)
+    }
+  return NGAP_OK;
+}
+
 extern "C" {
 
 int ngap_server_create(ngap_engine *eng, uint64_t budget, int32_t max_inflight,
@@ -484,6 +514,8 @@ int ngap_server_create(ngap_engine *eng, uint64_t budget, int32_t max_inflight,
       rc = s->slots.back()->ctx.init();
       if (rc) return rc;
     }
+    eng->servers->all.push_back(s.get());
+    s->peers = eng->servers;
     *out = s.release();
     return NGAP_OK;
   });
