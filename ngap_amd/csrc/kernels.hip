@@ -1670,14 +1670,14 @@ NGAP_DEV void block_append(const KParams &P, WaveState &W, uint32_t *count, uint
                            bool pred, uint32_t u) {
   const uint64_t m = wballot(pred);
   if (m == 0) return;
+  const uint32_t cnt = __popcll(m);
   uint32_t base = 0;
-  if (W.lane == 0) base = atomicAdd(count, (uint32_t)__popcll(m));
+  if (W.lane == 0) base = atomicAdd(count, cnt);
   base = from_first(base);
   const uint32_t slot = base + mask_rank(m);
-  if (pred) {
-    if (slot < P.spill_cap) buf[slot] = u;
-    else W.overflow = true;
-  }
+  if (pred && slot < P.spill_cap) buf[slot] = u;
+  // the wave's flag, whichever lane lost its state (lane 0 reports it)
+  if (base + cnt > P.spill_cap) W.overflow = true;
 }
 
 __global__ void __launch_bounds__(kBlockThreads) k_blocking(KParams P) {
