@@ -182,7 +182,7 @@ NGAP_HD inline int batched_kind(const KParams &P) {
 // cache, then: list positions in work (65 + 3 x 64 words), the root masks and
 // the open work items;
 constexpr uint32_t kWaveFixed = (kRbuf + kDc) * 8 + (65 + 3 * kWave + 16 + kMaxOpen + 1) / 2 * 8;
-NGAP_HD inline uint32_t wave_lds_bytes(uint32_t ring) { return kWaveFixed + ring * 8; }
+NGAP_HD constexpr uint32_t wave_lds_bytes(uint32_t ring) { return kWaveFixed + ring * 8; }
 
 // in k_scan: 64 marks, the waiting 3-grams (a wave's width less one and a search
 // of 128 positions more) and the open work items;
@@ -190,7 +190,25 @@ NGAP_HD inline uint32_t wave_lds_bytes(uint32_t ring) { return kWaveFixed + ring
 // fit a CU's 160 KiB.
 constexpr uint32_t kKeyCap = 3 * kWave;
 constexpr uint32_t kScanFixed = (kRbuf + kDc) * 8 + kWave * 4 + kKeyCap * 8 + kMaxOpen * 4;
-NGAP_HD inline uint32_t scan_table_bytes(uint32_t groups) { return (groups * 8 + 15) / 16 * 16; }
-NGAP_HD inline uint32_t scan_wave_bytes(uint32_t ring) { return kScanFixed + ring * 8; }
+NGAP_HD constexpr uint32_t scan_table_bytes(uint32_t groups) { return (groups * 8 + 15) / 16 * 16; }
+NGAP_HD constexpr uint32_t scan_wave_bytes(uint32_t ring) { return kScanFixed + ring * 8; }
+
+constexpr uint32_t kMaxGroups = 1024;  // ten group bits in a report id
+// LDS ring entries per wave: by default, and the range of ring_capacity
+constexpr uint32_t kRing = 256, kMinRing = 64, kMaxRing = 2048;
+// LDS bytes of a launch of the batched kernel `kind` over `groups` groups, and of
+// the other kernels with `waves` waves a workgroup; every size is within
+// kMaxLds, which each kernel's limit is set to (set_lds_limit).
+constexpr uint32_t lds_bytes(uint32_t ring = kRing, uint32_t waves = kBlockThreads / kWave) {
+  return 16 + waves * wave_lds_bytes(ring);
+}
+constexpr uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups) {
+  return kind < 5 ? lds_bytes(ring)
+                  : 16 + scan_table_bytes(groups) + kBlockThreads / kWave * scan_wave_bytes(ring);
+}
+constexpr uint32_t larger(uint32_t a, uint32_t b) { return a > b ? a : b; }
+constexpr uint32_t kMaxLds = larger(larger(lds_bytes(kMaxRing), lds_bytes(kRing, kPlainWaves)),
+                                    batched_lds(kMaxRing, 5, kMaxGroups));
+static_assert(kMaxLds <= 160 * 1024, "a workgroup's LDS");
 
 }  // namespace ngapamd

@@ -174,15 +174,6 @@ void RunCtx::drop_graph() {
   gkey.clear();
 }
 
-uint32_t lds_bytes(uint32_t ring) {
-  return 16 + (kBlockThreads / kWave) * wave_lds_bytes(ring);
-}
-
-uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups) {
-  if (kind < 5) return lds_bytes(ring);
-  return 16 + scan_table_bytes(groups) + (kBlockThreads / kWave) * scan_wave_bytes(ring);
-}
-
 // ring_capacity option -> LDS ring entries (0 = default); 0 when invalid
 uint32_t ring_of(const ngap_run_opts &o) {
   const uint32_t r = o.ring_capacity ? o.ring_capacity : kRing;
@@ -777,8 +768,7 @@ int run_plain(ngap_engine *eng, RunCtx &ctx, KParams P, const ngap_run_opts &o,
     if (const int rc = ctx.begin(P, units, false)) return rc;
     HIP_TRY(hipEventRecord(ctx.ev0, ctx.stream));  // times the matching kernel alone
     if (blocking) HIP_TRY(launch_blocking(ctx.stream, P, units, lds_bytes()));
-    else HIP_TRY(launch_plain(ctx.stream, P, units,
-                              16 + P.waves_per_block * wave_lds_bytes(kRing)));
+    else HIP_TRY(launch_plain(ctx.stream, P, units, lds_bytes(kRing, P.waves_per_block)));
     if (const int rc = ctx.finish(&ms, cnt, true)) return rc;
     all_ms += ms;
     // what a smaller part of a unit's worklist could not hold, four waves' can
@@ -848,7 +838,7 @@ int ngap_create(int32_t device, ngap_engine **out) {
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, device));
     e->num_cus = prop.multiProcessorCount;
-    HIP_TRY(set_lds_limit(std::max(lds_bytes(kMaxRing), batched_lds(kMaxRing, 5, 1024))));
+    HIP_TRY(set_lds_limit(kMaxLds));
     rc = noalloc_attach(device, &e->scratch);  // this device's scratch array (noalloc.cpp)
     if (rc) return rc;
     *out = e.release();

@@ -29,10 +29,6 @@ int ngap_fail(int code, const std::string &msg);
 
 namespace ngapamd {
 
-// LDS ring entries per wave, by default
-constexpr uint32_t kRing = 256;
-constexpr uint32_t kMinRing = 64, kMaxRing = 2048;  // batched ring_capacity range
-
 // Device memory for one load: the builder's temporaries and the arrays it
 // builds come out of a few large chunks, by best fit, and go back to them.  What
 // is given back is handed out again without waiting, so all of it is used on one
@@ -185,9 +181,6 @@ struct Mapping {
 };
 
 bool map_algorithm(int algorithm, int depth_req, int loaded_depth, Mapping &m, std::string &err);
-uint32_t lds_bytes(uint32_t ring = kRing);
-// LDS of a launch of the batched kernel `kind` over `groups` groups.
-uint32_t batched_lds(uint32_t ring, int kind, uint32_t groups);
 
 // Sorts ctx's last n reports (offsets below 2^offset_bits) on the device and
 // encodes them (reports.hip): into ctx.host_reports[1..] up to kSmallReports,
@@ -244,7 +237,7 @@ hipError_t launch_blocking(hipStream_t s, const KParams &P, uint32_t units, uint
 hipError_t launch_roots(hipStream_t s, const KParams &P, uint32_t lds);
 hipError_t launch_batched(hipStream_t s, const KParams &P, uint32_t blocks, uint32_t lds);
 hipError_t batched_occupancy(int *blocks_per_cu, uint32_t lds, int kind);  // kind: batched_kind()
-hipError_t set_lds_limit(uint32_t lds);
+hipError_t set_lds_limit(uint32_t lds);  // of every kernel with dynamic LDS
 
 }  // namespace ngapamd
 
