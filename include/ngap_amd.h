@@ -287,8 +287,8 @@ int ngap_server_take(ngap_server *srv, uint64_t req_id, int32_t *state, uint64_t
 int ngap_server_pending(ngap_server *srv, uint64_t *queued, uint64_t *inflight);
 
 /* Memory and admission figures of a server.  held_bytes counts the device
- * buffers of every launch slot (input, last-byte map, reports, work items,
- * worklist spill), in flight or kept for reuse; admission keeps it within
+ * buffers of every launch slot (input, last-byte map, list of requests, reports,
+ * work items, worklist spill), in flight or kept for reuse; admission keeps it within
  * budget_bytes (idle slots give their buffers back when a launch needs the
  * room).  A launch whose worklists or report buffer overflowed is re-run with
  * larger ones (redone), which may go past the budget for that re-run.  The

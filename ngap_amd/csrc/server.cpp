@@ -91,8 +91,8 @@ struct Slot {
   uint32_t blocks = 0;
   // device bytes this slot's launch buffers hold (reserved, in flight or not)
   uint64_t held() const {
-    return input.n + last_map.n + ctx.reports.n + ctx.spill.n + ctx.tasks.n + ctx.overflow.n +
-           ctx.task_items.n + ctx.fb_tasks.n + ctx.fb_spill.n;
+    return input.n + last_map.n + about.n + ctx.reports.n + ctx.spill.n + ctx.tasks.n +
+           ctx.overflow.n + ctx.task_items.n + ctx.fb_tasks.n + ctx.fb_spill.n;
   }
   // gives the launch buffers back (an idle slot, when the budget needs room)
   void release() {
@@ -127,26 +127,27 @@ uint32_t serve_window(uint64_t total, uint64_t waves) {
   return win;
 }
 
-// Device bytes of a launch's buffers: input, last-byte map, reports (an
-// overflow re-runs the launch with room for all), work items and their
-// flags, and the worklist spill of its workgroups (kServeSpill items per
+// Device bytes of a launch's buffers: input, last-byte map, the list of its
+// requests, reports (an overflow re-runs the launch with room for all), work
+// items and their flags, and the worklist spill of its workgroups (kServeSpill items per
 // wave).  A launch takes at most one workgroup per waves_per_block work
 // items, and fewer when the HBM budget leaves room for fewer.
 struct LaunchSize {
-  uint64_t input, map, reports, tasks, overflow;
+  uint64_t input, map, about, reports, tasks, overflow;
   uint64_t report_cap;
   uint32_t blocks;        // workgroups (spill areas)
   uint64_t per_block;     // spill bytes per workgroup
-  uint64_t fixed() const { return input + map + reports + tasks + overflow; }
+  uint64_t fixed() const { return input + map + about + reports + tasks + overflow; }
   uint64_t spill() const { return (uint64_t)blocks * per_block; }
   uint64_t total() const { return fixed() + spill(); }
 };
 
-LaunchSize launch_size(uint64_t bytes, uint64_t ntasks, uint32_t max_blocks,
+LaunchSize launch_size(uint64_t bytes, uint64_t requests, uint64_t ntasks, uint32_t max_blocks,
                        uint32_t waves_per_block) {
   LaunchSize z;
   z.input = bytes + 16;
   z.map = (bytes / 32 + 2) * 4;
+  z.about = requests * (sizeof(RequestSpan) + sizeof(RequestTasks));
   z.report_cap = std::max<uint64_t>(kMinReportCap, bytes / 2);
   z.reports = z.report_cap * 8;
   z.tasks = ntasks * sizeof(Task);
@@ -212,6 +213,7 @@ uint64_t held_by_others(const ngap_server *s, const Slot &sl) {
 bool fits_budget(ngap_server *s, Slot &sl, LaunchSize &z) {
   const uint64_t keep = std::max<uint64_t>(sl.input.n, z.input) +
                         std::max<uint64_t>(sl.last_map.n, z.map) +
+                        std::max<uint64_t>(sl.about.n, z.about) +
                         std::max<uint64_t>(sl.ctx.reports.n, z.reports) +
                         std::max<uint64_t>(sl.ctx.tasks.n, z.tasks) +
                         std::max<uint64_t>(sl.ctx.overflow.n, z.overflow) +
@@ -268,7 +270,7 @@ int launch_slot(ngap_server *s, Slot &sl) {
     // the window only grows with the launch's bytes: 256-position work items
     // bound the work-item count from above
     const uint64_t nt = ntasks_ub + (r.len + 255) / 256;
-    LaunchSize z = launch_size(need, nt, s->blocks_per_launch, wpb);
+    LaunchSize z = launch_size(need, sl.ids.size() + 1, nt, s->blocks_per_launch, wpb);
     if (!fits_budget(s, sl, z)) {
       if (!sl.ids.empty()) break;
       bool others = false;
@@ -315,11 +317,11 @@ int launch_slot(ngap_server *s, Slot &sl) {
   }
   // the actual work items are no more than the admission bound: the launch
   // needs no more than what was admitted
-  LaunchSize z = launch_size(total, ntasks, s->blocks_per_launch, wpb);
+  LaunchSize z = launch_size(total, n, ntasks, s->blocks_per_launch, wpb);
   z.blocks = std::min(z.blocks, adm_blocks);
   HIP_TRY(sl.input.reserve(z.input));
   HIP_TRY(sl.last_map.reserve(z.map));
-  const size_t order_at = n * sizeof(RequestSpan), about = order_at + n * sizeof(RequestTasks);
+  const size_t order_at = n * sizeof(RequestSpan), about = z.about;
   if (sl.about_cap < about) {
     if (sl.about_host) HIP_TRY(hipHostFree(sl.about_host));
     sl.about_host = nullptr;
@@ -328,7 +330,7 @@ int launch_slot(ngap_server *s, Slot &sl) {
     HIP_TRY(hipHostMalloc((void **)&sl.about_host, cap, hipHostMallocDefault));
     sl.about_cap = cap;
   }
-  HIP_TRY(sl.about.reserve(sl.about_cap));
+  HIP_TRY(sl.about.reserve(z.about));
   memcpy(sl.about_host, sl.spans.data(), order_at);
   memcpy(sl.about_host + order_at, sl.order.data(), about - order_at);
   HIP_TRY(hipMemcpyAsync(sl.about.p, sl.about_host, about, hipMemcpyHostToDevice, sl.ctx.stream));
