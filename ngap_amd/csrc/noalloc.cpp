@@ -108,7 +108,7 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
     uint32_t fewer = blocks;  // the grid that gives each wave a larger worklist
     if (!o.persistent_blocks) {
       fewer = job_blocks(blocks, P.waves_per_block, work, kSpillPositions);
-      blocks = job_blocks(blocks, P.waves_per_block, work);
+      blocks = eng->ctx.scratch_few ? fewer : job_blocks(blocks, P.waves_per_block, work);
     }
     const uint64_t waves = (uint64_t)blocks * P.waves_per_block;
     uint32_t win = o.window;
@@ -166,6 +166,7 @@ extern "C" int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts,
       // what a worklist of the larger grid could not hold, the smaller grid's may
       if ((uint32_t)cnt[3] == 0 || blocks <= fewer) break;
       blocks = fewer;
+      ctx.scratch_few = true;
     }
     ms = all_ms;
     if (st) {

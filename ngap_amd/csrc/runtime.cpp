@@ -745,7 +745,8 @@ int run_plain(ngap_engine *eng, RunCtx &ctx, KParams P, const ngap_run_opts &o,
   P.ring_cap = kRing;  // these launches size their LDS for the default ring
   const uint32_t few = P.waves_per_block;
   // a worklist capacity that the caller gives is a wave's of four
-  if (!blocking && !o.spill_capacity) P.waves_per_block = plain_waves(units, eng->num_cus);
+  if (!blocking && !o.spill_capacity && !ctx.plain_few)
+    P.waves_per_block = plain_waves(units, eng->num_cus);
   float ms = 0, all_ms = 0;
   unsigned long long cnt[4] = {0, 0, 0, 0};
   for (;;) {
@@ -774,6 +775,7 @@ int run_plain(ngap_engine *eng, RunCtx &ctx, KParams P, const ngap_run_opts &o,
     // what a smaller part of a unit's worklist could not hold, four waves' can
     if ((uint32_t)cnt[3] == 0 || P.waves_per_block == few) break;
     P.waves_per_block = few;
+    ctx.plain_few = true;
   }
   ms = all_ms;
   const uint64_t overflowed = (uint32_t)cnt[3];

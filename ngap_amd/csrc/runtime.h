@@ -133,7 +133,10 @@ struct RunCtx {
   // offsets (items), the areas and the per-work-item counts
   DevBuf pieces, root_off, root_items, root_count;
   uint32_t num_pieces = 0;
-  bool spill_most = false;      // a smaller worklist than the default overflowed
+  // a run whose waves had less than the largest default worklists overflowed:
+  // later runs of its kind do not try that again (batched; plain units on four
+  // waves; ngap_run_noalloc on the smaller grid)
+  bool spill_most = false, plain_few = false, scratch_few = false;
   uint32_t root_factor = 0;     // items per position the resident areas were sized for
   uint32_t root_boost = 1;      // doubles (up to 64x) after a root area overflowed,
   uint64_t root_gen = 0;        // for this engine generation (groups and input)
