@@ -427,14 +427,15 @@ __global__ void __launch_bounds__(256)
 struct Buf {
   void *p = nullptr;
   size_t n = 0;
-  ~Buf() {
-    if (p) (void)hipFree(p);
-  }
-  hipError_t reserve(size_t bytes) {
-    if (bytes <= n && p) return hipSuccess;
+  ~Buf() { release(); }
+  void release() {
     if (p) (void)hipFree(p);
     p = nullptr;
     n = 0;
+  }
+  hipError_t reserve(size_t bytes) {
+    if (bytes <= n && p) return hipSuccess;
+    release();
     hipError_t e = hipMalloc(&p, bytes ? bytes : 8);
     if (e == hipSuccess) n = bytes ? bytes : 8;
     return e;
@@ -444,8 +445,9 @@ struct Buf {
 
 }  // namespace
 
-// Samples that training keeps on the device, at most (15M samples).
-constexpr uint64_t kResident = 16ull << 30;
+// Samples that training keeps on the device while it runs, at most (15M), and
+// that the model goes on holding afterwards, for the next training (254,000).
+constexpr uint64_t kResident = 16ull << 30, kHeld = 256ull << 20;
 
 struct ngap_mlp {
   int device = 0;
@@ -459,6 +461,10 @@ namespace {
 uint32_t blocks_for(uint64_t n, uint64_t per_block, uint64_t most) {
   return (uint32_t)std::min<uint64_t>((n + per_block - 1) / per_block, most);
 }
+
+// k_gradient's workgroups over n samples, and what their sums take
+uint32_t grad_blocks(uint64_t n) { return blocks_for(n, kTile, kMaxGradBlocks); }
+size_t grad_bytes(uint64_t n) { return (size_t)grad_blocks(n) * kPart * 4; }
 
 int load_batch(ngap_mlp *m, const float *x, const float *t, uint64_t n) {
   MLP_TRY(m->X.reserve(n * kIn * 4));
@@ -474,8 +480,8 @@ int load_batch(ngap_mlp *m, const float *x, const float *t, uint64_t n) {
 // as an Adam step when grad is null; the loss sum goes to *loss (device).
 int grad_on_device(ngap_mlp *m, const uint32_t *idx, uint64_t n, float *grad, float *loss,
                    const Adam &o) {
-  const uint32_t blocks = blocks_for(n, kTile, kMaxGradBlocks);
-  MLP_TRY(m->G.reserve((size_t)blocks * kPart * 4));
+  const uint32_t blocks = grad_blocks(n);
+  MLP_TRY(m->G.reserve(grad_bytes(n)));
   hipLaunchKernelGGL(k_gradient, dim3(blocks), dim3(kThreads), kGradLds, 0, m->P.f(), m->X.f(),
                      m->T.f(), idx, n, m->G.f());
   MLP_TRY(hipGetLastError());
@@ -645,6 +651,18 @@ int ngap_mlp_train(ngap_mlp *m, const float *x, const float *t, uint64_t n, int3
     // kResident bytes), and a mini-batch is a range of the epoch's shuffled
     // row numbers; beyond that each mini-batch is gathered on the host.
     const uint64_t steps = (n + batch - 1) / batch;  // per epoch
+    MLP_TRY(m->loss.reserve(steps * 4));  // one sum per mini-batch of an epoch
+    MLP_TRY(m->G.reserve(grad_bytes(std::min<uint64_t>(batch, n))));
+    struct GiveBack {
+      ngap_mlp *m;
+      const size_t had;
+      ~GiveBack() {
+        if (m->X.n <= std::max<size_t>(had, kHeld)) return;
+        m->X.release();
+        m->T.release();
+        m->idx.release();
+      }
+    } give_back{m, m->X.n};
     const bool resident = n < (1ull << 32) && n <= kResident / (kIn * 4) &&
                           m->X.reserve(n * kIn * 4) == hipSuccess &&
                           m->T.reserve(n * 4) == hipSuccess && m->idx.reserve(n * 4) == hipSuccess;
@@ -653,7 +671,6 @@ int ngap_mlp_train(ngap_mlp *m, const float *x, const float *t, uint64_t n, int3
       const int rc = load_batch(m, x, t, n);
       if (rc) return rc;
     }
-    MLP_TRY(m->loss.reserve(steps * 4));  // one sum per mini-batch of an epoch
     std::vector<uint32_t> rows32(resident ? n : 0);
     std::vector<uint64_t> rows64(resident ? 0 : n);
     std::vector<float> bx(resident ? 0 : (size_t)batch * kIn), bt(resident ? 0 : batch);
