@@ -18,6 +18,7 @@
 #include <chrono>
 #include <cstring>
 #include <memory>
+#include <thread>
 
 // Schedule ids are unique across the engines of a process, so an id handed
 // back through ngap_run_opts.tasks_id never matches another engine's schedule.
@@ -59,6 +60,16 @@ hipError_t Slab::take(size_t bytes, void **p) {
   constexpr size_t kAlign = 256, kFirst = 4u << 20;
   const size_t want = (bytes + kAlign - 1) / kAlign * kAlign;
   *p = nullptr;
+  if (direct_) {
+    // what was freed just before comes back with a delay of some milliseconds
+    hipError_t e = hipMalloc(p, bytes);
+    for (int ms = 1; e == hipErrorOutOfMemory && ms <= 16; ms *= 2) {
+      (void)hipGetLastError();
+      std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+      e = hipMalloc(p, bytes);
+    }
+    return e;
+  }
   auto best = free_.end();
   for (auto f = free_.begin(); f != free_.end(); ++f)
     if (f->n >= want && (best == free_.end() || f->n < best->n)) best = f;
@@ -87,6 +98,10 @@ hipError_t Slab::take(size_t bytes, void **p) {
 }
 
 void Slab::give(void *p) {
+  if (direct_) {
+    (void)hipFree(p);
+    return;
+  }
   for (size_t i = 0; i < used_.size(); i++) {
     if (used_[i].first != p) continue;
     const Piece x = used_[i].second;
@@ -865,8 +880,9 @@ namespace {
 // 256 B.  The matching kernels gather from these arrays at random; with the
 // arrays built among the builder's temporaries they ran up to 5 % slower
 // than from one fresh allocation.  If the arena cannot be allocated next to
-// the arrays (a very large image), they stay where they are.
-int pack_image(ngap_engine *eng) {
+// the arrays (a very large image), they stay where they are, and *packed is
+// false.
+int pack_image(ngap_engine *eng, bool *packed) {
   using ngapamd::DevBuf;
   const auto arr = eng->image_arrays();
   constexpr size_t kBig = 2u << 20, kSmall = 256;
@@ -880,6 +896,7 @@ int pack_image(ngap_engine *eng) {
       off[i] = total;
       total += arr[i]->n;
     }
+  *packed = total == 0;
   if (total == 0) return NGAP_OK;
   // an arena of the last load that fits, and is no more than twice as large, stays
   if (eng->d_arena.n < total || eng->d_arena.n / 2 > total) {
@@ -904,7 +921,32 @@ int pack_image(ngap_engine *eng) {
     arr[i]->owned = false;
   }
   eng->build_slab.clear();
+  *packed = true;
   return NGAP_OK;
+}
+
+// One build on the device, into the slab, or, with memory short, the arrays and
+// the builder's temporaries in allocations of their own; then the arena.
+int build_and_pack(ngap_engine *eng, const std::vector<HostGroup> &hg, int depth, bool direct,
+                   bool *packed, std::string &err) {
+  for (DevBuf *d : eng->image_arrays()) {
+    d->release();
+    d->slab = &eng->build_slab;
+  }
+  eng->build_slab.clear();
+  eng->build_slab.set_direct(direct);
+  if (direct) eng->d_arena.release();  // (the last load's)
+  int rc = build_image_device(eng, hg.data(), (int32_t)hg.size(), depth, eng->ctx.stream,
+                              eng->img, eng->img_sizes, err);
+  if (direct)
+    for (DevBuf *d : eng->image_arrays()) d->slab = nullptr;
+  eng->build_slab.set_direct(false);
+  if (!rc) return pack_image(eng, packed);
+  (void)hipGetLastError();
+  (void)hipStreamSynchronize(eng->ctx.stream);
+  for (DevBuf *d : eng->image_arrays()) d->release();
+  eng->build_slab.clear();
+  return rc;
 }
 
 }  // namespace
@@ -936,20 +978,26 @@ int ngap_load_groups_ex(ngap_engine *eng, const ngap_group_desc *groups, int32_t
     eng->ctx.have_run = false;
     eng->ctx.drop_graph();
     const int depth = max_depth < 1 ? 1 : max_depth;
-    for (DevBuf *d : eng->image_arrays()) {
-      d->release();
-      d->slab = build == NGAP_BUILD_DEVICE ? &eng->build_slab : nullptr;
-    }
-    eng->build_slab.clear();  // (holds what a failed load, or one without an arena, left)
+    bool packed = false;
     if (build == NGAP_BUILD_DEVICE) {
-      const int rc = build_image_device(eng, hg.data(), num_groups, depth, eng->ctx.stream,
-                                        eng->img, eng->img_sizes, err);
-      if (rc) {
-        for (DevBuf *d : eng->image_arrays()) d->release();
-        eng->build_slab.clear();
-        return err.empty() ? rc : ngap_fail(rc, err);
-      }
+      // The slab's chunks hold the temporaries beside the arrays and are larger
+      // than both.  Where they, or the arena next to them, do not fit, the image
+      // is built again without the slab: no more than the arrays stays then.  Its
+      // many allocations, of whole pages each, can need more than the chunks did:
+      // then the arrays stay in those after all.
+      int rc = build_and_pack(eng, hg, depth, false, &packed, err);
+      const bool fitted = !rc;
+      if (rc == NGAP_ERR_OOM || (!rc && !packed))
+        rc = build_and_pack(eng, hg, depth, true, &packed, err);
+      if (rc == NGAP_ERR_OOM && fitted)
+        rc = build_and_pack(eng, hg, depth, false, &packed, err);
+      if (rc) return err.empty() ? rc : ngap_fail(rc, err);
     } else {
+      for (DevBuf *d : eng->image_arrays()) {
+        d->release();
+        d->slab = nullptr;
+      }
+      eng->build_slab.clear();
       if (!build_image(hg.data(), num_groups, depth, eng->img, err))
         return ngap_fail(NGAP_ERR_INVALID, err);
       Image &im = eng->img;
@@ -988,7 +1036,8 @@ int ngap_load_groups_ex(ngap_engine *eng, const ngap_group_desc *groups, int32_t
       kept.total_states = im.total_states;
       im = std::move(kept);
     }
-    if (const int rc = pack_image(eng)) return rc;
+    if (build == NGAP_BUILD_HOST)
+      if (const int rc = pack_image(eng, &packed)) return rc;
     for (int &n : eng->batched_per_cu) n = 0;  // k_scan's LDS depends on the groups
     eng->built_on_device = build == NGAP_BUILD_DEVICE;
     eng->build_ms =

@@ -35,6 +35,7 @@ namespace ngapamd {
 // stream.  (A load made 65 hipMalloc and 65 hipFree calls, 8.5 of its 20 ms at
 // 128 automata of up to 50,000 states: each free waits for the device and unmaps.
 // With a few chunks, and the uploads through the pinned blocks, it takes 5.5 ms.)
+// Where memory is short it hands out allocations of their own instead (direct).
 class Slab {
  public:
   Slab() = default;
@@ -46,6 +47,8 @@ class Slab {
   hipError_t take(size_t bytes, void **p);
   void give(void *p);
   void clear();  // frees the chunks; nothing taken may be used any more
+  // (while nothing is taken) each piece its own allocation, freed when given back
+  void set_direct(bool direct) { direct_ = direct; }
 
  private:
   struct Piece {
@@ -55,6 +58,7 @@ class Slab {
   std::vector<Piece> free_;  // ascending (chunk, at), neighbours joined
   std::vector<std::pair<void *, Piece>> used_;
   size_t expected_ = 0, total_ = 0;
+  bool direct_ = false;
 };
 
 struct DevBuf {

@@ -1,13 +1,15 @@
 """Calls that go another way where device memory is short: training that cannot
 keep its samples on the device gathers each mini-batch on the host, and reports
-whose radix sort has no work area are sorted on the host.  The same results.  What
-training took for its samples is given back."""
+whose radix sort has no work area are sorted on the host, an image whose builder's
+chunks or arena do not fit is built without them.  The same results.  What training
+took for its samples is given back, and a load keeps no more than its image."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
 
-from ngap_amd import Engine
+from ngap_amd import Engine, NgapError, synth
 from ngap_amd.groups import make_group
 from ngap_amd.mlp import MLP
 
@@ -40,10 +42,20 @@ class Device:
                 size //= 2
         self.hip.hipFree(spare)
 
-    def free(self):
-        for p in self.taken:
-            self.hip.hipFree(p)
-        self.taken = []
+    def room(self):
+        """What can still be taken, in steps of 8 MiB (what was freed just before comes
+        back with a delay)."""
+        time.sleep(0.1)
+        had, n = len(self.taken), 0
+        while self.take(8 * MIB):
+            n += 8 * MIB
+        self.give(had)
+        return n
+
+    def give(self, left=0):
+        while len(self.taken) > left:
+            self.hip.hipFree(self.taken.pop())
+
 
 
 def test_results_with_little_device_memory():
@@ -69,7 +81,7 @@ def test_results_with_little_device_memory():
             print("[case] training without resident samples", flush=True)
             loss2 = models[1].train(x, t, epochs=2, batch=batch, seed=5)
         finally:
-            dev.free()
+            dev.give()
         assert np.array_equal(got, (np.uint64(1) << np.uint64(32)) |
                               (2 * np.arange(m, dtype=np.uint64) + np.uint64(1)))
     assert loss2 == loss
@@ -93,3 +105,40 @@ def test_training_gives_its_samples_back():
     for m in models:
         m.train(x, t, epochs=1, batch=50_000)
     assert before - free() < 2 << 30
+
+
+def test_loads_with_little_device_memory():
+    rng = np.random.default_rng(2)
+    groups = [synth.regex_group(rng, 60000) for _ in range(4)]
+    dev = Device()
+    with Engine(0) as ref, Engine(0) as e:
+        ref.load_groups(groups, 3)
+        image = ref.image_info()["bytes"]
+        try:
+            print("[case] taking device memory", flush=True)
+            dev.leave(800 * MIB)
+            room, had, short = dev.room(), len(dev.taken), False
+            for free in range(room // MIB, 0, -40):
+                while dev.room() > free * MIB:
+                    assert dev.take(8 * MIB)
+                before = dev.room()
+                try:
+                    e.load_groups(groups, 3)
+                except NgapError as x:
+                    assert x.code == 3, x
+                    short = True
+                    break
+                kept = before - dev.room()
+                print("[case] load", free, before // MIB, kept // MIB, image // MIB, flush=True)
+                # 31 arrays in allocations of whole 2 MiB pages, and one step of the count
+                assert kept <= image + (2 * 31 + 8) * MIB
+                for name in ("succ4", "xp3", "list3", "xr2", "meta"):
+                    assert np.array_equal(e.image_array(name), ref.image_array(name)), name
+                # the next load starts without this one's image
+                e.close()
+                e.__init__(0)
+            assert short
+        finally:
+            dev.give()
+        e.load_groups(groups, 3)  # after the failed one
+        assert np.array_equal(e.image_array("xs3"), ref.image_array("xs3"))
