@@ -929,9 +929,9 @@ NGAP_DEV void drain(const KParams &P, WaveState &W, Src &src) {
   }
 }
 
-// A wave's claims of work items.  A workgroup's own items (item i * workgroups +
-// workgroup is its i-th) are taken by its waves with an LDS counter, the others
-// are in one queue an XCD, from which a wave claims by an atomic in memory.  Such
+// A wave's claims of work items.  A workgroup's own items (one a row, own_item) are
+// taken by its waves with an LDS counter, the others are in one queue an XCD
+// (queue_item), from which a wave claims by an atomic in memory.  Such
 // an atomic is a round trip of 2 us, and those of thousands of waves on one address
 // take 20 ns each, one after the other: 2 MiB scanned in two items a wave took
 // 0.086 ms with all claimed so (the queues' ends found by two more atomics a wave)
@@ -985,14 +985,14 @@ struct Claims {
         i = from_first(i);
       }
       first = false;
-      const uint64_t t = (uint64_t)i * gridDim.x + blockIdx.x;
+      const uint64_t t = own_item(i, blockIdx.x, gridDim.x);
       if ((i < per) & (t < P.num_tasks)) return (uint32_t)t;
       own = false;
     }
     ask(P, W);
     if (!asked) return P.num_tasks;
     asked = false;
-    const uint64_t t = (uint64_t)per * gridDim.x + (uint64_t)from_first(ahead) * queues + q;
+    const uint64_t t = (uint64_t)per * gridDim.x + queue_item(from_first(ahead), q, queues);
     if (t < P.num_tasks) return (uint32_t)t;
     dry = true;
     if (W.lane == 0) word[1] = 1;
