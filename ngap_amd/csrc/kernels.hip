@@ -382,9 +382,10 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
 // go out together instead of one branch (and one wait) at a time.
 // Deep: the lists of depth 2 and 3 with their entries' filters.  Where a unit's
 // waves take their positions one batch after the other (drain) they spare a step
-// too seldom: 1,024 automata, 2 MiB, depth 3 5.9 ms without and 6.05 with them, while
-// work items whose roots and expansions overlap (drain_stream) take 6.25 and 6.12.
-// At depth 1 they always pay: 11.1 and 8.7 ms, 10.9 and 8.1.
+// too seldom (1,024 automata, 2 MiB, depth 3: 5.9 ms without and 6.05 with them,
+// before the step itself became cheaper), while work items whose roots and
+// expansions overlap (drain_stream) took 6.25 and 6.12.  At depth 1 they always pay:
+// 11.1 and 8.7 ms, 10.9 and 8.1.
 template <bool Stage = false, bool Deep = true>
 NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) {
   const uint8_t *in = P.input;
@@ -753,27 +754,39 @@ NGAP_DEV void expand(const KParams &P, WaveState &W, bool &valid, uint32_t &v,
     const int32_t es[4] = {rec.ids.x, rec.ids.y, rec.ids.z, rec.ids.w};
     const uint32_t ts[4] = {rec.tests.x, rec.tests.y, rec.tests.z, rec.tests.w};
     // class words of the successors that are not decided by their test word;
-    // successors fill the slots from 0, so the later slots are often empty in
-    // every lane
-    bool need[4], hit[4], keep[4];
+    // successors fill the slots from 0 (a continuation link is in the last), so
+    // the later slots are often empty in every lane, and are skipped then: tested
+    // all the same, units of the plain schedule took 5.10 ms and take 4.88 (1,024
+    // automata, 2 MiB, depth 2)
+    bool need[4], hit[4] = {false, false, false, false}, keep[4] = {false, false, false, false};
     uint32_t cw[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
+    bool rep = false, dup = false;
+    auto fetch = [&](int s) {
       need[s] = more & (es[s] >= 0) & (ts[s] == 0u);
       if (wballot(need[s])) {
         const uint32_t u = (uint32_t)es[s] & (uint32_t)kIdMask;
         cw[s] = P.img.cls[need[s] ? (size_t)(lg.cls_base + u) * 8 + (b >> 5) : 0];
       }
-    }
-    bool rep = false, dup = false;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
+    };
+    auto test = [&](int s) {
       const bool in_class = ((cw[s] >> (b & 31)) & 1u) != 0;
       hit[s] = more & ((ts[s] == (b | kTestLiteral)) | (ts[s] == kTestAll) | (need[s] & in_class));
       rep |= hit[s] & ((es[s] & kFlagReport) != 0);
       keep[s] = hit[s] & ((es[s] & kFlagDeadEnd) == 0) & !last;
       dup |= keep[s] & ((es[s] & kFlagDedup) != 0);
+    };
+    fetch(0);
+    if (wballot(more & (es[1] >= 0))) {
+      fetch(1);
+      if (wballot(more & (es[2] >= 0))) {
+        fetch(2);
+        fetch(3);
+        test(2);
+        test(3);
+      }
+      test(1);
     }
+    test(0);
     if (wballot(rep)) {
 #pragma unroll
       for (int s = 0; s < 4; s++)
