@@ -51,10 +51,11 @@ class HostPool {
   size_t width() const { return th_.size() + 1; }
 
   // Parts of about n / width() bytes (at least kPart, 4 KiB-aligned) covering
-  // [0, n): how run_parts cuts a range.
+  // [0, n): how run_parts cuts a range.  At most width() parts, whatever n leaves
+  // over (callers keep a record per part).
   size_t part_bytes(size_t n) const {
     const size_t parts = std::max<size_t>(1, std::min(width(), n / kPart));
-    return std::max<size_t>(4096, (n / parts + 4095) & ~(size_t)4095);
+    return std::max<size_t>(4096, ((n + parts - 1) / parts + 4095) & ~(size_t)4095);
   }
 
   // f(i, begin, end) for the parts of [0, n); returns when all have run.
