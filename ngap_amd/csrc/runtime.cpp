@@ -332,10 +332,15 @@ uint32_t job_blocks(uint32_t full_blocks, uint32_t waves_per_block, uint64_t wor
 // of positions and 1,024.  Fewer even out the waves' times too little (1,024
 // automata, 8 MiB: one a wave 0.207 ms, two 0.215, four 0.188), longer ones above
 // 4,096 positions a wave too (64 MiB: windows of 8,192 positions 1.35 ms, 4,096
-// 1.16, 1,024 1.09, 256 1.15); shorter ones cost their set-up.
+// 1.16, 1,024 1.09, 256 1.15); shorter ones cost their set-up.  Above 64 MiB they
+// grow again, to stay at 65,536 work items or little more: a list of them is
+// made and uploaded for every new input (1 GiB, 256 automata: 8.2 ms for the first
+// run with windows of 1,024 and 5.5 with 16,384, 5.16 and 5.24 for the next ones).
 uint32_t cross_window(uint64_t positions, uint64_t waves) {
+  constexpr uint64_t kMostItems = 65536;
   const uint64_t per = (positions + 4 * waves - 1) / std::max<uint64_t>(1, 4 * waves);
-  return (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(128, (per + 63) / 64 * 64));
+  const uint64_t win = std::min<uint64_t>(1024, std::max<uint64_t>(128, (per + 63) / 64 * 64));
+  return (uint32_t)std::max(win, ((positions + kMostItems - 1) / kMostItems + 63) / 64 * 64);
 }
 
 // Root pass set-up for the resident work items: each work item's area of
