@@ -148,10 +148,11 @@ int RunCtx::init() {
   HIP_TRY(hipEventCreate(&ev1));
   static_assert(kCounterBytes % 8 == 0, "report slots follow the counters");
   HIP_TRY(counters.reserve(kCounterBytes + kSmallReports * 8));
-  // the reset kernel clears the counters a run uses; the rest stays zero
-  HIP_TRY(hipMemset(counters.p, 0, kCounterBytes));
+  // the reset kernel clears the counters a run uses; the rest stays zero (on the
+  // context's stream, which does not wait for the null stream)
+  HIP_TRY(hipMemsetAsync(counters.p, 0, kCounterBytes, stream));
   report_slots = counters.as<uint64_t>() + kCounterBytes / 8;
-  HIP_TRY(hipMemset(report_slots, 0xFF, kSmallReports * 8));  // every slot empty
+  HIP_TRY(hipMemsetAsync(report_slots, 0xFF, kSmallReports * 8, stream));  // every slot empty
   HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&host_cnt),
                         kCounterBytes + (kSmallReports + 1) * 8, hipHostMallocDefault));
   host_reports = reinterpret_cast<uint64_t *>(host_cnt) + kCounterBytes / 8;
