@@ -103,9 +103,10 @@ typedef struct {
   uint64_t result_capacity;     /* --result-capacity (reports) */
   uint32_t window;              /* batched: positions per work item, 0 = auto */
   uint32_t spill_capacity;      /* items per wave beyond the LDS ring, 0 = auto */
-  uint32_t persistent_blocks;   /* batched: workgroups, 0 = auto (the device's
-                                   occupancy, fewer for a job of fewer than
-                                   640 positions per wave) */
+  uint32_t persistent_blocks;   /* batched: workgroups, at most what the device
+                                   holds at once (more are lowered to that);
+                                   0 = auto (as many, fewer for a job of fewer
+                                   than 128 positions per wave) */
   int32_t use_graph;            /* batched: replay a captured hipGraph */
   const ngap_task *tasks;       /* batched: work items in run order (NULL = the
                                    engine's static schedule) */
@@ -210,14 +211,16 @@ int ngap_run(ngap_engine *eng, const ngap_run_opts *opts, ngap_run_stats *stats)
  * library (one per device, held until the process ends), and its work items
  * are generated on the device (the static schedule's shape: all-group
  * windows at depth >= 2, else one group per work item;
- * opts->window or about two work items per wave).  Runs the batched
+ * opts->window or, as ngap_run's, about four all-group work items per wave,
+ * two of one group).  Runs the batched
  * streaming engine on the engine's stream and waits for it.  Reports are
  * written raw in the device encoding ((offset << 32) | (state | group << 22)),
  * unordered and possibly repeated; sorting, removing repeats and swapping
  * the halves gives ngap_get_reports' output.  stats->reports_raw is their
  * count.  Errors: more than 1M work items (use a larger window), a grid
  * whose worklists do not fit the array, NGAP_ERR_OVERFLOW when a worklist
- * (no fallback here) or report_cap overflows.  Calls that overlap on one
+ * (no fallback here; a default grid is run again on fewer waves with larger
+ * worklists first) or report_cap overflows.  Calls that overlap on one
  * device race on the shared array. */
 int ngap_run_noalloc(ngap_engine *eng, const ngap_run_opts *opts, const uint8_t *d_input,
                      uint64_t chunk_len, uint32_t num_seg, uint64_t *d_reports,
@@ -324,7 +327,10 @@ int ngap_mlp_predict_pairs(ngap_mlp *m, const float *hist, uint32_t num_windows,
 /* Gradient of the mean squared error over (x, t) into grad[num_params]. */
 int ngap_mlp_gradient(ngap_mlp *m, const float *x, const float *t, uint64_t n, float *grad,
                       float *loss);
-/* Adam, mini-batches of `batch`, `epochs` passes; final epoch mean loss. */
+/* Adam, mini-batches of `batch`, `epochs` passes; final epoch mean loss.  The
+ * samples (about 1 KiB each) are on the device while it runs, up to 16 GiB and
+ * where they fit, else each mini-batch is copied; up to 256 MiB of them stay
+ * allocated for the next training. */
 int ngap_mlp_train(ngap_mlp *m, const float *x, const float *t, uint64_t n, int32_t epochs,
                    uint32_t batch, float lr, uint64_t seed, float *final_loss);
 

@@ -52,8 +52,8 @@ constexpr uint32_t kErrRowOrder = 1, kErrColRange = 2, kErrAasRange = 4, kErrSod
 // Bits that hold every value up to n (so that no value below n is all ones: the
 // sentinel stays the largest key).  A sort takes a pass per 8 bits of its keys:
 // with the bits that can differ, and lists, whose indices come in order, by their
-// d-gram alone, a load of 128 automata of up to 50,000 states takes 5.13 ms, with
-// all bits 5.4.
+// d-gram alone, a load of 128 automata of up to 50,000 states takes 0.3 ms less
+// than with all bits (5.1 to 5.6 ms in all, by the host that copies).
 inline int bits_of(uint64_t n) {
   int b = 1;
   while (b < 64 && (n >> b)) b++;

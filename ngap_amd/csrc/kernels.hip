@@ -382,10 +382,10 @@ NGAP_DEV void flatten(const KParams &P, WaveState &W, uint32_t cnt, uint32_t beg
 // go out together instead of one branch (and one wait) at a time.
 // Deep: the lists of depth 2 and 3 with their entries' filters.  Where a unit's
 // waves take their positions one batch after the other (drain) they spare a step
-// too seldom (1,024 automata, 2 MiB, depth 3: 5.9 ms without and 6.05 with them,
-// before the step itself became cheaper), while work items whose roots and
-// expansions overlap (drain_stream) took 6.25 and 6.12.  At depth 1 they always pay:
-// 11.1 and 8.7 ms, 10.9 and 8.1.
+// too seldom (1,024 automata of up to 5,000 states, 2 MiB, plain: depth 2 4.91 ms
+// without and 5.05 with them, depth 3 4.73 and 4.84).  Work items whose roots and
+// expansions overlap (drain_stream) gain 2 % by them, and at depth 1 they always
+// pay (11.1 and 8.7 ms plain, 10.9 and 8.1 batched, with 50,000 states).
 template <bool Stage = false, bool Deep = true>
 NGAP_DEV void roots(const KParams &P, WaveState &W, uint32_t p0, uint32_t pend) {
   const uint8_t *in = P.input;
@@ -1176,11 +1176,11 @@ NGAP_DEV T load_at(const void *base, uint32_t byte_offset) {
 // there.  A kernel of its own: without the other levels' index arrays its
 // scalar state fits the scalar registers (the general kernel spills over a
 // hundred of them into vector lanes, and moving them back and forth is vector
-// work), and the roots need a third of the instructions.  Before it (one kernel
-// for all levels, a slot read and both tables for every position, successors
-// without filters) and now: 400,000 states over 16 MiB 0.213 and 0.152 ms,
-// 1,024 automata over 8 MiB 0.272 and 0.206, over 64 MiB 1.77 and 1.31, eight
-// automata of short words over 4 MiB of text 0.139 and 0.126.  What bounds it is
+// work), and the roots need a third of the instructions.  With it, the filters and
+// the present windows and claims, against one kernel for all levels without them:
+// 400,000 states over 16 MiB 0.213 -> 0.120 ms, 1,024 automata over 8 MiB 0.272 ->
+// 0.191, over 64 MiB 1.77 -> 1.11, eight automata of short words over 4 MiB of text
+// 0.139 -> 0.100.  (The general kernel of now beside it: scan_image.)  What bounds it is
 // the latency of its gathers (slot, pairs, records: 4 MiB of L2 per XCD against
 // 128 MiB of slots) and, at the end of a run, of the last chains' steps.
 
@@ -1200,10 +1200,10 @@ struct ScanLds {
 // group, by the presence bitmap (2 MiB: it stays in L2, where the 128 MiB of
 // slots do not).  Two neighbouring positions a lane, from one 8-byte load of
 // the input (at most P.load_last, so that it stays inside the input).  The
-// slots are read by whole waves of present 3-grams (take_keys).  Against a slot
-// read at every position: 0.153 and 0.184 ms where the lists cover one 3-gram in
-// 28 (400,000 states, 16 MiB), 1.31 and 1.27 where they cover nearly half (1,024
-// automata, 64 MiB).
+// slots are read by whole waves of present 3-grams (take_keys).  It takes 0.83 of
+// the time of a slot read at every position where the lists cover one 3-gram in 28
+// (400,000 states, 16 MiB), 1.03 where they cover nearly half (1,024 automata, 64
+// MiB).
 NGAP_DEV void find_keys(const KParams &P, WaveState &W, ScanLds &S, uint32_t a, uint32_t b) {
   const uint32_t p = a + 2 * W.lane;
   // 3-grams end before the chunk does

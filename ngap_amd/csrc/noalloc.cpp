@@ -20,8 +20,8 @@
 namespace ngapamd {
 
 // Layout of the scratch array: the run counters (kCounterBytes of them: the
-// report count, the queue heads, the empty-queue masks and the item-count
-// lanes, cleared by the reset kernel) then the per-work-item overflow flags,
+// report count, the queue heads and the item-count lanes, cleared by the reset
+// kernel) then the per-work-item overflow flags,
 // then the worklist spill areas.
 constexpr uint64_t kScratchCounters = 8192;
 constexpr uint64_t kScratchFlags = 4ull << 20;  // 1M work items

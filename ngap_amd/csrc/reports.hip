@@ -16,12 +16,13 @@
 //    (reports_large.hip, a module of its own: a process's first use of rocPRIM's
 //    kernels loads them, 4 ms that few reports need not wait for).
 // The line between them: two ngap_get_reports calls (count, then copy) over
-// 2,048 reports take 25 us, over 4,096 31, 8,192 44, 16,384 70 by rank; 16,385
-// by radix (10 launches, the copy by hipMemcpy) 141, 131,072 558.  One 1,024-
-// thread workgroup closes the gaps of at most 16 slots per thread, held in
-// registers, which is the other reason for the line.  The host's std::sort, run
-// by both calls, took 158 us over 2,522 reports, 840 over 13,997 and 8,100 over
-// 154,507 (207 now).  The rank kernel is bound by its 64-bit comparisons: 14k
+// 2,048 reports take 25 us, over 4,096 31, 8,192 44, 16,384 70 by rank; by radix
+// (about 10 launches, the copy by hipMemcpy) over 16,385 98 to 146, 40,000 209,
+// 131,072 548, 154,507 194 (the library sorts in another way from some size on),
+// 1,000,000 1,520.  One 1,024-thread workgroup closes the gaps of at most 16 slots
+// per thread, held in registers, which is the other reason for the line.  The
+// host's std::sort, run by both calls, took 158 us over 2,522 reports, 840 over
+// 13,997, 8,100 over 154,507 and 26,100 over 1,000,000.  The rank kernel is bound by its 64-bit comparisons: 14k
 // keys in 59 us with a scalar load per key, 39 with one per eight.
 #include <hip/hip_runtime.h>
 

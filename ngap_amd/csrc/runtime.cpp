@@ -749,8 +749,8 @@ int host_tasks(const ngap_engine *eng, const ngap_run_opts &o, int memo_depth,
 // the lock-step baseline (k_blocking, blockinggroups).
 // Waves of a unit in k_plain: four, and while the grid stays below kPlainPerCu a
 // CU more of them, since few units leave the chip idle.  Kernel, ms, at four waves
-// a unit and so: one unit of 1 MiB 9.4 and 1.16, 256 units of 16 KiB 0.167 and
-// 0.096 (eight waves 0.119), 1,024 units of 4 KiB 0.094 either way.
+// a unit and so: one unit of 1 MiB 1.34 and 0.44, 256 units of 16 KiB 0.066 and
+// 0.028, 1,024 units of 4 KiB 0.029 either way (automata of 50 to 500 states).
 constexpr uint64_t kPlainPerCu = 16;
 uint32_t plain_waves(uint32_t units, uint32_t cus) {
   uint32_t waves = kBlockThreads / kWave;

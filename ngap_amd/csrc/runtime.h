@@ -303,10 +303,10 @@ void attach_ctx(KParams &P, RunCtx &ctx);
 int engine_kind(const ngap_run_opts &o, bool scan);
 // Whether all-group work items of this engine's runs take k_scan: memo depth
 // 3, no depth-1 or depth-2 reports in the image, records and classes below
-// 4 GiB each, and an input that holds an 8-byte load.  It was the faster one
-// wherever it can run: at equal windows of 1,024 positions 0.149 against 0.199 ms
-// (400,000 states, 16 MiB), 0.205 / 0.234 (1,024 automata, 8 MiB), 1.09 / 1.12
-// (64 MiB), 0.107 / 0.128 (short words in text).
+// 4 GiB each, and an input that holds an 8-byte load.  It is the faster one
+// wherever it can run: 0.120 ms against the general kernel's 0.161 (400,000 states,
+// 16 MiB), 0.191 / 0.194 (1,024 automata, 8 MiB), 1.11 / 1.13 (64 MiB), 0.100 / 0.114
+// (short words in text), 0.026 / 0.030 (DNA literals, 1 MiB).
 bool scan_image(const ngap_engine *eng, const Mapping &mp, uint64_t input_len);
 // Persistent grid of the batched kernel `kind` (batched_occupancy) for ring.
 int persistent_blocks(const ngap_engine *eng, uint32_t requested, uint32_t *blocks,
