@@ -330,17 +330,22 @@ int launch_slot(ngap_server *s, Slot &sl) {
     HIP_TRY(hipHostMalloc((void **)&sl.about_host, cap, hipHostMallocDefault));
     sl.about_cap = cap;
   }
-  HIP_TRY(sl.about.reserve(z.about));
-  memcpy(sl.about_host, sl.spans.data(), order_at);
-  memcpy(sl.about_host + order_at, sl.order.data(), about - order_at);
-  HIP_TRY(hipMemcpyAsync(sl.about.p, sl.about_host, about, hipMemcpyHostToDevice, sl.ctx.stream));
-  for (uint64_t id : sl.ids) s->reqs[id].state = 1;
   HIP_TRY(sl.ctx.tasks.reserve(z.tasks));
   sl.ctx.tasks_resident = false;
   HIP_TRY(sl.ctx.overflow.reserve(z.overflow));
   HIP_TRY(sl.ctx.reports.reserve(z.reports));
   sl.ctx.report_cap = z.report_cap;
   HIP_TRY(sl.ctx.spill.reserve(z.spill()));
+  if (sl.about.n < z.about) {
+    // with room for more requests than these where the budget has it: to enlarge a
+    // buffer is to wait for the device
+    const uint64_t others = s->held() - sl.about.n, more = std::max<uint64_t>(16384, 2 * z.about);
+    HIP_TRY(sl.about.reserve(others + more <= s->budget ? more : z.about));
+  }
+  memcpy(sl.about_host, sl.spans.data(), order_at);
+  memcpy(sl.about_host + order_at, sl.order.data(), about - order_at);
+  HIP_TRY(hipMemcpyAsync(sl.about.p, sl.about_host, about, hipMemcpyHostToDevice, sl.ctx.stream));
+  for (uint64_t id : sl.ids) s->reqs[id].state = 1;
   KParams P = base_params(s->eng, s->mp, s->opts);
   P.input = sl.input.as<uint8_t>();
   P.chunk_len = 0;
